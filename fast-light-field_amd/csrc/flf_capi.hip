@@ -31,10 +31,15 @@ struct Group {
     TileDesc* d_tiles = nullptr;
     int* d_bu = nullptr;
     int* d_au = nullptr;
-    int* d_uoff = nullptr;
-    int* d_s2 = nullptr;
+    int2* d_pairs = nullptr;
+    ushort4* d_wpos = nullptr;
+    int* d_colidx = nullptr;
     std::vector<unsigned char> enable_host;   // planes of the current projection (kernel-argument mask)
-    float2* d_G[2] = {nullptr, nullptr};
+    uint4* d_G[2] = {nullptr, nullptr};   // split spectra and output factors per direction (k_spec_pack)
+    float2* d_E[2] = {nullptr, nullptr};
+    float2* d_psi = nullptr;          // (the same for both directions)
+    int kg = 0;                       // 16-byte units per item and plane
+    int plane0 = 0;                   // planes of the groups before this one
     long long* d_srcoff_fwd = nullptr;   // active frame count's tables (point into the *_T lists)
     long long* d_Soff_fwd = nullptr;
     std::vector<long long*> srcoff_T, soff_T;    // [T - 1]: tables for every frame count <= Tcap
@@ -69,20 +74,22 @@ struct flf_ctx {
     std::vector<int2> fdims_host;
     bool ragged = false;
     float2* d_T_bwd = nullptr;
+    // Largest small-FFT component per source plane and frame (FLF_SMAX_WAYS
+    // parts), zero between projections: forward [planes, by group][frame],
+    // backward [group][frame].
+    float *d_smax_fwd = nullptr, *d_smax_bwd = nullptr;
     long long* d_zeros = nullptr;     // zero offsets (length max planes per group)
     double* d_fitpart = nullptr;
     double* d_fitout = nullptr;
     size_t max_lds = 65536;
-    int ipt = 2;                      // MAC items per lane pair's thread: 2 = lane pairs share two items
-                                      // and split the spectra (FLF_ITEMS_PER_THREAD=1 selects one item
-                                      // per thread); plan time
     int radix_order = 0;              // pass order of every FFT plan (make_radix_plan); plan time
-    int fb_max = 2;                   // frames per MAC workgroup at T >= 2 (FLF_MAC_FRAMES overrides)
     int fwd_split = 0;                // forward plane ranges, 0 = automatic (FLF_FWD_SPLIT overrides)
-    int bwd_planes = 1;               // planes per backward MAC workgroup
+    int bwd_planes = 0;               // planes per backward MAC workgroup, 0 = automatic (never set)
     int bwd_fgroup = 0;               // backward MAC frame blocks dispatched side by side (0: all)
-    bool mfma = false;                // matrix-core MAC (k_mac_tc, 8 frames per workgroup) for calls of >= 2
-                                      // frames (option mac_mfma, FLF_MAC_MFMA=1; chosen by the autotuner)
+    // Options of earlier multiply-accumulate kernels, accepted and kept as
+    // values (callers set and restore them); the matrix-core MAC takes 8
+    // frames per workgroup whatever they say.
+    int opt_ipt = 2, opt_frames = 2, opt_mfma = 0;
     // Fourier-grid groups of one projection side by side on streams of
     // their own (default priority, non-blocking), forked from and joined
     // back to the caller's stream by events; option "group_streams", off by
@@ -204,6 +211,7 @@ void free_all(flf_ctx* ctx) {
     ctx->ragged = false;
     ctx->d_T_bwd = nullptr;
     ctx->d_zeros = nullptr;
+    ctx->d_smax_fwd = ctx->d_smax_bwd = nullptr;
     ctx->d_fitpart = nullptr;
     ctx->d_fitout = nullptr;
 }
@@ -356,19 +364,17 @@ hipEvent_t take_event(flf_ctx* ctx) {
     return e;
 }
 
-// Frames per MAC workgroup: each spectrum value read serves fb frames.
-int mac_frames(const flf_ctx* ctx, const GridTables& gt) {
-    int fb = std::max(1, std::min(ctx->fb_max, ctx->T));
-    while (fb > 1 && mac_lds(gt.slots, gt.nu, ctx->N, fb) > ctx->max_lds) --fb;
-    return fb;
+int mac_frame_blocks(const flf_ctx* ctx, int slots) {
+    const int fb = mac_frames(slots, ctx->T);
+    return (ctx->T + fb - 1) / fb;
 }
 
-// Plane ranges of the forward MAC: about 4096 workgroups (4 per slot of the
-// 256 CUs x 4 resident workgroups), at most FWD_SPLIT_MAX ranges and one
-// plane per range (FLF_FWD_SPLIT overrides).
+// Plane ranges of the forward MAC: about 1024 workgroups (2 to 4 per
+// resident one), at most FWD_SPLIT_MAX ranges and one plane per range
+// (FLF_FWD_SPLIT overrides).
 int fwd_split(const flf_ctx* ctx, const Group& g, int nP) {
-    const long long per = (long long)g.gt.chunks.size() * ((ctx->T + mac_frames(ctx, g.gt) - 1) / mac_frames(ctx, g.gt));
-    int sp = (int)std::max<long long>(1, (4096 + per - 1) / std::max<long long>(per, 1));
+    const long long per = (long long)g.gt.chunks.size() * mac_frame_blocks(ctx, g.gt.slots);
+    int sp = (int)std::max<long long>(1, (1024 + per - 1) / std::max<long long>(per, 1));
     if (ctx->fwd_split > 0) sp = ctx->fwd_split;
     return std::max(1, std::min(std::min(sp, FWD_SPLIT_MAX), nP));
 }
@@ -384,9 +390,7 @@ int run_mac(flf_ctx* ctx, const MacArgs& m, const Group& g, int nplanes_grid, hi
         eb = take_event(ctx);
         if (ea && eb) HIPCHK(hipEventRecord(ea, st));
     }
-    // the matrix-core kernel (8 frames per workgroup) for calls of several frames
-    const bool tc = ctx->mfma && m.T >= 2 && m.tiles && mac_tc_lds(gt.slots, m.N) <= ctx->max_lds;
-    HIPCHK(launch_mac(m, gt.slots, gt.ipt, mac_frames(ctx, gt), (int)gt.chunks.size(), nplanes_grid, tc, st));
+    HIPCHK(launch_mac(m, gt.slots, (int)gt.chunks.size(), nplanes_grid, st));
     if (ctx->prof && ea && eb) {
         HIPCHK(hipEventRecord(eb, st));
         int np = 0;
@@ -403,27 +407,10 @@ long long s_frame_stride(const flf_ctx* ctx, const Group& g) {
     return (long long)g.gt.chunks.size() * ctx->N * ctx->N * g.gt.slots;
 }
 
-const int2* frame_dims(const flf_ctx* ctx) { return ctx->ragged ? ctx->d_fdims : nullptr; }
+// Accumulators of one frame: every item's slots (k_mac's order).
+long long acc_stride(const Group& g) { return (long long)g.gt.items.size() * g.gt.slots; }
 
-// Small FFTs of the backward source (the image) for one group.
-int run_small_fft_image(flf_ctx* ctx, Group& g, const float* img, hipStream_t st) {
-    SmallFFTArgs a{};
-    a.src = img;
-    a.src_off = ctx->d_zeros;
-    a.src_tstride = (long long)ctx->Y * ctx->X;
-    a.src_pitch = ctx->X;
-    a.Y = ctx->Y; a.X = ctx->X; a.N = ctx->N;
-    a.rpY = g.rpYr; a.rpX = g.rpXr;
-    a.twY = g.twRY; a.twX = g.twRX;
-    a.S = g.d_S_bwd;
-    a.S_off = ctx->d_zeros;
-    a.chunks = g.d_chunks; a.nchunks = (int)g.gt.chunks.size(); a.NH = g.gt.slots;
-    a.fY = g.gt.fY; a.fX = g.gt.fX;
-    a.S_tstride = s_frame_stride(ctx, g);
-    a.fdims = frame_dims(ctx);
-    HIPCHK(launch_small_fft(a, 1, ctx->T, st));
-    return FLF_OK;
-}
+const int2* frame_dims(const flf_ctx* ctx) { return ctx->ragged ? ctx->d_fdims : nullptr; }
 
 // The work of one grid group in one projection, as the kernels take it:
 // its small FFTs (nsrc source planes), its MAC (nranges plane ranges) and
@@ -450,20 +437,19 @@ int launch_group_work(flf_ctx* ctx, const GroupWork& w, hipStream_t st) {
 }
 
 // All groups' stages as one dispatch each on st.  done = false when this is
-// not possible (fewer than two groups, the matrix-core MAC, mixed item
-// shapes, LDS): the caller then launches group by group.
+// not possible (fewer than two groups, mixed item shapes, LDS): the caller
+// then launches group by group.
 int launch_grouped(flf_ctx* ctx, const std::vector<GroupWork>& ws, hipStream_t st, bool& done) {
     done = false;
-    if (!ctx->grouped || ws.size() < 2 || ws.size() > FLF_MAX_GROUPS || ctx->mfma) return FLF_OK;
+    if (!ctx->grouped || ws.size() < 2 || ws.size() > FLF_MAX_GROUPS) return FLF_OK;
     const GridTables& g0 = ctx->groups[ws[0].gi].gt;
-    int fb = 4, CB = 8;
+    int CB = 8;
     bool prime = false;
     for (const GroupWork& w : ws) {
         const Group& g = ctx->groups[w.gi];
-        if (g.gt.slots != g0.slots || g.gt.ipt != g0.ipt) return FLF_OK;
+        if (g.gt.slots != g0.slots) return FLF_OK;
         // the grouped kernels hold the register-held transforms only
         if (small_fft_big(g.gt.rY, g.gt.rX) || wave_big(g.gt.fY)) return FLF_OK;
-        fb = std::min(fb, mac_frames(ctx, g.gt));
         CB = std::min(CB, g.CBi);
         prime = prime || plan_has_prime(w.ca.rpY);
     }
@@ -471,8 +457,8 @@ int launch_grouped(flf_ctx* ctx, const std::vector<GroupWork>& ws, hipStream_t s
     MacGrouped mg{};
     IfftColGrouped cg{};
     sg.gg.ngroups = mg.gg.ngroups = cg.gg.ngroups = (int)ws.size();
-    mg.nfb = (ctx->T + fb - 1) / fb;
-    size_t lds_s = 0, lds_m = 0, lds_c = 0;
+    mg.nfb = mac_frame_blocks(ctx, g0.slots);
+    size_t lds_s = 0, lds_c = 0;
     double bytes = 0;
     for (size_t k = 0; k < ws.size(); ++k) {
         const GroupWork& w = ws[k];
@@ -486,10 +472,9 @@ int launch_grouped(flf_ctx* ctx, const std::vector<GroupWork>& ws, hipStream_t s
         mg.gg.start[k + 1] = mg.gg.start[k] + (nch * w.nranges * mg.nfb + 7) / 8 * 8;   // XCD-aligned (k_mac_grouped)
         mg.gg.nchunks[k] = nch;
         mg.gg.nranges[k] = w.nranges;
-        lds_m = std::max(lds_m, mac_lds(g.gt.slots, g.gt.nu, ctx->N, fb));
         cg.a[k] = w.ca;
         cg.a[k].CB = CB;
-        const int ncb = (w.ca.rfX + CB - 1) / CB;
+        const int ncb = ifft_col_blocks(cg.a[k]);
         cg.gg.start[k + 1] = cg.gg.start[k] + ncb * w.nbatch;
         cg.gg.nchunks[k] = ncb;
         cg.gg.nranges[k] = w.nbatch;
@@ -498,7 +483,7 @@ int launch_grouped(flf_ctx* ctx, const std::vector<GroupWork>& ws, hipStream_t s
         for (unsigned char e : g.enable_host) np += e ? 1 : 0;
         bytes += (double)np * g.gt.nu * g.gt.fY * g.gt.rfX * sizeof(float2);
     }
-    if (lds_s > ctx->max_lds || lds_m > ctx->max_lds || lds_c > ctx->max_lds) return FLF_OK;
+    if (lds_s > ctx->max_lds || lds_c > ctx->max_lds) return FLF_OK;
     HIPCHK(launch_small_fft_grouped(sg, ctx->N, ctx->T, lds_s, st));
     hipEvent_t ea = nullptr, eb = nullptr;
     if (ctx->prof) {
@@ -506,7 +491,7 @@ int launch_grouped(flf_ctx* ctx, const std::vector<GroupWork>& ws, hipStream_t s
         eb = take_event(ctx);
         if (ea && eb) HIPCHK(hipEventRecord(ea, st));
     }
-    HIPCHK(launch_mac_grouped(mg, g0.slots, g0.ipt, fb, mg.nfb, lds_m, st));
+    HIPCHK(launch_mac_grouped(mg, g0.slots, st));
     if (ctx->prof && ea && eb) {
         HIPCHK(hipEventRecord(eb, st));
         ctx->prof_recs.push_back({ea, eb, bytes});
@@ -557,37 +542,48 @@ int run_backward_groups(flf_ctx* ctx, const float* img, const std::vector<char>&
         a.S_tstride = s_frame_stride(ctx, g);
         a.fdims = frame_dims(ctx);
         a.tsplit = T;
+        a.smax = ctx->d_smax_bwd + gi * ctx->Tcap * FLF_SMAX_WAYS;
+        a.smax_zstride = 0;
         w.nsrc = 1;
         MacArgs& m = w.ma;
-        m.G = g.d_G[1];
-        m.chunks = g.d_chunks; m.items = g.d_items; m.u_bu = g.d_bu; m.u_au = g.d_au; m.uoff = g.d_uoff;
-        m.tiles = g.d_tiles;
-        m.S = g.d_S_bwd; m.S_off = ctx->d_zeros;
+        m.smax = a.smax; m.smax_pstride = 0;
+        m.G = g.d_G[1]; m.E = g.d_E[1]; m.psi = g.d_psi;
+        m.chunks = g.d_chunks; m.wpos = g.d_wpos; m.tiles = g.d_tiles; m.pairs = g.d_pairs;
+        m.kg = g.kg;
+        m.S = g.d_S_bwd; m.S_pstride = 0;
         m.S_tstride = s_frame_stride(ctx, g);
-        m.s2 = g.d_s2; m.enable = plane_mask(g);
+        m.enable = plane_mask(g);
         m.nP = (int)g.planes.size();
         m.A = g.d_A_bwd;
-        m.A_tstride = (long long)gt.fY * gt.rfX;
-        m.A_pstride = (long long)T * gt.fY * gt.rfX;
-        m.N = N; m.fY = gt.fY; m.fX = gt.fX; m.rY = gt.rY; m.rX = gt.rX; m.rfX = gt.rfX; m.nu = gt.nu;
+        m.A_tstride = acc_stride(g);
+        m.A_pstride = T * m.A_tstride;
+        m.N = N; m.nu = gt.nu;
         m.T = T;
-        m.rs = mac_row_stride(gt.slots, gt.nu);
         // Each workgroup takes bwd_planes consecutive planes (loads run on
         // across the plane boundary) and stores every plane's accumulator.
         m.per_plane = 1;
         m.fgroup = ctx->bwd_fgroup;
-        const int bp = std::max(1, ctx->bwd_planes);
+        // Three planes amortise its start (the first table waits for the
+        // small-FFT values) and keep its loads running across the boundary
+        // (1455^2 x 41 planes: T = 1 4.68 -> 4.40 ms, T = 8 7.77 -> 7.12); one
+        // plane when that would leave fewer than about 2048 workgroups.
+        const long long wgs = (long long)gt.chunks.size() * m.nP * mac_frame_blocks(ctx, gt.slots);
+        const int bp = ctx->bwd_planes > 0 ? ctx->bwd_planes : (int)std::min<long long>(3, std::max<long long>(1, wgs / 2048));
         w.nranges = (m.nP + bp - 1) / bp;
         IfftColArgs& ic = w.ca;
         ic.A = g.d_A_bwd;
-        ic.A_bstride = (long long)gt.fY * gt.rfX;
+        ic.A_bstride = acc_stride(g);
+        ic.colidx = g.d_colidx;
+        ic.N = N; ic.rY = gt.rY;
         ic.nsum = 1;
         ic.rfX = gt.rfX; ic.CB = g.CBi; ic.Yout = ctx->Y;
         ic.rpY = g.rpYw;
         ic.twY = g.twY;
         ic.out = ctx->d_T_bwd + g.Tbwd_off;
         ic.out_bstride = (long long)ctx->Y * gt.rfX;
-        w.nbatch = m.nP * T;
+        ic.T = T;
+        ic.FB = mac_frames(gt.slots, T);
+        w.nbatch = m.nP * mac_frame_blocks(ctx, gt.slots);
         ws.push_back(w);
     }
     return run_group_work(ctx, ws, fk);
@@ -636,11 +632,15 @@ int run_backward(flf_ctx* ctx, const float* img, float* vol, const float* Htf, c
         }
     if (ids.empty()) return FLF_OK;
     IfftRowPlaneArgs r{};
+    r.smax = ctx->d_smax_bwd;
+    r.nsmax = (int)ctx->groups.size() * ctx->Tcap * FLF_SMAX_WAYS;
     r.pd = ctx->d_rowdesc;
     for (size_t i = 0; i < ids.size(); ++i) r.plane_ids[i] = (unsigned short)ids[i];
     r.Tbuf = ctx->d_T_bwd;
     r.vol = vol; r.Htf = Htf; r.trust = trust;
     r.mode = mode; r.T = ctx->T; r.Y = ctx->Y; r.X = ctx->X;
+    r.FB4 = mac_frames(4, ctx->T);
+    r.FB2 = mac_frames(2, ctx->T);
     r.wbuf = wbuf;
     r.prime = prime;
     r.big = big;
@@ -668,18 +668,9 @@ int flf_create(int device, flf_ctx** out) {
     if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) == hipSuccess && lds > 0)
         c->max_lds = (size_t)lds;
     if (configure_kernels(c->max_lds) != hipSuccess) c->max_lds = 65536;
-    if (const char* e = getenv("FLF_ITEMS_PER_THREAD")) {
-        int v = atoi(e);
-        if (v == 1 || v == 2) c->ipt = v;
-    }
-    if (const char* e = getenv("FLF_MAC_MFMA")) c->mfma = atoi(e) != 0;
     if (const char* e = getenv("FLF_FWD_SPLIT")) {
         int v = atoi(e);
         if (v >= 1 && v <= 4) c->fwd_split = v;
-    }
-    if (const char* e = getenv("FLF_MAC_FRAMES")) {
-        int v = atoi(e);
-        if (v >= 1 && v <= 4) c->fb_max = v;
     }
     // set-up of the no-allocation data fit's scratch address on this device
     // (not required by the context: on failure flf_datafit_noalloc retries
@@ -732,7 +723,7 @@ int flf_plan(flf_ctx* ctx, int nnum, int Y, int X, int T, int nz, const int* s2)
             if ((int)ctx->groups.size() >= FLF_MAX_GROUPS) return fail(ctx, FLF_EINVAL, "too many distinct Fourier grids");
             ctx->groups.emplace_back();
             Group& g = ctx->groups.back();
-            std::string e = build_grid_tables(nnum, fY, fX, g.gt, ctx->ipt);
+            std::string e = build_grid_tables(nnum, fY, fX, g.gt);
             if (!e.empty()) return fail(ctx, FLF_EINVAL, e);
             const int ro = ctx->radix_order;
             if (!make_radix_plan(fY, g.rpY, false, ro) || !make_radix_plan(fX, g.rpX, false, ro) ||
@@ -750,7 +741,7 @@ int flf_plan(flf_ctx* ctx, int nnum, int Y, int X, int T, int nz, const int* s2)
     }
 
     // Device tables and buffers.
-    int maxP = 1;
+    int maxP = 1, plane0 = 0;
     long long Tbwd_total = 0;
     std::vector<RowPlaneDesc> rowdesc(nz);
     for (auto& g : ctx->groups) {
@@ -794,10 +785,20 @@ int flf_plan(flf_ctx* ctx, int nnum, int Y, int X, int T, int nz, const int* s2)
         if ((rc = upload(ctx, &g.d_tiles, gt.tiles))) return rc;
         if ((rc = upload(ctx, &g.d_bu, gt.u_bu))) return rc;
         if ((rc = upload(ctx, &g.d_au, gt.u_au))) return rc;
-        if ((rc = upload(ctx, &g.d_uoff, gt.uoff))) return rc;
-        std::vector<int> s2g;
-        for (int p = 0; p < nP; ++p) s2g.push_back(s2[g.planes[p]]);
-        if ((rc = upload(ctx, &g.d_s2, s2g))) return rc;
+        std::vector<int2> pairs;
+        for (size_t q = 0; q + 1 < gt.pairs.size(); q += 2) pairs.push_back(make_int2(gt.pairs[q], gt.pairs[q + 1]));
+        if ((rc = upload(ctx, &g.d_pairs, pairs))) return rc;
+        std::vector<ushort4> wpos;
+        for (size_t q = 0; q + 3 < gt.wpos.size(); q += 4)
+            wpos.push_back(make_ushort4(gt.wpos[q], gt.wpos[q + 1], gt.wpos[q + 2], gt.wpos[q + 3]));
+        if ((rc = upload(ctx, &g.d_colidx, gt.colidx))) return rc;
+        if ((rc = upload(ctx, &g.d_wpos, wpos))) return rc;
+        g.kg = gt.slots == 4 ? gt.nu : (gt.nu + 1) / 2;
+        g.plane0 = plane0;
+        plane0 += nP;
+        if (mac_lds(gt.slots, T) > ctx->max_lds || mac_lds(gt.slots, 1) > ctx->max_lds ||
+            spec_pack_lds(gt.nu, gt.slots) > ctx->max_lds)
+            return fail(ctx, FLF_EINVAL, "lenslet pitch too large for the multiply-accumulate kernel's LDS");
         // Volume-plane and small-FFT offsets depend on the frame count: one
         // table per count up to the capacity, selected by flf_set_frames.
         const long long Sper = (long long)T * s_frame_stride(ctx, g);
@@ -817,14 +818,16 @@ int flf_plan(flf_ctx* ctx, int nnum, int Y, int X, int T, int nz, const int* s2)
         g.d_Soff_fwd = g.soff_T[T - 1];
         g.enable_host.assign(nP, 1);
         const long long items = (long long)gt.items.size();
+        if ((rc = dalloc(ctx, &g.d_psi, gt.chunks.size() * nP * 5 * gt.slots))) return rc;
         for (int d = 0; d < 2; ++d) {
-            if ((rc = dalloc(ctx, &g.d_G[d], (size_t)items * gt.slots * gt.nu * nP))) return rc;
+            if ((rc = dalloc(ctx, &g.d_G[d], (size_t)items * nP * g.kg * 2))) return rc;
+            if ((rc = dalloc(ctx, &g.d_E[d], (size_t)items * nP * gt.slots))) return rc;
             g.have[d].assign(nP, 0);
         }
         if ((rc = dalloc(ctx, &g.d_S_fwd, (size_t)(nP * Sper)))) return rc;
         if ((rc = dalloc(ctx, &g.d_S_bwd, (size_t)Sper))) return rc;
-        if ((rc = dalloc(ctx, &g.d_A_fwd, (size_t)FWD_SPLIT_MAX * T * gt.fY * gt.rfX))) return rc;
-        if ((rc = dalloc(ctx, &g.d_A_bwd, (size_t)nP * T * gt.fY * gt.rfX))) return rc;
+        if ((rc = dalloc(ctx, &g.d_A_fwd, (size_t)FWD_SPLIT_MAX * T * acc_stride(g)))) return rc;
+        if ((rc = dalloc(ctx, &g.d_A_bwd, (size_t)nP * T * acc_stride(g)))) return rc;
         if ((rc = dalloc(ctx, &g.d_T_fwd, (size_t)T * Y * gt.rfX))) return rc;
         // Offsets into the shared backward buffer scale with the frame count:
         // unit offsets here, multiplied per count below.
@@ -834,6 +837,7 @@ int flf_plan(flf_ctx* ctx, int nnum, int Y, int X, int T, int nz, const int* s2)
             rd.T_off = Tbwd_total + (long long)p * Y * gt.rfX;
             rd.T_tstride = (long long)Y * gt.rfX;
             rd.rfX = gt.rfX;
+            rd.slots = gt.slots;
             rd.scale = 1.0f / ((float)gt.fY * (float)gt.fX);
             rd.rp = g.rpXw;
             rd.rph = g.rpXhw;
@@ -861,6 +865,8 @@ int flf_plan(flf_ctx* ctx, int nnum, int Y, int X, int T, int nz, const int* s2)
     }
     ctx->d_rowdesc = ctx->rowdesc_T[T - 1];
     if ((rc = upload(ctx, &ctx->d_zeros, std::vector<long long>(maxP, 0)))) return rc;
+    if ((rc = upload(ctx, &ctx->d_smax_fwd, std::vector<float>((size_t)nz * T * FLF_SMAX_WAYS, 0.f)))) return rc;
+    if ((rc = upload(ctx, &ctx->d_smax_bwd, std::vector<float>(ctx->groups.size() * T * FLF_SMAX_WAYS, 0.f)))) return rc;
     if ((rc = dalloc(ctx, &ctx->d_fitpart, (size_t)2 * FIT_BLOCKS * T))) return rc;
     if ((rc = dalloc(ctx, &ctx->d_fitout, (size_t)2 * T))) return rc;
     if ((rc = dalloc(ctx, &ctx->d_fdims, (size_t)T))) return rc;
@@ -932,9 +938,9 @@ int flf_set_option(flf_ctx* ctx, const char* name, int value) {
         ctx->fwd_split = value;
     } else if (n == "mac_frames") {
         if (value < 1 || value > 4) return fail(ctx, FLF_EINVAL, "mac_frames must be 1..4");
-        ctx->fb_max = value;
+        ctx->opt_frames = value;
     } else if (n == "mac_mfma") {
-        ctx->mfma = value != 0;
+        ctx->opt_mfma = value != 0;
     } else if (n == "bwd_planes") {
         if (value < 1 || value > 8) return fail(ctx, FLF_EINVAL, "bwd_planes must be 1..8");
         ctx->bwd_planes = value;
@@ -948,9 +954,9 @@ int flf_set_option(flf_ctx* ctx, const char* name, int value) {
     } else if (n == "radix_order") {             // takes effect at the next flf_plan
         if (value < 0 || value >= FLF_RADIX_ORDERS) return fail(ctx, FLF_EINVAL, "radix_order must be 0..3");
         ctx->radix_order = value;
-    } else if (n == "mac_ipt") {                 // takes effect at the next flf_plan
+    } else if (n == "mac_ipt") {
         if (value != 1 && value != 2 && value != 4) return fail(ctx, FLF_EINVAL, "mac_ipt must be 1, 2 or 4");
-        ctx->ipt = value;
+        ctx->opt_ipt = value;
     } else if (n == "ifft_col_batch") {
         if (!ctx->planned) return fail(ctx, FLF_ESTATE, "flf_plan has not been called");
         if (value < 1 || value > 8) return fail(ctx, FLF_EINVAL, "ifft_col_batch must be 1..8");
@@ -968,14 +974,14 @@ int flf_get_option(const flf_ctx* ctx, const char* name, int* value) {
     if (!ctx || !name || !value) return FLF_EINVAL;
     const std::string n(name);
     if (n == "fwd_split") *value = ctx->fwd_split;
-    else if (n == "mac_frames") *value = ctx->fb_max;
-    else if (n == "mac_mfma") *value = ctx->mfma ? 1 : 0;
-    else if (n == "bwd_planes") *value = ctx->bwd_planes;
+    else if (n == "mac_frames") *value = ctx->opt_frames;
+    else if (n == "mac_mfma") *value = ctx->opt_mfma;
+    else if (n == "bwd_planes") *value = std::max(1, ctx->bwd_planes);
     else if (n == "bwd_frame_group") *value = ctx->bwd_fgroup;
     else if (n == "group_streams") *value = ctx->group_streams ? 1 : 0;
     else if (n == "grouped_launch") *value = ctx->grouped ? 1 : 0;
     else if (n == "radix_order") *value = ctx->radix_order;
-    else if (n == "mac_ipt") *value = ctx->ipt;
+    else if (n == "mac_ipt") *value = ctx->opt_ipt;
     else if (n == "ifft_col_batch") *value = ctx->groups.empty() ? 0 : ctx->groups[0].CBi;
     else return FLF_EINVAL;
     return FLF_OK;
@@ -1024,8 +1030,8 @@ int flf_set_psf(flf_ctx* ctx, int z, int dir, const float* quadrant_host) {
     if (e == hipSuccess) e = launch_psf_cols(ca, gt.nu, 0);
     SpecPackArgs pa{};
     pa.spec = dspec; pa.chunks = g.d_chunks; pa.items = g.d_items; pa.u_bu = g.d_bu; pa.u_au = g.d_au;
-    pa.fY = gt.fY; pa.rfX = gt.rfX; pa.N = ctx->N; pa.slots = gt.slots; pa.nu = gt.nu;
-    pa.nP = (int)g.planes.size(); pa.p = ctx->idx_in_group[z]; pa.G = g.d_G[dir]; pa.s2 = s2;
+    pa.fY = gt.fY; pa.fX = gt.fX; pa.rfX = gt.rfX; pa.N = ctx->N; pa.slots = gt.slots; pa.nu = gt.nu; pa.kg = g.kg;
+    pa.nP = (int)g.planes.size(); pa.p = ctx->idx_in_group[z]; pa.G = g.d_G[dir]; pa.E = g.d_E[dir]; pa.psi = g.d_psi; pa.s2 = s2;
     if (e == hipSuccess) e = launch_spec_pack(pa, (int)gt.chunks.size(), 0);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     cleanup();
@@ -1087,7 +1093,10 @@ int run_forward(flf_ctx* ctx, const float* vol, const float* vol2, float* img, c
     if (rc) return rc;
     const int T = ctx->T;
     IfftRowSumArgs rs{};
+    rs.smax = ctx->d_smax_fwd;
+    rs.nsmax = ctx->nz * ctx->Tcap * FLF_SMAX_WAYS;
     rs.ngroups = (int)ctx->groups.size();
+    rs.T = T;
     rs.X = ctx->X;
     rs.Y = ctx->Y;
     rs.img = img;
@@ -1109,6 +1118,7 @@ int run_forward(flf_ctx* ctx, const float* vol, const float* vol2, float* img, c
         rs.grp[gi].T = g.d_T_fwd;
         rs.grp[gi].tstride = (long long)ctx->Y * gt.rfX;
         rs.grp[gi].rfX = gt.rfX;
+        rs.grp[gi].FB = mac_frames(gt.slots, T);
         rs.grp[gi].scale = 1.0f / ((float)gt.fY * (float)gt.fX);
         rs.grp[gi].rp = g.rpXw;
         rs.grp[gi].rph = g.rpXhw;
@@ -1158,27 +1168,31 @@ int run_forward_groups(flf_ctx* ctx, const float* vol, const float* vol2, const 
         a.fY = gt.fY; a.fX = gt.fX;
         a.S_tstride = s_frame_stride(ctx, g);
         a.fdims = frame_dims(ctx);
+        a.smax = ctx->d_smax_fwd + (long long)g.plane0 * ctx->Tcap * FLF_SMAX_WAYS;
+        a.smax_zstride = T;
         w.nsrc = nP;
         MacArgs& m = w.ma;
-        m.G = g.d_G[0];
-        m.chunks = g.d_chunks; m.items = g.d_items; m.u_bu = g.d_bu; m.u_au = g.d_au; m.uoff = g.d_uoff;
-        m.tiles = g.d_tiles;
-        m.S = g.d_S_fwd; m.S_off = g.d_Soff_fwd; m.S_tstride = a.S_tstride;
-        m.s2 = g.d_s2; m.enable = plane_mask(g);
+        m.smax = a.smax; m.smax_pstride = T;
+        m.G = g.d_G[0]; m.E = g.d_E[0]; m.psi = g.d_psi;
+        m.chunks = g.d_chunks; m.wpos = g.d_wpos; m.tiles = g.d_tiles; m.pairs = g.d_pairs;
+        m.kg = g.kg;
+        m.S = g.d_S_fwd; m.S_pstride = T * a.S_tstride; m.S_tstride = a.S_tstride;
+        m.enable = plane_mask(g);
         m.nP = nP;
         m.A = g.d_A_fwd;
-        m.A_tstride = (long long)gt.fY * gt.rfX;
-        m.A_pstride = (long long)T * gt.fY * gt.rfX;     // one partial accumulator per plane range
-        m.N = N; m.fY = gt.fY; m.fX = gt.fX; m.rY = gt.rY; m.rX = gt.rX; m.rfX = gt.rfX; m.nu = gt.nu;
+        m.A_tstride = acc_stride(g);
+        m.A_pstride = T * m.A_tstride;                   // one partial accumulator per plane range
+        m.N = N; m.nu = gt.nu;
         m.T = T;
-        m.rs = mac_row_stride(gt.slots, gt.nu);
         // Split the plane sum into ranges so that the launch has enough
         // workgroups to keep the tail short; the column transform adds the
         // partial accumulators in a fixed order.
         w.nranges = fwd_split(ctx, g, nP);
         IfftColArgs& ic = w.ca;
         ic.A = g.d_A_fwd;
-        ic.A_bstride = (long long)gt.fY * gt.rfX;
+        ic.A_bstride = acc_stride(g);
+        ic.colidx = g.d_colidx;
+        ic.N = N; ic.rY = gt.rY;
         ic.nsum = w.nranges;
         ic.A_sstride = m.A_pstride;
         ic.rfX = gt.rfX; ic.CB = g.CBi; ic.Yout = ctx->Y;
@@ -1186,7 +1200,9 @@ int run_forward_groups(flf_ctx* ctx, const float* vol, const float* vol2, const 
         ic.twY = g.twY;
         ic.out = g.d_T_fwd;
         ic.out_bstride = (long long)ctx->Y * gt.rfX;
-        w.nbatch = T;
+        ic.T = T;
+        ic.FB = mac_frames(gt.slots, T);
+        w.nbatch = mac_frame_blocks(ctx, gt.slots);
         ws.push_back(w);
     }
     return run_group_work(ctx, ws, fk);
@@ -1347,28 +1363,29 @@ int flf_radix_plan(int L, int wide, int order, int* radices, int* npass) {
 int flf_grid_check(int nnum, int fY, int fX, long long* stats) {
     if (!stats) return FLF_EINVAL;
     GridTables gt;
-    // the tables the projector plans by default: lane pairs of two items
-    std::string e = build_grid_tables(nnum, fY, fX, gt, 2);
+    std::string e = build_grid_tables(nnum, fY, fX, gt);
     if (!e.empty()) return FLF_EINVAL;
-    // every workgroup holds whole pairs, and the two items of a pair share
-    // their residues (one P/M table row serves both)
+    // every chunk is its tiles one after the other, one per wave, and the
+    // items of a tile share their residues (one table column set serves them)
     for (auto& c : gt.chunks) {
-        if (c.n_items % 2) return FLF_EINVAL;
-        for (int i = 0; i < c.n_items; i += 2) {
-            const ItemDesc& x = gt.items[c.item_base + i];
-            const ItemDesc& y = gt.items[c.item_base + i + 1];
-            for (int j = 0; j < 4; ++j)
-                if (x.res[j] != y.res[j]) return FLF_EINVAL;
+        int n = 0;
+        if (c.n_tiles < 1 || c.n_tiles > FLF_CHUNK_TILES) return FLF_EINVAL;
+        for (int t = 0; t < c.n_tiles; ++t) {
+            const TileDesc& td = gt.tiles[c.tile_base + t];
+            if (td.start != n || td.count < 1 || td.count > FLF_TILE) return FLF_EINVAL;
+            n += td.count;
+            for (int i = 0; i < td.count; ++i)
+                for (int j = 0; j < 4; ++j)
+                    if (gt.items[c.item_base + td.start + i].res[j] != td.res[j]) return FLF_EINVAL;
         }
+        if (n != c.n_items || n > FLF_CHUNK_MAX) return FLF_EINVAL;
     }
-    int max_items = 0;
-    for (auto& c : gt.chunks) max_items = std::max(max_items, c.n_items);
     stats[0] = (long long)gt.chunks.size();
     stats[1] = (long long)gt.items.size();
     stats[2] = gt.max_res;
     stats[3] = gt.nu;
     stats[4] = gt.slots;
-    stats[5] = max_items;
+    stats[5] = gt.max_items;
     return FLF_OK;
 }
 

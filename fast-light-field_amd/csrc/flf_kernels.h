@@ -3,6 +3,7 @@
 #include "flf_common.h"
 
 #define FLF_MAX_GROUPS 8
+#define FLF_SMAX_WAYS 4          // words that share the maximum of one (plane, frame)
 #define FLF_MAX_PLANES 256       // planes per plan: the plane selection travels in kernel arguments
 
 // Planes of a grid group selected for one projection, as a bitmask carried
@@ -41,6 +42,8 @@ struct SmallFFTArgs {
     const long long* S_off;      // per source plane z: element offset into S (device array)
     long long S_tstride;         // per frame
     const int2* fdims;           // per frame valid (Y, X) <= (Y, X), or null (all full size)
+    float* smax;                 // per source plane and frame: largest |component| of S, in FLF_SMAX_WAYS parts
+    int smax_zstride;
     const float* src2;           // frames t >= tsplit read from src2 (frame t - tsplit), or null
     int tsplit;
 };
@@ -67,30 +70,34 @@ struct SpecPackArgs {
     const ItemDesc* items;
     const int* u_bu;
     const int* u_au;
-    int fY, rfX, N, slots, nu, nP, p;
+    int fY, fX, rfX, N, slots, nu, nP, p;
+    int kg;                      // 16-byte units per item, plane and half (square: nu, else ceil(nu / 2))
     int s2;                      // PSF side of the plane (sets the folded phase ratios)
-    float2* G;                   // orbit-major spectra of the grid group
+    uint4* G;                    // orbit-major split spectra of the grid group
+    float2* E;                   // output factors of the grid group
+    float2* psi;                 // flip factors of the grid group
 };
 
 struct MacArgs {
-    const float2* G;
+    const uint4* G;              // k_spec_pack's G, E and psi
+    const float2* E;
+    const float2* psi;
     const ChunkDesc* chunks;
-    const ItemDesc* items;
-    const int* u_bu;
-    const int* u_au;
-    const int* uoff;             // [nu][8 or 4]: s-table column of each use, N*N if absent
+    const ushort4* wpos;         // per item: the place of each slot's bin in its chunk (GridTables::wpos)
+    const TileDesc* tiles;
+    const int2* pairs;           // [nu][slots]: the plain and conjugated use of each pair type (GridTables::pairs)
     const float2* S;
-    const long long* S_off;      // per plane in group
+    long long S_pstride;         // per plane in group (0: one image for all)
     long long S_tstride;
-    const int* s2;               // per plane in group
+    const float* smax;           // SmallFFTArgs::smax; smax_pstride floats per plane (0: one image for all)
+    int smax_pstride;
     PlaneMask enable;            // planes of the group in this projection
     int nP;
     float2* A;
     long long A_tstride, A_pstride;
-    int N, fY, fX, rY, rX, rfX, nu;
-    int T;                       // frames (grid z covers them in blocks of FB)
-    const TileDesc* tiles;       // residue-class tiles (matrix-core kernel)
-    int rs;                      // P/M table residue-row stride (mac_row_stride)
+    int N, nu;
+    int kg;                      // 16-byte units per item and plane
+    int T;                       // frames, in blocks of mac_frames(slots, T)
     int per_plane;               // 1: store each plane's accumulator at A + p * A_pstride (back
                                  // projection); 0: sum the planes of a range, store at
                                  // A + range * A_pstride (forward projection)
@@ -99,7 +106,10 @@ struct MacArgs {
 
 struct IfftColArgs {
     const float2* A;
-    long long A_bstride;
+    long long A_bstride;         // per frame
+    const int* colidx;           // [k1][y0][m]: place of bin (y0 + m rY, k1) (GridTables::colidx)
+    int N, rY;
+    int T, FB;                   // frames, interleaved in blocks of FB (mac_frames)
     int nsum;                    // partial accumulators summed on load (>= 1)
     long long A_sstride;
     int rfX, CB, Yout;
@@ -127,9 +137,10 @@ struct IfftColGrouped {
 };
 
 struct IfftRowGroup {
-    const float2* T;             // (T, Y, rfX)
-    long long tstride;
+    const float2* T;             // per block of FB frames (Y, rfX, frames)
+    long long tstride;           // per frame
     int rfX;
+    int FB;
     int active;
     float scale;
     RadixPlan rp;                // length fX
@@ -140,9 +151,11 @@ struct IfftRowGroup {
 
 struct IfftRowSumArgs {
     IfftRowGroup grp[FLF_MAX_GROUPS];
+    float* smax;                 // nsmax maxima to zero (SmallFFTArgs::smax)
+    int nsmax;
     int ngroups;
     int maxfX;
-    int X, Y;
+    int X, Y, T;
     float* img;                  // forward image, or null (not stored)
     long long img_tstride;
     const int2* fdims;           // per frame valid size; outside it the image is 0
@@ -151,9 +164,10 @@ struct IfftRowSumArgs {
 };
 
 struct RowPlaneDesc {
-    long long T_off;             // element offset of this plane's (T, Y, rfX) block
-    long long T_tstride;
+    long long T_off;             // element offset of this plane's column transforms
+    long long T_tstride;         // per frame
     int rfX;
+    int slots;                   // of the grid (4 square, 2 else)
     float scale;
     RadixPlan rp;                // length fX
     RadixPlan rph;               // length fX/2 (even fX)
@@ -164,12 +178,15 @@ struct RowPlaneDesc {
 struct IfftRowPlaneArgs {
     const RowPlaneDesc* pd;      // per plane z
     unsigned short plane_ids[FLF_MAX_PLANES];   // planes to process (grid z), by value
+    float* smax;                 // nsmax maxima to zero
+    int nsmax;
     const float2* Tbuf;
     float* vol;                  // (nz, T, Y, X)
     const float* Htf;            // mode 1
     const float* trust;          // mode 2 (optional, (nz, 1, Y, X))
     int mode;                    // 0 store, 1 Prevedel update, 2 standard update
     int T, Y, X;
+    int FB4, FB2;                // frames interleaved per block on square and other grids
     int wbuf;                    // per-wave LDS buffer (float2): max over planes of fX/2 (even) or fX
     const int2* fdims;           // per frame valid size; outside it the volume is set to 0
     int prime;                   // some plane's row plan ends with an odd prime radix above 5
@@ -199,16 +216,16 @@ int c2r_wave_buffer(int fX);
 hipError_t launch_small_fft(const SmallFFTArgs& a, int nsrc, int T, hipStream_t s);
 // Grouped launches (the groups' arguments by value).
 hipError_t launch_small_fft_grouped(const SmallFFTGrouped& ga, int N, int T, size_t lds, hipStream_t s);
-hipError_t launch_mac_grouped(const MacGrouped& ga, int slots, int ipt, int fb, int nfb, size_t lds, hipStream_t s);
+hipError_t launch_mac_grouped(const MacGrouped& ga, int slots, hipStream_t s);
 hipError_t launch_ifft_cols_grouped(const IfftColGrouped& ga, int CB, bool prime, size_t lds, hipStream_t s);
 hipError_t launch_psf_rows(const PsfRowArgs& a, int nu, hipStream_t s);
 hipError_t launch_psf_cols(const PsfColArgs& a, int nu, hipStream_t s);
+size_t spec_pack_lds(int nu, int slots);
 hipError_t launch_spec_pack(const SpecPackArgs& a, int nchunks, hipStream_t s);
-int mac_row_stride(int slots, int nu);
-size_t mac_tc_lds(int slots, int N);
-size_t mac_lds(int slots, int nu, int N, int fb);
-hipError_t launch_mac(const MacArgs& a, int slots, int ipt, int fb, int nchunks, int nplanes_grid, bool mfma,
-                      hipStream_t s);
+int mac_frames(int slots, int T);             // frames per MAC workgroup
+size_t mac_lds(int slots, int T);
+hipError_t launch_mac(const MacArgs& a, int slots, int nchunks, int nplanes_grid, hipStream_t s);
+int ifft_col_blocks(const IfftColArgs& a);
 hipError_t launch_ifft_cols(const IfftColArgs& a, int nbatch, hipStream_t s);
 hipError_t launch_ifft_rows_sum(const IfftRowSumArgs& a, int Y, int T, hipStream_t s);
 hipError_t launch_ifft_rows_plane(const IfftRowPlaneArgs& a, int nplanes, hipStream_t s);

@@ -10,6 +10,8 @@
 // and once per PSF set: k_psf_rows + k_psf_cols (pruned 2-D FFT of each
 // quadrant PSF) and k_spec_pack (gather into the MAC's orbit-major layout).
 #include <algorithm>
+#include <type_traits>
+#include <vector>
 
 #include "flf_common.h"
 #include "flf_fft.h"
@@ -92,6 +94,25 @@ __device__ __forceinline__ GroupPick pick_group(const GroupedGrid& gg, int b) {
     return p;
 }
 
+// Maximum over the wave's 64 lanes, in every lane.
+__device__ __forceinline__ float wave_max(float x) {
+#define FLF_DPP_MAX(ctrl) \
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), ctrl, 0xf, 0xf, true)))
+    FLF_DPP_MAX(0xB1);                            // quad_perm: lane ^ 1
+    FLF_DPP_MAX(0x4E);                            // quad_perm: lane ^ 2
+    FLF_DPP_MAX(0x124);                           // row_ror 4
+    FLF_DPP_MAX(0x128);                           // row_ror 8
+#undef FLF_DPP_MAX
+    x = fmaxf(x, __shfl_xor(x, 16));
+    return fmaxf(x, __shfl_xor(x, 32));
+}
+// Zero the MAC scales' maxima for the next projection (the last kernel of a
+// projection does, after the MAC has read them).
+__device__ __forceinline__ void reset_smax(float* smax, int n) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0)
+        for (int i = threadIdx.x; i < n; i += blockDim.x) smax[i] = 0.f;
+}
+
 // One (lenslet offset, frame, source plane) of a grid group; src0/src2/
 // tsplit: the source buffers of the call.
 template <bool BIG>
@@ -107,6 +128,8 @@ __device__ __forceinline__ void small_fft_body(const SmallFFTArgs& a, const floa
     float2* twX = twY + rY;                       // [rX]
     float2* phY = twX + rX;                       // [rY]
     float2* phX = phY + rY;                       // [rX]
+    unsigned* wgmax = reinterpret_cast<unsigned*>(phX + rX);
+    if (threadIdx.x == 0) *wgmax = 0;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     for (int i = threadIdx.x; i < rY; i += blockDim.x) twY[i] = a.twY[i];
     for (int i = threadIdx.x; i < rX; i += blockDim.x) twX[i] = a.twX[i];
@@ -204,6 +227,7 @@ __device__ __forceinline__ void small_fft_body(const SmallFFTArgs& a, const floa
     // used.
     const int NH = a.NH, NN = N * N;
     const int total = a.nchunks * NH;
+    float mx = 0.f;                               // largest component written
     constexpr int OU = 4;
     for (int i0 = threadIdx.x; i0 < total; i0 += OU * blockDim.x) {
         int k0[OU], k1[OU];
@@ -223,9 +247,19 @@ __device__ __forceinline__ void small_fft_body(const SmallFFTArgs& a, const floa
                                              : cconj(H[((rY - k0[u]) % rY) * rXh + (rX - k1[u])]);
                 v = cmul(v, cmul(phY[k0[u]], phX[k1[u]]));
                 S[((long long)w * NN + off) * NH + j] = v;
+                mx = fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y)));   // (NaN does not count: it scales to NaN)
             }
         }
     }
+    // The plane's and frame's largest component, for the MAC's scales: one
+    // atomic per workgroup, spread over FLF_SMAX_WAYS words (atomics on one
+    // word follow each other at about 25 ns: 225 took 6 us).
+    mx = wave_max(mx);
+    if (lane == 0) atomicMax(wgmax, __builtin_bit_cast(unsigned, mx));
+    __syncthreads();
+    if (threadIdx.x == 0)
+        atomicMax(reinterpret_cast<unsigned*>(a.smax + ((long long)z * a.smax_zstride + t) * FLF_SMAX_WAYS) + off % FLF_SMAX_WAYS,
+                  *wgmax);
 }
 
 template <bool BIG>
@@ -301,21 +335,60 @@ __global__ __launch_bounds__(FFT_THREADS) void k_psf_cols(PsfColArgs a) {
 
 // ---------------------------------------------------------------------------
 // Gather the natural-layout spectra of one plane into the orbit-major layout
-// G[chunk][plane][u][slot pair][item][2], each value pre-multiplied by
-// w^(bu*m2 + au*n2), w = exp(-2 pi i / (2N)) (m2, n2: half-unit aliases).
-// grid (nchunks, nu), block FLF_CHUNK_MAX.
+// of the MAC, each value pre-multiplied by w^(bu*m2 + au*n2) and rho^{-1/2},
+// w = exp(-2 pi i / (2N)) (m2, n2: half-unit aliases; see k_mac), and split
+// into two fp16 numbers:
+//   G[chunk][plane][kg][hi, lo][item][8 halves]
+// One 16-byte unit (item, kg) holds the (Re, Im) of 4 spectrum values: the 4
+// slots of stored spectrum u = kg (square grids), or the 2 slots of u = 2 kg
+// and 2 kg + 1 (non-square; zeros past the last u).  Values are scaled by a
+// power of two per (item, plane) so that the item's largest component lies in
+// [2^14, 2^15): hi + lo then holds 23 of its 24 significant bits (measured
+// against 64 bits at k_mac).  The imaginary parts of items whose first slot
+// lies on a negated residue are negated (see k_mac).  E[chunk][plane][item]
+// [slot] is the factor of the item's outputs: outer phase, 'same'-crop shift
+// and the inverse of the scale; psi[chunk][plane][residue][5] the flip factors.
+// grid (ceil(FLF_CHUNK_MAX / PACK_ITEMS), nchunks), block 256: PACK_ITEMS
+// items x 8 lanes over the spectra, the float values held in LDS between the
+// search for the largest and the split (each value read from memory once).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(FLF_CHUNK_MAX) void k_spec_pack(SpecPackArgs a) {
-    const int cidx = xcd_block(blockIdx.x, gridDim.x);
+constexpr int PACK_ITEMS = 32;
+__device__ __forceinline__ unsigned pack_half2(float a, float b) {
+    const _Float16 x = (_Float16)a, y = (_Float16)b;
+    return (unsigned)__builtin_bit_cast(unsigned short, x) | ((unsigned)__builtin_bit_cast(unsigned short, y) << 16);
+}
+// What fp16 rounding leaves of x (exact: x has 24 significant bits, the
+// rounded value 11 of them or x is below the fp16 range's bottom).
+__device__ __forceinline__ float half_rest(float x) { return x - (float)(_Float16)x; }
+// 2^e as a float (e clamped to [-120, 120]).
+__device__ __forceinline__ float exp2_int(int e) {
+    e = e < -120 ? -120 : (e > 120 ? 120 : e);
+    return __builtin_bit_cast(float, (unsigned)(127 + e) << 23);
+}
+// Power of two that brings the magnitude m into [2^top, 2^(top+1)); 1 for
+// zero, infinity and NaN (which then reach the results unscaled).
+__device__ __forceinline__ int scale_exp(float m, int top) {
+    const unsigned b = __builtin_bit_cast(unsigned, m) & 0x7fffffffu;
+    const int ex = (int)(b >> 23);
+    const int e = min(max(top + 127 - ex, -120), 120);       // (a denormal m: 120)
+    return b == 0 || ex == 255 ? 0 : e;
+}
+
+__global__ __launch_bounds__(256) void k_spec_pack(SpecPackArgs a) {
+    extern __shared__ float2 pk[];                   // [nu][PACK_ITEMS][slots], then the lanes' maxima [8][PACK_ITEMS]
+    float* mx = reinterpret_cast<float*>(pk + a.nu * PACK_ITEMS * a.slots);
+    const int cidx = blockIdx.y;
     const ChunkDesc* ch = a.chunks + cidx;
-    const int u = blockIdx.y;
-    const int i = threadIdx.x;
     const int n_items = ch->n_items;
-    if (i >= n_items) return;
+    const int i0 = blockIdx.x * PACK_ITEMS;
+    if (i0 >= n_items) return;
+    const int il = threadIdx.x & (PACK_ITEMS - 1), ug = threadIdx.x / PACK_ITEMS;
+    const int i = min(i0 + il, n_items - 1);         // lanes past the end repeat the last item, unwritten
+    const bool valid = i0 + il < n_items;
     const long long item_base = ch->item_base;
     const ItemDesc it = a.items[item_base + i];
-    const int bu = a.u_bu[u], au = a.u_au[u];
-    const int sig = a.s2 - 2 + a.N;
+    const int slots = a.slots, NH = slots, N = a.N;
+    const int sig = a.s2 - 2 + N;
     const int m2 = it.m2[0], n2 = it.n2[0];
     // rho_i^{-1/2}: the phase ratio of the two uses reading slot i, the same
     // for all output slots of the item (exponents in 1/(4N) turns).
@@ -324,19 +397,122 @@ __global__ __launch_bounds__(FLF_CHUNK_MAX) void k_spec_pack(SpecPackArgs a) {
     rho[1] = sig * (n2 - m2);
     rho[2] = sig * (m2 + n2);
     rho[3] = sig * (m2 - n2);
-    const float2* spec = a.spec + (long long)u * a.fY * a.rfX;
-    // Slots (0,1) of all items, then slots (2,3): a wave's 16-byte loads of
-    // one slot pair cover whole cache lines.
-    float2* G = a.G + item_base * a.slots * a.nu * a.nP + ((long long)a.p * a.nu + u) * n_items * a.slots;
-    for (int j = 0; j < a.slots; ++j) {
-        float2 v = spec[it.pos[j]];
-        long long e = 2LL * ((long long)bu * it.m2[j] + (long long)au * it.n2[j]) - rho[j];
-        G[(long long)(j >> 1) * n_items * 2 + 2 * i + (j & 1)] = cmul(v, phase_frac(e, 4 * a.N));
+    const bool neg = it.res[0] >= NH;
+    float m = 0.f;
+    for (int u = ug; u < a.nu; u += 8) {
+        const int bu = a.u_bu[u], au = a.u_au[u];
+        const float2* spec = a.spec + (long long)u * a.fY * a.rfX;
+        for (int j = 0; j < slots; ++j) {
+            const long long e = 2LL * ((long long)bu * it.m2[j] + (long long)au * it.n2[j]) - rho[j];
+            float2 v = cmul(spec[it.pos[j]], phase_frac(e, 4 * N));
+            if (neg) v.y = -v.y;
+            m = fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y)));
+            pk[(u * PACK_ITEMS + il) * slots + j] = v;
+        }
+    }
+    mx[ug * PACK_ITEMS + il] = m;
+    __syncthreads();
+    for (int q = 0; q < 8; ++q) m = fmaxf(m, mx[q * PACK_ITEMS + il]);
+    const int ea = scale_exp(m, 14);
+    const float s = exp2_int(ea);
+    uint4* G = a.G + (item_base * a.nP + (long long)a.p * n_items) * a.kg * 2;
+    for (int g = ug; g < a.kg; g += 8) {
+        unsigned h[4], l[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int u = slots == 4 ? g : 2 * g + (q >> 1), j = slots == 4 ? q : (q & 1);
+            float2 v = u < a.nu ? pk[(u * PACK_ITEMS + il) * slots + j] : make_float2(0.f, 0.f);
+            v.x *= s;
+            v.y *= s;
+            h[q] = pack_half2(v.x, v.y);
+            l[q] = pack_half2(half_rest(v.x), half_rest(v.y));
+        }
+        if (valid) {
+            G[(2LL * g + 0) * n_items + i] = make_uint4(h[0], h[1], h[2], h[3]);
+            G[(2LL * g + 1) * n_items + i] = make_uint4(l[0], l[1], l[2], l[3]);
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x < NH) {
+        // flip factors of the chunk's residues: exp(-2 pi i (s2-1) kt / f), as
+        // [residue][1, row flip, column flip, both, 0]
+        float2 w[2];
+        for (int ax = 0; ax < 2; ++ax) {
+            const int k = ax == 0 ? ch->res0[threadIdx.x] : ch->res1[threadIdx.x];
+            const int f = ax == 0 ? a.fY : a.fX, r = f / N;
+            w[ax] = phase_frac((long long)(a.s2 - 1) * centred_res(k, r), f);
+        }
+        float2* o = a.psi + (((long long)cidx * a.nP + a.p) * NH + threadIdx.x) * 5;
+        o[0] = make_float2(1.f, 0.f);
+        o[1] = w[0];
+        o[2] = w[1];
+        o[3] = cmul(w[0], w[1]);
+        o[4] = make_float2(0.f, 0.f);
+    }
+    if (ug < slots && valid) {
+        const int j = ug;
+        const int c2 = (a.s2 - 1) / 2;
+        const int outer = j == 0 ? sig * (m2 + n2) : j == 1 ? sig * (n2 - m2) : j == 2 ? sig * (n2 + m2) : sig * (m2 - n2);
+        const int k0 = it.pos[j] / a.rfX, k1 = it.pos[j] - k0 * a.rfX;
+        // exp(+2 pi i c2 (k0/fY + k1/fX)): c2 < f / 2 and k < f <= FLF_MAX_FOURIER, 32-bit products
+        float fr = (float)((c2 * k0) % a.fY) / (float)a.fY + (float)((c2 * k1) % a.fX) / (float)a.fX;
+        fr -= rintf(fr);
+        float sn, cs;
+        sincospif(2.0f * fr, &sn, &cs);
+        const float2 v = cmul(phase_frac_i(outer, 4 * N), make_float2(cs, sn));
+        const float is = exp2_int(-ea);
+        a.E[(item_base * a.nP + (long long)a.p * n_items + i) * slots + j] = make_float2(v.x * is, v.y * is);
     }
 }
 
 // ---------------------------------------------------------------------------
-// The multiply-accumulate over the N*N lenslet offsets (k_mac below).
+// The multiply-accumulate over the N*N lenslet offsets.
+//
+// For an item with base alias (m2, n2) (half units) and output slots P0..P3,
+// every output accumulates
+//   A_j = w4^(outer_j) * sum_u sum_i [ P_{j,i,u} Re g_i + M_{j,i,u} Im g_i ]
+// with g_i the stored spectrum value of slot i (pre-multiplied by
+// w2^(bu m2_i + au n2_i) and rho_i^{-1/2}), w4 = exp(-2 pi i/(4N)),
+// outer = sig*(m2+n2), sig*(n2-m2), sig*(n2+m2), sig*(m2-n2), sig = s2-2+N.
+// P and M combine the small-FFT values s of the two uses reading slot i at
+// output j, s = S_{b,a}(kappa) exp(-2 pi i (beta_b kt0/fY + alpha_a kt1/fX)),
+// beta = b (b <= N/2) or b + s2 - 1 (row-flipped offsets), likewise alpha:
+// P = s_plain + s_conj, M = i (s_plain - s_conj).
+// This is the accumulation of py_light_field.cpp:303-341, 1029-1087 with the
+// mirror multipliers of projector.py:137-151 and the 'same' crop
+// (projector.py:792-796) folded into phases.
+//
+// As a matrix product.  The pair type of source slot i at output slot j is
+// pt = i XOR j, so for the items of one residue class (their slots lie on the
+// same residues res_j) and one output slot j
+//   out_j[item][(f, c)] = sum_{(u, i, r)} A[item][(u, i, r)] B_j[(u, i, r)][(f, c)]
+// with A the item's stored values (r = Re, Im), shared by every slot, and B_j
+// the P (r = Re) and M (r = Im) components c of frame f at residue res_j, pair
+// type i XOR j.  S(-k) = conj S(k) makes the table of a negated residue
+// (P*, -M*): such outputs take the table of the positive residue with the
+// sign of M flipped and are conjugated afterwards, so only the first NH
+// residues of an orbit have tables.  M also changes sign for odd j and
+// pt >= 2 (the alias order of the transposed slots).
+//
+// Matrix cores.  v_mfma_f32_16x16x32_f16: 16 items x 16 columns (NS slots x
+// 8 / NS frames x (Re, Im)), K = 32 = 4 spectra of a square grid.  Both
+// operands are fp32 numbers split into two fp16 ones (hi + lo: 23 of 24
+// significant bits, after a power-of-two scale per item and per frame), and all
+// four products hi*hi, lo*hi, hi*lo, lo*lo are taken with fp32 accumulation;
+// the three small ones are summed apart, so an accumulator is rounded 5 times
+// per 4 spectra where an fp32 FMA chain rounds 32 times.  Relative L2 error of
+// whole projections against 64 bits, this kernel / the fp32 FMA kernel it
+// replaced: 1455^2 x 41 planes forward 1.06e-7 / 1.04e-7, backward 1.63e-7 /
+// 1.66e-7; RL at 2048^2 3.28e-7 / 3.25e-7, 997 x 1171 (Nnum 13) 2.74e-7 /
+// 3.00e-7, 1273 x 1463 (Nnum 19) 6.43e-7 / 6.34e-7.
+//
+// One workgroup: one chunk, 8 waves, one tile (<= 32 items of a class) per
+// wave; a plane range's planes in turn.  Per plane the table of P and M goes
+// to LDS once (read as 16-byte B operands, conflict free) while the previous
+// plane's products run; the stored spectra are streamed from memory straight
+// into the A operands, RING K steps ahead.  Bound: HBM up to 4 frames (1455^2 x
+// 41 planes, one frame: forward 3.16 ms for 17.8 GB = 5.6 TB/s, a plain read
+// of such runs reaches 6.2; the FMA kernel 4.07 ms), matrix and vector issue
+// at 8 (forward 13.3 -> 4.4 ms, backward 17.0 -> 5.5 ms).
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -346,472 +522,416 @@ namespace {
 // conjugated read; their pair types (plain, conj) are
 //   quad:  0 (id, both)  1 (row, col)  2 (Tid, Tboth)  3 (Tcol, Trow)
 //   pair:  0 (id, both)  1 (row, col)
-__device__ constexpr int kPairPlain[4] = {0, 2, 4, 7};
-__device__ constexpr int kPairConj[4] = {1, 3, 5, 6};
-// Output slot j, source slot i -> pair type and sign of the M term.
-__device__ constexpr int kQuadPT[4][4] = {{0, 1, 2, 3}, {1, 0, 3, 2}, {2, 3, 0, 1}, {3, 2, 1, 0}};
-__device__ constexpr int kQuadSG[4][4] = {{1, 1, 1, 1}, {1, 1, -1, -1}, {1, 1, 1, 1}, {-1, -1, 1, 1}};
-__device__ constexpr int kPairPT[2][2] = {{0, 1}, {1, 0}};
+// (the planner's pair table lists their source offsets).
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
-// Spectra are streamed once per projection.  Plain loads measured 10% faster
-// than non-temporal ones on MI355X (FLF_MAC_NT=1 selects the latter).
-#ifndef FLF_MAC_NT
-#define FLF_MAC_NT 0
-#endif
-__device__ __forceinline__ v4f load_stream(const v4f* q) {
-#if FLF_MAC_NT
-    return __builtin_nontemporal_load(q);
-#else
-    return *q;
-#endif
-}
-// Item ti of one (chunk, plane, spectrum) block of n_items items: slots
-// (0,1) at ti, slots (2,3) n_items entries further.
-template <int SLOTS>
-__device__ __forceinline__ void load_g(float2 (&g)[4], const float2* blk, int ti, int n_items) {
-    const v4f* q = reinterpret_cast<const v4f*>(blk) + ti;
-    v4f x = load_stream(q);
-    g[0] = make_float2(x.x, x.y);
-    g[1] = make_float2(x.z, x.w);
-    if constexpr (SLOTS == 4) {
-        v4f y = load_stream(q + n_items);
-        g[2] = make_float2(y.x, y.y);
-        g[3] = make_float2(y.z, y.w);
-    } else {
-        g[2] = g[3] = make_float2(0.f, 0.f);
-    }
+__device__ __forceinline__ v4f mfma_f16(v4u a, v4u b, v4f c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0, 0);
 }
 
 }  // namespace
 
-// acc[a][j] += P * Re(g[a][i]) + sg * M * Im(g[a][i]) for every output slot
-// j, source slot i and item a of the thread (the items share residues, so
-// each 16-byte LDS entry (P, M) serves all of them).
-// P = s_plain + s_conj, M = i (s_plain - s_conj).
-template <int SLOTS, int IPT, int FB>
-__device__ __forceinline__ void mac_spectrum(float2 (&acc)[FB][IPT][4], const float2 (&g)[IPT][4],
-                                             const float4* __restrict__ pm, int tab, const int (&rb)[4], int u) {
-    constexpr int NPT = SLOTS == 4 ? 4 : 2;
-#pragma unroll
-    for (int f = 0; f < FB; ++f) {
-#pragma unroll
-        for (int j = 0; j < SLOTS; ++j) {
-            const float4* row = pm + f * tab + rb[j] + u * NPT;
-#pragma unroll
-            for (int i = 0; i < SLOTS; ++i) {
-                const int pt = SLOTS == 4 ? kQuadPT[j][i] : kPairPT[j][i];
-                const float sg = SLOTS == 4 ? (float)kQuadSG[j][i] : 1.0f;
-                const float4 q = row[pt];          // (P.x, P.y, M.x, M.y)
-                const float mx = sg * q.z, my = sg * q.w;
-#pragma unroll
-                for (int a = 0; a < IPT; ++a) {
-                    acc[f][a][j].x = fmaf(q.x, g[a][i].x, acc[f][a][j].x);
-                    acc[f][a][j].y = fmaf(q.y, g[a][i].x, acc[f][a][j].y);
-                    acc[f][a][j].x = fmaf(mx, g[a][i].y, acc[f][a][j].x);
-                    acc[f][a][j].y = fmaf(my, g[a][i].y, acc[f][a][j].y);
-                }
-            }
-        }
-    }
+constexpr int MAC_THREADS = 64 * FLF_CHUNK_TILES;
+
+// Shapes of a MAC workgroup.  NS output slots share the 16 columns of a
+// matrix instruction, so it takes FB = 8 / NS frames: few frames with NS = 1
+// would leave most columns empty.
+template <int SLOTS, int NS>
+struct MacShape {
+    static constexpr int NH = SLOTS;              // residues with tables (the rest by conjugation)
+    static constexpr int NPT = SLOTS;             // pair types
+    static constexpr int UPG = SLOTS == 4 ? 1 : 2;   // spectra per 16-byte unit
+    static constexpr int FB = FLF_MAC_FB / NS;
+    static constexpr int COLS = 2 * FB;           // table columns per (residue, unit)
+    // Waves per SIMD: 4 (two workgroups per CU) where the tables leave LDS and
+    // the accumulators registers for it, else 2 with more loads in flight each.
+    static constexpr int WAVES = NS == SLOTS ? 4 : 2;
+    static constexpr int RING = WAVES == 4 ? 2 : 3;   // K steps of A operands in flight per wave
+    static constexpr int KB = WAVES == 4 ? 10 : 9;    // K steps per table batch, a multiple of RING
+    static constexpr int NF = SLOTS / NS;         // B operands (groups of NS slots) per K step
+    // 16-byte units of one residue's table; the pad puts the residues that one
+    // operand read touches (NS > 1) on different banks
+    static constexpr int RS = 4 * KB * COLS + (NS > 1 ? COLS : 0);
+    static constexpr int TAB = NH * RS;           // units of one half (hi or lo) of a table
+    static constexpr int NT = (KB * 4 * UPG * NPT * FB + MAC_THREADS - 1) / MAC_THREADS;   // entries per thread
+    static constexpr int E = FLF_CHUNK_TILES * FLF_TILE * SLOTS;                              // output factors
+    static constexpr int HM = (FLF_MAX_N + 1) / 2, PAIRS = (SLOTS == 4 ? HM * (HM + 1) / 2 : HM * HM) * NPT;   // the most
+    // two tables (the one in use and the next), the output factors of every
+    // wave's tile, the items' bins, the pair list, the inverse scales of two
+    // planes, every wave's flip factors
+    static constexpr size_t LDS = (size_t)4 * TAB * 16 + (size_t)E * 8 + (size_t)FLF_CHUNK_MAX * 8 + (size_t)PAIRS * 4 + (size_t)2 * FB * 4 +
+                                  (size_t)FLF_CHUNK_TILES * 5 * NH * 8;
+};
+
+// The value of lane ^ 1.
+__device__ __forceinline__ float lane_xor1(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, true));
 }
 
-#ifndef FLF_MAC_UNR
-#define FLF_MAC_UNR 2
-#endif
-#ifndef FLF_MAC_UNR2
-#define FLF_MAC_UNR2 1
-#endif
-#ifndef FLF_MAC_UNR2_FB1
-#define FLF_MAC_UNR2_FB1 2
-#endif
-#ifndef FLF_MAC_WAVES
-#define FLF_MAC_WAVES 4
-#endif
-
-// Wave-uniform read of a per-plane value through the scalar cache (the array
-// is read-only while the kernel runs).  Scalar loads keep such reads off the
-// vector-memory counter, so they never make the accumulation wait for the
-// spectrum loads in flight.
-// The value is moved to scalar registers at once (readfirstlane), so a load
-// that had to go through a vector register is consumed on every path.
-__device__ __forceinline__ int const_load(const int* base, int i) {
-    return __builtin_amdgcn_readfirstlane(((const __attribute__((address_space(4))) int*)base)[i]);
-}
-__device__ __forceinline__ long long const_load(const long long* base, int i) {
-    const long long v = ((const __attribute__((address_space(4))) long long*)base)[i];
-    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(v & 0xffffffffLL));
-    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)((unsigned long long)v >> 32));
-    return (long long)(((unsigned long long)hi << 32) | lo);
-}
-// s_waitcnt vmcnt(0) issued through the builtin, so that the compiler's own
-// wait counting knows every vector-memory access has completed.
-__device__ __forceinline__ void wait_vmem_all() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
-// Copy of the chunk's small-FFT blocks of plane p, frames t0 .. t0+nf-1, into
-// s_stage ([f][NN][NH]) by global-to-LDS loads: every load of the block is in
-// flight at once and no registers are held; completion is awaited (vmcnt) by
-// mac_tables.  (Started earlier, during the previous plane's accumulation,
-// the copy would make the compiler drain all vector loads before every LDS
-// read of the accumulation.)  The block size is a multiple of 64 threads.
-template <int SLOTS>
-__device__ __forceinline__ void mac_stage_async(const MacArgs& a, int cidx, int p, int t0, int nf, float2* s_stage) {
-    constexpr int NH = SLOTS == 4 ? 4 : 2;
-    const int blk = a.N * a.N * NH;              // float2 per frame block
-    const int nd = 2 * blk;                       // dwords per frame block
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    const long long sbase = const_load(a.S_off, p) + (long long)t0 * a.S_tstride + (long long)cidx * blk;
-    for (int f = 0; f < nf; ++f) {
-        const float* src = reinterpret_cast<const float*>(a.S + sbase + f * a.S_tstride);
-        float* dst = reinterpret_cast<float*>(s_stage + f * blk);
-        for (int c = wv * 64; c < nd; c += nw * 64)
-            if (c + lane < nd)
-                __builtin_amdgcn_global_load_lds(src + c + lane, (__attribute__((address_space(3))) void*)(dst + c), 4,
-                                                 0, 0);
-    }
-}
-
-// Per-plane set-up of a MAC workgroup: flip factors, then per frame f < nf
-// the P/M table of the chunk's small-FFT block (staged in LDS beforehand)
-//   pm[f][rho * rs + u * NPT + pt] = (P, M),  P = s_plain + s_conj,
-//   M = i (s_plain - s_conj)
-// for residue rho, stored spectrum u and pair type pt (all threads; contains
-// barriers; frames past nf keep the tables of earlier planes and their
-// accumulators are never stored).
-template <int SLOTS>
-__device__ __forceinline__ void mac_tables(const MacArgs& a, const ChunkDesc* ch, int cidx, int p, int t0, int nf,
-                                           float4* pm_tab, float2* s_stage, float2* psi, int rs) {
-    constexpr int NUSE = SLOTS == 4 ? 8 : 4;
-    constexpr int NPT = SLOTS == 4 ? 4 : 2;
-    constexpr int NRES = SLOTS == 4 ? 8 : 4;
-    constexpr int NH = NRES / 2;
-    const int tid = threadIdx.x;
-    const int N = a.N, NN = N * N, c = N / 2;
-    const int nu = a.nu;
-    const int tab = NRES * rs;
-    const int s2 = const_load(a.s2, p);
-    // flip factors per residue: exp(-2 pi i (s2-1) kt / f) (psi was last read
-    // before the closing barrier of the previous plane's set-up)
-    if (tid < 2 * NRES) {
-        const int rho = tid >> 1;
-        const bool isY = (tid & 1) == 0;
-        const int k = isY ? ch->res0[rho] : ch->res1[rho];
-        const int r = isY ? a.rY : a.rX;
-        const int f = isY ? a.fY : a.fX;
-        const int kt = (2 * k < r) ? k : ((2 * k > r) ? k - r : 0);
-        int m = (int)(((long long)(s2 - 1) * kt) % f);
-        if (m < 0) m += f;
-        float sn, cs;
-        sincospif(-2.0f * (float)m / (float)f, &sn, &cs);
-        psi[tid] = make_float2(cs, sn);
-    }
-    // Copy the small-FFT blocks of all nf frames into s_stage, wait for the
-    // copy, then build every frame's table (the barrier also orders these
-    // writes of pm_tab after every wave's reads of the previous plane's
-    // table).
-    const int blk = NN * NH;
-    mac_stage_async<SLOTS>(a, cidx, p, t0, nf, s_stage);
-    wait_vmem_all();
-    __syncthreads();
-    {
-        // Thread -> table column q = (u, pt) and a share of the rows
-        // (f, rho): the column's two source offsets and flip flags are
-        // decoded once, the rows then cost two LDS reads and the P/M
-        // arithmetic each (no integer division per entry).
-        const int Q = nu * NPT;
-        const int nt = blockDim.x;
-        const bool fits = Q <= nt;
-        const int rstep = fits ? nt / Q : 1;
-        const int r0 = fits ? tid / Q : 0;
-        const int rows = nf * NRES;
-        for (int q = (fits ? (r0 < rstep ? tid - r0 * Q : Q) : tid); q < Q; q += nt) {
-            const int pt = q % NPT, u = q / NPT;
-            int src[2], flip[2];
-#pragma unroll
-            for (int w = 0; w < 2; ++w) {
-                const int off = a.uoff[u * NUSE + (w == 0 ? kPairPlain[pt] : kPairConj[pt])];
-                const int bo = off / N, ao = off - bo * N;
-                src[w] = off < NN ? off * NH : -1;
-                flip[w] = (bo > c ? 1 : 0) | (ao > c ? 2 : 0);
-            }
-            for (int row = r0; row < rows; row += rstep) {
-                const int f = row / NRES, rho = row % NRES;
-                const float2* sf = s_stage + f * blk;
-                const int rb0 = rho < NH ? rho : rho - NH;
-                float2 sv[2];
-#pragma unroll
-                for (int w = 0; w < 2; ++w) {
-                    float2 r = make_float2(0.f, 0.f);
-                    if (src[w] >= 0) {
-                        r = sf[src[w] + rb0];
-                        if (rho >= NH) r = cconj(r);
-                        if (flip[w] & 1) r = cmul(r, psi[2 * rho]);
-                        if (flip[w] & 2) r = cmul(r, psi[2 * rho + 1]);
-                    }
-                    sv[w] = r;
-                }
-                const float2 P = cadd(sv[0], sv[1]);
-                const float2 d = csub(sv[0], sv[1]);
-                pm_tab[f * tab + rho * rs + u * NPT + pt] = make_float4(P.x, P.y, -d.y, d.x);   // M = i * d
-            }
-        }
-    }
-    __syncthreads();
-}
-
-// For an item with base alias (m2, n2) (half units) and output slots
-// P0..P3, every output accumulates
-//   A_j = w4^(outer_j) * sum_u sum_i [ P_{j,i,u} Re g_i + M_{j,i,u} Im g_i ]
-// with g_i the stored spectrum value of slot i (pre-multiplied by
-// w2^(bu m2_i + au n2_i) and rho_i^{-1/2}), w4 = exp(-2 pi i/(4N)),
-// outer = sig*(m2+n2), sig*(n2-m2), sig*(n2+m2), sig*(m2-n2), sig = s2-2+N.
-// P and M combine the small-FFT values s of the two uses reading slot i at
-// output j, s = S_{b,a}(kappa) exp(-2 pi i (beta_b kt0/fY + alpha_a kt1/fX)),
-// beta = b (b <= N/2) or b + s2 - 1 (row-flipped offsets), likewise alpha.
-// This is the accumulation of py_light_field.cpp:303-341, 1029-1087 with the
-// mirror multipliers of projector.py:137-151 and the 'same' crop
-// (projector.py:792-796) folded into phases.  IPT = 1: one item per
-// thread; IPT = 2 (4): a lane pair (quad) owns two (four) consecutive items
-// that share their residues and splits the spectra between its lanes.  FB frames per
-// workgroup: every stored spectrum value loaded serves FB frames, and the
-// frame blocks of one chunk run side by side on one XCD (block ids below).
 // One workgroup: chunk cidx, plane range `range` of nranges, frame block
-// fblock.
-template <int SLOTS, int IPT, int FB>
+// fblock.  PER_PLANE: store each plane's accumulator (back projection);
+// otherwise the planes of the range are summed (forward projection).
+template <int SLOTS, int NS, bool PER_PLANE>
 __device__ __forceinline__ void mac_body(const MacArgs& a, int cidx, int range, int nranges, int fblock) {
-    extern __shared__ float4 pm_tab[];            // [FB][NRES][rs: nu*NPT + pad], then staging
-    constexpr int NRES = SLOTS == 4 ? 8 : 4;      // residues per orbit (canonical list)
-    constexpr int NH = NRES / 2;                  // residues stored by the small-FFT kernel
-    // spectra whose loads are issued together
-    constexpr int UNR = IPT >= 2 ? (FB == 1 ? FLF_MAC_UNR2_FB1 : FLF_MAC_UNR2) : FLF_MAC_UNR;
+    using M = MacShape<SLOTS, NS>;
+    constexpr int NH = M::NH, NPT = M::NPT, UPG = M::UPG, FB = M::FB, NF = M::NF, NT = M::NT, MAC_KB = M::KB, MAC_RING = M::RING;
+    extern __shared__ uint4 mac_lds[];
+    char* T = reinterpret_cast<char*>(mac_lds);                   // [2 stages][hi, lo][residue][unit][column], 16 bytes each
+    float2* Es = reinterpret_cast<float2*>(T + 4 * M::TAB * 16);
+    ushort4* wpos = reinterpret_cast<ushort4*>(Es + M::E);        // [item]: GridTables::wpos
+    unsigned* prs = reinterpret_cast<unsigned*>(wpos + FLF_CHUNK_MAX);   // [spectrum][pair type]: GridTables::pairs, 16 bits each
+    float* inv = reinterpret_cast<float*>(prs + M::PAIRS);        // [2 planes][frame]
+    float2* psis = reinterpret_cast<float2*>(inv + 2 * FB);       // [wave][NH][5], see k_spec_pack
+
     const ChunkDesc* ch = a.chunks + cidx;
     const long long item_base = ch->item_base;
-    const int n_items = ch->n_items;
-    const int tid = threadIdx.x;
-    // IPT = 2 or 4: a group of IPT lanes owns IPT items that share their
-    // residues and splits the stored spectra between its lanes (lane lsub
-    // takes u = lsub, lsub + IPT, ...), so every P/M table read serves IPT
-    // items while the workgroup keeps one thread per item slot; the group
-    // adds its partial sums before each plane's epilogue.
-    static_assert(IPT == 1 || IPT == 2 || IPT == 4, "items per lane group: 1, 2 or 4");
-    constexpr int USTEP = IPT;
-    const int lsub = tid % USTEP;
-    const int slot = tid / USTEP;
-    const bool valid = slot * IPT < n_items;
-    const int tsafe = valid ? slot : 0;          // idle lanes read item 0 (in bounds) and never write
-    const int N = a.N, NN = N * N, fourN = 4 * N;
+    const int n_items = __builtin_amdgcn_readfirstlane(ch->n_items);
+    const int n_tiles = __builtin_amdgcn_readfirstlane(ch->n_tiles);
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, kq = lane >> 4;    // operand column / row, K group
+    const int jj = col / M::COLS;                 // this lane's output column: slot jj + NS t of operand t,
+    const int f = (col % M::COLS) >> 1, c = col & 1;              // frame, component
+    const int NN = a.N * a.N;
     const int t0 = fblock * FB;
-    const int nf = min(FB, a.T - t0);            // frames of this block (block-uniform)
-    const int nu = a.nu;
-    // Residue rows are a.rs = nu*NPT + pad entries apart, rs = 1 (mod 16):
-    // threads of one wave read the same (u, pair type) entry of up to 8
-    // different residues, which then fall on distinct LDS banks.
-    const int rs = a.rs;
-    const int tab = NRES * rs;                    // table entries per frame
-    float2* s_stage = reinterpret_cast<float2*>(pm_tab + FB * tab);   // [FB][NN][NH]
-    float2* psi = s_stage + FB * NN * NH;                                   // [NRES][2]
-    // The item descriptors are re-read (from the caches) where they are
-    // needed instead of living in registers across the spectrum loop.
-    const ItemDesc* itp = a.items + item_base + (long long)tsafe * IPT;
-    int rb[4];
-    {
-        const ItemDesc i0 = itp[0];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) rb[j] = i0.res[j] * rs;
-    }
-    // The descriptor pointer plus an opaque zero, so that the compiler does
-    // not hoist the epilogue's loads out of the plane loop.  The pointer
-    // itself stays transparent: the compiler knows it addresses global
-    // memory and emits global loads (FLAT loads would make every later
-    // vector-memory wait drain all loads in flight, the next spectrum batch
-    // included).
-    auto items_now = [&]() {
-        int z = 0;
-        asm volatile("" : "+v"(z));
-        return itp + z;
-    };
+    const int nf = min(FB, a.T - t0);             // frames of this block
+    const int nu = a.nu, KG = a.kg;
+    const int nkr = (KG + 3) / 4;                 // K steps with data
+    const int nks = (nkr + MAC_RING - 1) / MAC_RING * MAC_RING;   // a multiple of the ring (zeros in the table)
+    const int nbatch = (nks + MAC_KB - 1) / MAC_KB;               // table batches per plane
 
-    constexpr int QT = 1;                         // items whose totals a lane keeps
-    float2 tot[FB][QT][4];
+    // This wave's tile (waves without one repeat tile 0 and store nothing).
+    const bool active = wv < n_tiles;
+    const TileDesc td = a.tiles[ch->tile_base + (active ? wv : 0)];
+    const int start = __builtin_amdgcn_readfirstlane(td.start);
+    const int count = __builtin_amdgcn_readfirstlane(td.count);
+    // Per operand t, for this lane's slot j = jj + NS t (wave-uniform for NS = 1):
+    int tb[NF];                                   // byte offset of its table unit, K step 0
+    bool cj[NF];                                  // it lies on a negated residue
+    unsigned mlo[NF], mhi[NF];                    // sign of M for pair types 0, 1 and 2, 3
+    const bool cj0 = (int)td.res[0] >= NH;
 #pragma unroll
-    for (int f = 0; f < FB; ++f)
+    for (int t = 0; t < NF; ++t) {
+        int q = __builtin_amdgcn_readfirstlane((int)td.res[NS * t]);
 #pragma unroll
-        for (int q = 0; q < QT; ++q)
+        for (int s = 1; s < NS; ++s) q = jj == s ? __builtin_amdgcn_readfirstlane((int)td.res[NS * t + s]) : q;
+        cj[t] = q >= NH;
+        tb[t] = ((cj[t] ? q - NH : q) * M::RS + kq * M::COLS + 2 * f + c) * 16;
+        mlo[t] = cj[t] != cj0 ? 0x80000000u : 0u;
+        mhi[t] = mlo[t] ^ (SLOTS == 4 && ((jj + NS * t) & 1) ? 0x80000000u : 0u);
+    }
+    // A operand rows: lane l holds item l % 16 of each 16-item half of the
+    // tile (rows past the tile repeat its last item; their results are unused)
+    // and unit l / 16 of the K step, as byte offsets; in the last step with
+    // data, units past the last one repeat it (against zeros in the table).
+    unsigned ao[2], al[2];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) tot[f][q][j] = make_float2(0.f, 0.f);
+    for (int h = 0; h < 2; ++h) {
+        const int row = start + min(16 * h + col, count - 1);
+        ao[h] = (unsigned)(kq * 2 * n_items + row) * 16;
+        al[h] = (unsigned)(min(kq, KG - 1 - 4 * (nkr - 1)) * 2 * n_items + row) * 16;
+    }
 
     // Planes of this workgroup: an even share of the group's nP planes for
     // nranges plane ranges (nranges = nP gives one plane per workgroup).
     const int pb = (int)(((long long)range * a.nP) / nranges);
     const int pe = (int)(((long long)(range + 1) * a.nP) / nranges);
-    const long long ustride = (long long)n_items * SLOTS;
-    const int nul = (nu + USTEP - 1) / USTEP;     // spectra per lane and plane
-    const int nb = (nul + UNR - 1) / UNR;         // spectrum batches per plane
-
-    // Per-plane set-up: flip factors, then per frame stage the chunk's
-    // small-FFT block and build its P/M table (all threads; contains
-    // barriers; frames past nf keep the tables of earlier planes and their
-    // accumulators are never stored).
-    auto prologue = [&](int p) {
-        mac_tables<SLOTS>(a, ch, cidx, p, t0, nf, pm_tab, s_stage, psi, rs);
+    auto next_plane = [&](int p) {
+        while (p < pe && !a.enable.on(p)) ++p;
+        return p;
     };
 
-    auto gbase = [&](int p) { return a.G + item_base * SLOTS * nu * a.nP + ((long long)p * nu) * ustride; };
-    // Loads of one batch; spectra past nu re-read the last one (in bounds, unused).
-    auto load_batch = [&](float2 (&g)[UNR][IPT][4], int p, int b) {
-        const float2* Gp = gbase(p);
-#pragma unroll
-        for (int k = 0; k < UNR; ++k) {
-            const int u = min((b * UNR + k) * USTEP + lsub, nu - 1);
-#pragma unroll
-            for (int q = 0; q < IPT; ++q) load_g<SLOTS>(g[k][q], Gp + u * ustride, tsafe * IPT + q, n_items);
-        }
+    const char* Gc = reinterpret_cast<const char*>(a.G) + item_base * a.nP * KG * 32;
+    const long long gplane = (long long)KG * n_items * 32;
+    auto load_a = [&](v4u (&q)[4], int p, int ks) {
+        const int k = min(ks, nkr - 1);
+        const char* b = Gc + p * gplane + (long long)k * n_items * 128;
+        const bool last = k == nkr - 1;
+        const unsigned o0 = last ? al[0] : ao[0], o1 = last ? al[1] : ao[1];
+        q[0] = *reinterpret_cast<const v4u*>(b + o0);
+        q[1] = *reinterpret_cast<const v4u*>(b + n_items * 16 + o0);
+        q[2] = *reinterpret_cast<const v4u*>(b + o1);
+        q[3] = *reinterpret_cast<const v4u*>(b + n_items * 16 + o1);
     };
 
-    // Store the totals at A + slice * A_pstride (each lane of a pair stores
-    // its own item), frames of this block only.
-    auto store = [&](int slice) {
-        const auto ip = items_now();
+    // ---- the table, one stage = (plane, batch of K steps) ----
+    // Thread's entries: q = tid + 512 k -> pair type, frame, spectrum.
+    // (from an opaque copy of the thread id at each use, so that what follows
+    // from it is not kept in registers across the plane loop)
+    constexpr int ESTEP = MAC_THREADS / (NPT * FB);
+    struct Entry {
+        int pt, f, u;
+    };
+    auto entry = [&]() {
+        int t = tid;
+        asm volatile("" : "+v"(t));
+        return Entry{t & (NPT - 1), (t / NPT) & (FB - 1), t / (NPT * FB)};
+    };
+    float2* psi = psis + wv * 5 * NH;
+    auto use_of = [&](int b, int ul, int pt) {    // the entry's plain and conjugated use (past the last spectrum: zeros)
+        const int u = b * (MAC_KB * 4 * UPG) + ul;
+        const unsigned w = prs[min(u, nu - 1) * NPT + pt];
+        return u < nu && ul < MAC_KB * 4 * UPG ? make_int2(w & 0xffff, w >> 16) : make_int2(4, 4);
+    };
+    v4f sp[NT][NH / 2], sc[NT][NH / 2];           // small-FFT values of the plain and conjugated use, all residues
+    float2 ps;                                    // flip factor of lane < 5 NH
+    v4f smx[FLF_SMAX_WAYS / 4];                   // largest small-FFT components of the entry's frame
+    auto fetch = [&](int p, int b) {
+        const char* sb = reinterpret_cast<const char*>(a.S + p * a.S_pstride + (long long)t0 * a.S_tstride +
+                                                       (long long)cidx * NN * NH);
+        const Entry en = entry();
+        const int fc = min(en.f, nf - 1);
+        const unsigned fo = (unsigned)(fc * a.S_tstride * 8);
+        ps = a.psi[((long long)cidx * a.nP + p) * 5 * NH + min(lane, 5 * NH - 1)];
+        const v4f* sm = reinterpret_cast<const v4f*>(a.smax + ((long long)p * a.smax_pstride + t0 + fc) * FLF_SMAX_WAYS);
 #pragma unroll
-        for (int f = 0; f < FB; ++f) {
-            if (f >= nf) break;
-            float2* A = a.A + (long long)(t0 + f) * a.A_tstride + (long long)slice * a.A_pstride;
+        for (int i = 0; i < FLF_SMAX_WAYS / 4; ++i) smx[i] = sm[i];
 #pragma unroll
-            for (int q = 0; q < QT; ++q) {
-                const ItemDesc& it = ip[IPT >= 2 ? lsub : q];
+        for (int k = 0; k < NT; ++k) {
+            const int2 pr = use_of(b, en.u + k * ESTEP, en.pt);
+            const v4f* x = reinterpret_cast<const v4f*>(sb + (fo + (unsigned)(pr.x & ~7) * NH));
+            const v4f* y = reinterpret_cast<const v4f*>(sb + (fo + (unsigned)(pr.y & ~7) * NH));
 #pragma unroll
-                for (int j = 0; j < SLOTS; ++j)
-                    if ((it.writemask >> j) & 1) A[it.pos[j]] = tot[f][q][j];
+            for (int r = 0; r < NH / 2; ++r) {
+                sp[k][r] = x[r];
+                sc[k][r] = y[r];
             }
         }
     };
-
-    float2 acc[FB][IPT][4];
-    // Epilogue of plane p: outer phase and the 'same'-crop shift.
-    auto epilogue = [&](int p) {
-        const int s2 = const_load(a.s2, p);
-        const int sig = s2 - 2 + N;
-        const int c2 = (s2 - 1) / 2;
-        // IPT = 2: each lane keeps its own item (q = lsub): it sends the
-        // partner's item and adds what the partner sends for its own.
-        // IPT = 4: the same in two steps, first between lanes lsub and
-        // lsub ^ 2 (each keeps the two items whose bit 1 is its own), then
-        // between lsub and lsub ^ 1.
-        float2 own[FB][4];
-        if constexpr (IPT == 2) {
+    // The thread's entries of the table of stage st (a plane of parity par).
+    // The frame's scale brings the largest small-FFT component of the plane
+    // into [2^13, 2^14): P and M components, at most 2^1.5 times as large,
+    // stay within fp16, and values down to 2^-17 of the largest keep all 23
+    // bits of the split.
+    auto convert = [&](int b, int st, int par) {
+        const Entry en = entry();
+        float m = 0.f;
 #pragma unroll
-            for (int f = 0; f < FB; ++f)
+        for (int i = 0; i < FLF_SMAX_WAYS / 4; ++i) m = fmaxf(fmaxf(m, fmaxf(smx[i][0], smx[i][1])), fmaxf(smx[i][2], smx[i][3]));
+        const int e = scale_exp(m, 13);
+        const float s = exp2_int(e);
+        if (tid < NPT * FB && en.pt == 0) inv[par * FB + en.f] = exp2_int(-e);
+        if (lane < 5 * NH) psi[lane] = ps;
+        wave_sync();
+        // dword (residue, unit, column, pair type) of the table's halves
+        unsigned* hi = reinterpret_cast<unsigned*>(T + st * (2 * M::TAB * 16));
+        unsigned* lo = hi + 4 * M::TAB;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float2 mine = lsub ? acc[f][1][j] : acc[f][0][j];
-                    const float2 give = lsub ? acc[f][0][j] : acc[f][1][j];
-                    own[f][j] = make_float2(mine.x + __shfl_xor(give.x, 1), mine.y + __shfl_xor(give.y, 1));
-                }
-        } else if constexpr (IPT == 4) {
-            const bool hi = (lsub & 2) != 0, odd = (lsub & 1) != 0;
+        for (int k = 0; k < NT; ++k) {
+            const int ul = en.u + k * ESTEP;
+            if ((NT * ESTEP == MAC_KB * 4 * UPG || ul < MAC_KB * 4 * UPG) && en.f < nf) {
+                const int2 pr = use_of(b, ul, en.pt);
+                const int d0 = ((ul / UPG) * M::COLS + 2 * en.f) * 4 + (SLOTS == 4 ? en.pt : 2 * (ul & 1) + en.pt);
 #pragma unroll
-            for (int f = 0; f < FB; ++f)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    float2 k[2];
-#pragma unroll
-                    for (int c = 0; c < 2; ++c) {
-                        const float2 keep = hi ? acc[f][2 + c][j] : acc[f][c][j];
-                        const float2 give = hi ? acc[f][c][j] : acc[f][2 + c][j];
-                        k[c] = make_float2(keep.x + __shfl_xor(give.x, 2), keep.y + __shfl_xor(give.y, 2));
-                    }
-                    const float2 mine = odd ? k[1] : k[0];
-                    const float2 give = odd ? k[0] : k[1];
-                    own[f][j] = make_float2(mine.x + __shfl_xor(give.x, 1), mine.y + __shfl_xor(give.y, 1));
-                }
-        }
-        const auto ip = items_now();
-#pragma unroll
-        for (int q = 0; q < QT; ++q) {
-            const ItemDesc itq = ip[IPT >= 2 ? lsub : q];
-            const int m2 = itq.m2[0], n2 = itq.n2[0];
-            int outer[4];
-            outer[0] = sig * (m2 + n2);
-            outer[1] = sig * (n2 - m2);
-            outer[2] = sig * (n2 + m2);
-            outer[3] = sig * (m2 - n2);
-#pragma unroll
-            for (int j = 0; j < SLOTS; ++j) {
-                const int k0 = itq.pos[j] / a.rfX, k1 = itq.pos[j] - k0 * a.rfX;
-                const float2 po = phase_frac_i(outer[j], fourN);
-                // exp(+2 pi i c2 (k0/fY + k1/fX))
-                // c2 < f / 2 and k < f <= FLF_MAX_FOURIER: 32-bit products
-                const int e0 = (c2 * k0) % a.fY;
-                const int e1 = (c2 * k1) % a.fX;
-                float fr = (float)e0 / (float)a.fY + (float)e1 / (float)a.fX;
-                fr -= rintf(fr);
-                float sn, cs;
-                sincospif(2.0f * fr, &sn, &cs);
-                const float2 pc = make_float2(cs, sn);
-#pragma unroll
-                for (int f = 0; f < FB; ++f) {
-                    const float2 av = IPT >= 2 ? own[f][j] : acc[f][q][j];
-                    tot[f][q][j] = cadd(tot[f][q][j], cmul(cmul(av, po), pc));
+                for (int r = 0; r < NH; ++r) {
+                    const v4f vp = sp[k][r / 2], vc = sc[k][r / 2];
+                    const float2 x = cmul(r & 1 ? make_float2(vp.z, vp.w) : make_float2(vp.x, vp.y), psi[5 * r + (pr.x & 7)]);
+                    const float2 y = cmul(r & 1 ? make_float2(vc.z, vc.w) : make_float2(vc.x, vc.y), psi[5 * r + (pr.y & 7)]);
+                    const float2 P = cadd(x, y);
+                    const float2 d = csub(x, y);                               // M = i d = (-d.y, d.x)
+                    const float p0 = P.x * s, p1 = P.y * s, m0 = -d.y * s, m1 = d.x * s;
+                    const int o = r * (4 * M::RS) + d0;
+                    hi[o] = pack_half2(p0, m0);
+                    hi[o + 4] = pack_half2(p1, m1);
+                    lo[o] = pack_half2(half_rest(p0), half_rest(m0));
+                    lo[o + 4] = pack_half2(half_rest(p1), half_rest(m1));
                 }
             }
-        }
-        if (a.per_plane) {                       // back projection: one output per plane
-            if (valid) store(p);
-#pragma unroll
-            for (int f = 0; f < FB; ++f)
-#pragma unroll
-                for (int q = 0; q < QT; ++q)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) tot[f][q][j] = make_float2(0.f, 0.f);
+            __builtin_amdgcn_sched_barrier(0);    // one entry's values live at a time
         }
     };
 
-    // Software pipeline over (plane, batch): the loads of the next batch (also
-    // across a plane boundary, i.e. before the next plane's set-up) are in
-    // flight while the current batch is accumulated.
-    int p = pb;
-    while (p < pe && !a.enable.on(p)) ++p;
-    if (p < pe) {
-        float2 gA[UNR][IPT][4], gB[UNR][IPT][4];
-        load_batch(gA, p, 0);
-        int b = 0;
-        auto step = [&](float2 (&cur)[UNR][IPT][4], float2 (&nxt)[UNR][IPT][4]) -> bool {
-            // The current batch (and anything older) has landed: the only
-            // loads in flight during the accumulation below are the next
-            // batch's and the staging copy (which writes no registers).
-            wait_vmem_all();
-            if (b == 0) {
-                prologue(p);
+    v4f tot[2][NF], acc[2][NF];
 #pragma unroll
-                for (int f = 0; f < FB; ++f)
+    for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-                    for (int q = 0; q < IPT; ++q)
+        for (int t = 0; t < NF; ++t) tot[rt][t] = acc[rt][t] = v4f{0.f, 0.f, 0.f, 0.f};
+
+    // Store v[rt][t] (component c of frame f, slot jj + NS t) at A + slice *
+    // A_pstride.  The accumulators lie chunk by chunk, a chunk's bins by
+    // column (GridTables::wpos), the block's frames interleaved: a workgroup
+    // writes one contiguous run, which L2 holds together.  (In the natural
+    // order of the grid a chunk's bins lie rX columns apart; the neighbours
+    // of an 8-byte bin came from other workgroups, after L2 had evicted its
+    // line: 49 million write requests per 1455^2 x 41-plane back projection
+    // where 7 million lines hold the data.)  Of a lane pair (re, im) the even
+    // lane writes row r's bin and the odd lane row r + 1's.  The positions come
+    // from LDS: a load from memory here would wait for every A operand in
+    // flight, which under load takes as long as a plane.
+    auto store = [&](const v4f (&v)[2][NF], int slice) {
+        // uniform base, 32-bit lane offsets
+        char* A = reinterpret_cast<char*>(a.A + (long long)t0 * a.A_tstride + (long long)slice * a.A_pstride +
+                                          item_base * SLOTS * nf);
+        const unsigned fo = 8 * f, bs = 8 * nf;
+        int z = 0;
+        asm volatile("" : "+v"(z));               // (the rows' addresses are not kept across the plane loop)
+        const int k4 = 4 * kq + c + z;
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) acc[f][q][j] = make_float2(0.f, 0.f);
+        for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int i = 16 * rt + k4 + 2 * h;
+                const unsigned short* ws = reinterpret_cast<const unsigned short*>(wpos + start + min(i, count - 1)) + jj;
+                const bool in = active && f < nf && i < count;
+#pragma unroll
+                for (int t = 0; t < NF; ++t) {
+                    const unsigned w = ws[NS * t];
+                    const float got = lane_xor1(c ? v[rt][t][2 * h] : v[rt][t][2 * h + 1]);
+                    const float2 o = c ? make_float2(got, v[rt][t][2 * h + 1]) : make_float2(v[rt][t][2 * h], got);
+                    if (in && w != 0xffff) *reinterpret_cast<float2*>(A + (fo + bs * w)) = o;
+                }
+                __builtin_amdgcn_sched_barrier(0);        // one row pair's addresses live at a time
             }
-            int pn = p, bn = b + 1;
-            if (bn == nb) {
-                bn = 0;
-                pn = p + 1;
-                while (pn < pe && !a.enable.on(pn)) ++pn;
-            }
-            if (pn < pe) load_batch(nxt, pn, bn);
+    };
+
+    // Products of one K step: the B operand of slot j is its residue's unit with
+    // the dwords (pair types) in the order i XOR j.
+    auto products = [&](const v4u (&q)[4], const char* tk) {
 #pragma unroll
-            for (int k = 0; k < UNR; ++k) {
-                const int u = (b * UNR + k) * USTEP + lsub;
-                if (u < nu) mac_spectrum<SLOTS, IPT, FB>(acc, cur[k], pm_tab, tab, rb, u);
+        for (int t = 0; t < NF; ++t) {
+            v4u b[2];
+            b[0] = *reinterpret_cast<const v4u*>(tk + tb[t]);
+            b[1] = *reinterpret_cast<const v4u*>(tk + tb[t] + M::TAB * 16);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                v4u d = b[h];
+                if constexpr (SLOTS == 4) {
+                    d[0] ^= mlo[t];
+                    d[1] ^= mlo[t];
+                    d[2] ^= mhi[t];
+                    d[3] ^= mhi[t];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) d[i] ^= mlo[t];
+                }
+                if constexpr (NS == 1) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) b[h][i] = d[i ^ t];
+                } else {
+                    const bool odd = jj & 1;      // bit 0 of the slot by lane, bit 1 by lane (NS = 4) or operand
+                    v4u e;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) e[i] = odd ? d[i ^ 1] : d[i];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) b[h][i] = NS == 4 ? (jj & 2 ? e[i ^ 2] : e[i]) : e[i ^ (2 * t)];
+                }
             }
-            if (b == nb - 1) epilogue(p);
-            p = pn;
-            b = bn;
-            return pn < pe;
-        };
-        while (step(gA, gB) && step(gB, gA)) {
+            // hi*hi into the accumulators; the small products lo*hi + hi*lo +
+            // lo*lo on their own first, one fp32 addition for all of them
+            const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
+            v4f x0 = mfma_f16(q[1], b[0], zero), x1 = mfma_f16(q[3], b[0], zero);
+            acc[0][t] = mfma_f16(q[0], b[0], acc[0][t]);
+            acc[1][t] = mfma_f16(q[2], b[0], acc[1][t]);
+            x0 = mfma_f16(q[0], b[1], x0);
+            x1 = mfma_f16(q[2], b[1], x1);
+            x0 = mfma_f16(q[1], b[1], x0);
+            x1 = mfma_f16(q[3], b[1], x1);
+            acc[0][t] += x0;
+            acc[1][t] += x1;
         }
+    };
+
+    int p = next_plane(pb);
+    if (p >= pe && PER_PLANE) return;
+    v4u ring[MAC_RING][4];
+    if (p < pe)
+#pragma unroll
+        for (int d = 0; d < MAC_RING; ++d) load_a(ring[d], p, d);
+    if (tid < n_items) wpos[tid] = a.wpos[item_base + tid];
+    for (int i = tid; i < nu * NPT; i += MAC_THREADS) {
+        const int2 w = a.pairs[i];
+        prs[i] = (unsigned)w.x | (unsigned)w.y << 16;
     }
+    __syncthreads();
+    if (p >= pe) {                                // no plane enabled: a sum of zeros
+        store(tot, range);
+        return;
+    }
+    fetch(p, 0);
+    convert(0, 0, 0);
 
-    if (valid && !a.per_plane) store(range);
+    float2* Ew = Es + wv * FLF_TILE * SLOTS;      // this wave's output factors
+    int b = 0, st = 0, par = 0;
+    while (true) {
+        // Every wave's part of this stage's table is written, and every wave is
+        // done with the previous stage's, which convert() below overwrites.
+        __syncthreads();
+        const bool lastb = b + 1 == nbatch;
+        const int pa = next_plane(p + 1);
+        const int pl = pa < pe ? pa : p;          // plane of the loads past this one's last step
+        const int pn = lastb ? pa : p, bn = lastb ? 0 : b + 1;
+        const bool more = pn < pe;
+        // The next stage's small-FFT values and this plane's output factors are
+        // in flight during this stage's products.  No branch surrounds a load
+        // here (past the last stage they load something in bounds, unused), so
+        // that the compiler's waits leave the newer loads in flight.
+        fetch(more ? pn : p, bn);
+        const v4u ev = reinterpret_cast<const v4u*>(a.E + (item_base * a.nP + (long long)p * n_items + start) *
+                                                              SLOTS)[min(lane, count * SLOTS / 2 - 1)];
+        const int kse = min((b + 1) * MAC_KB, nks);
+        const char* tk = T + st * (2 * M::TAB * 16);
+        int k0 = b * MAC_KB;
+        do {                                      // (at least one turn: no path around the loads)
+#pragma unroll
+            for (int d = 0; d < MAC_RING; ++d) {
+                // step ks uses slot ks % MAC_RING; past the last step the slots
+                // take the next plane's first steps
+                const int ks = k0 + d;
+                products(ring[d], tk + d * (4 * M::COLS * 16));
+                const bool in = ks + MAC_RING < nks;
+                load_a(ring[d], in ? p : pl, in ? ks + MAC_RING : d);
+                if constexpr (M::WAVES == 4) __builtin_amdgcn_sched_barrier(0);   // one step's operands live at a time
+            }
+            k0 += MAC_RING;
+            tk += MAC_RING * 4 * M::COLS * 16;
+        } while (k0 < kse);
+        // Epilogue of the plane.  Lane l holds D[item 4 (l / 16) + r][column
+        // l % 16]; the other component of its frame is in lane l ^ 1.
+        if (lastb) {
+            if (lane < FLF_TILE * SLOTS / 2) reinterpret_cast<v4u*>(Ew)[lane] = ev;
+            wave_sync();
+            int z = 0;
+            asm volatile("" : "+v"(z));           // (the rows' addresses are not kept across the plane loop)
+            const float is = inv[par * FB + min(f, nf - 1)];
+            float q1[NF], q2[NF];
+#pragma unroll
+            for (int t = 0; t < NF; ++t) {
+                const float sg = cj[t] ? -1.f : 1.f;
+                q1[t] = c ? sg * is : is;         // times own component x factor.x
+                q2[t] = c ? is : -sg * is;        // times other component x factor.y
+            }
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int i = min(16 * rt + 4 * kq + r + z, count - 1);
+#pragma unroll
+                    for (int t = 0; t < NF; ++t) {
+                        const float2 e = Ew[i * SLOTS + jj + NS * t];
+                        const float mine = acc[rt][t][r];
+                        const float other = lane_xor1(mine);
+                        const float v = fmaf(q1[t], mine * e.x, q2[t] * (other * e.y));
+                        if constexpr (PER_PLANE) acc[rt][t][r] = v;
+                        else tot[rt][t][r] += v;
+                    }
+                    __builtin_amdgcn_sched_barrier(0);    // one row's factors live at a time
+                }
+            if constexpr (PER_PLANE) store(acc, p);
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+                for (int t = 0; t < NF; ++t) acc[rt][t] = v4f{0.f, 0.f, 0.f, 0.f};
+        }
+        if (!more) break;
+        par = lastb ? par ^ 1 : par;
+        st ^= 1;
+        convert(bn, st, par);
+        p = pn;
+        b = bn;
+    }
+    if constexpr (!PER_PLANE) store(tot, range);
 }
 
 // Block id w in [0, R * nfb) -> frame block and the rest r in [0, R):
@@ -827,17 +947,18 @@ __device__ __forceinline__ void split_frames(int w, int R, int nfb, int S, int& 
     r = rem / sc;
 }
 
-template <int SLOTS, int IPT, int FB>
-__global__ __launch_bounds__(FLF_CHUNK_MAX) __attribute__((amdgpu_waves_per_eu(IPT * FB >= 3 ? 2 : (IPT * FB == 2 ? 3 : FLF_MAC_WAVES))))
+template <int SLOTS, int NS, bool PER_PLANE>
+__global__ __launch_bounds__(MAC_THREADS) __attribute__((amdgpu_waves_per_eu(MacShape<SLOTS, NS>::WAVES)))
 void k_mac(MacArgs a) {
     // grid x = chunk x frame block, frame blocks of a chunk consecutive (in
     // super-blocks of a.fgroup): after the XCD remap they share one XCD's L2
     // for the spectra they all read
+    constexpr int FB = MacShape<SLOTS, NS>::FB;
     const int nfb = (a.T + FB - 1) / FB;
     const int w = xcd_block(blockIdx.x, gridDim.x);
     int fblock, cidx;
     split_frames(w, gridDim.x / nfb, nfb, a.fgroup, fblock, cidx);
-    mac_body<SLOTS, IPT, FB>(a, cidx, blockIdx.y, gridDim.y, fblock);
+    mac_body<SLOTS, NS, PER_PLANE>(a, cidx, blockIdx.y, gridDim.y, fblock);
 }
 
 // All active grid groups of one projection: grid x flattened over (group,
@@ -852,8 +973,8 @@ void k_mac(MacArgs a) {
 // once from HBM for all of them.  fgroup < nfb dispatches them in
 // super-blocks of fgroup instead, so that more chunks run side by side
 // (their scattered accumulator stores then combine in L2 more often).
-template <int SLOTS, int IPT, int FB>
-__global__ __launch_bounds__(FLF_CHUNK_MAX) __attribute__((amdgpu_waves_per_eu(IPT * FB >= 3 ? 2 : (IPT * FB == 2 ? 3 : FLF_MAC_WAVES))))
+template <int SLOTS, int NS, bool PER_PLANE>
+__global__ __launch_bounds__(MAC_THREADS) __attribute__((amdgpu_waves_per_eu(MacShape<SLOTS, NS>::WAVES)))
 void k_mac_grouped(MacGrouped ga) {
     const GroupPick p = pick_group(ga.gg, blockIdx.x);
     const int w = xcd_block(p.rem, p.n);
@@ -861,333 +982,73 @@ void k_mac_grouped(MacGrouped ga) {
     if (w >= R * ga.nfb) return;                  // padding
     int fblock, r;
     split_frames(w, R, ga.nfb, ga.a[p.g].fgroup, fblock, r);
-    mac_body<SLOTS, IPT, FB>(ga.a[p.g], r % p.nch, r / p.nch, p.nr, fblock);
-}
-
-// Matrix-core multiply-accumulate, TC_FB = 8 frames per workgroup
-// (v_mfma_f32_16x16x4_f32: FP32 operands and accumulation, as the vector
-// kernel).  The pair type of source slot i at output slot j is i XOR j
-// (kQuadPT, kPairPT), so with the P/M table of one residue rho as the B
-// operand,
-//   out_j[item][(f, c)] = sum_{u, pt, r} A_j[item][(u, pt, r)] B_rho[(u, pt, r)][(f, c)],
-//   B_rho[(u, pt, Re)][(f, c)] = P_c,   B_rho[(u, pt, Im)][(f, c)] = M_c,
-//   A_j[item][(u, pt, r)] = component r of the stored value of slot pt XOR j
-//                           (times the M sign of (j, i) for r = Im),
-// one B per residue serves every output slot and every item of that
-// residue; the per-slot permutation is a choice between two registers of
-// the A operand.  Items come in tiles of <= 16 of one residue class
-// (TileDesc), so each slot's residue is uniform within a tile.  B lives in
-// LDS in the MFMA's operand order (lane l reads float l of a 64-float block:
-// no bank conflicts), built per batch of TC_UB stored spectra from the
-// cached small-FFT values; lane l supplies A[l % 16][l / 16] (its tile row's
-// item, read from the cached spectra: each value once per frame block) and
-// holds D[4 (l / 16) + r][l % 16] (items 4 (l / 16) + r, column (f, c) =
-// l % 16).  Wave w owns tiles w, w + TC_WAVES, ...
-constexpr int TC_FB = 8;
-constexpr int TC_WAVES = 8;
-constexpr int TC_UB = 12;
-template <int SLOTS>
-__global__ __launch_bounds__(64 * TC_WAVES) void k_mac_tc(MacArgs a) {
-    extern __shared__ float4 tc_lds[];
-    constexpr int NRES = SLOTS == 4 ? 8 : 4;
-    constexpr int NH = NRES / 2;
-    constexpr int NPT = SLOTS == 4 ? 4 : 2;
-    constexpr int KS = SLOTS / 2;                 // 4-deep k steps per stored spectrum
-    constexpr int NUSE = SLOTS == 4 ? 8 : 4;
-    constexpr int MAXT = (FLF_MAX_TILES + TC_WAVES - 1) / TC_WAVES;
-    float* Bt = reinterpret_cast<float*>(tc_lds);                          // [TC_UB][NRES][KS][64]
-    float2* psi = reinterpret_cast<float2*>(Bt + TC_UB * NRES * KS * 64);  // [NRES][2]
-    float2* s_stage = psi + 2 * NRES;                                      // [TC_FB][N*N][NH]
-    // grid x = chunk x frame block, frame block fastest (as k_mac)
-    const int nfb = (a.T + TC_FB - 1) / TC_FB;
-    const int wblk = xcd_block(blockIdx.x, gridDim.x);
-    const int cidx = wblk / nfb;
-    const ChunkDesc* ch = a.chunks + cidx;
-    const long long item_base = ch->item_base;
-    const int n_items = ch->n_items;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int row = lane & 15, kq = lane >> 4;
-    const int col = row, f_col = col >> 1, c_col = col & 1;
-    const int N = a.N, NN = N * N, c = N / 2, fourN = 4 * N;
-    const int t0 = (wblk - cidx * nfb) * TC_FB;
-    const int nf = min(TC_FB, a.T - t0);
-    const int nu = a.nu;
-    const TileDesc* tiles = a.tiles + ch->tile_base;
-    const int ntiles = ch->n_tiles;
-    const long long ustride = (long long)n_items * SLOTS;
-
-    int it_of[MAXT];                              // this lane's A-row item (chunk-relative), -1 if none
-#pragma unroll
-    for (int q = 0; q < MAXT; ++q) {
-        const int tq = wv + TC_WAVES * q;
-        it_of[q] = -1;
-        if (tq < ntiles) {
-            const TileDesc td = tiles[tq];
-            if (row < td.count) it_of[q] = td.start + row;
-        }
-    }
-    v4f tot[MAXT][SLOTS];
-#pragma unroll
-    for (int q = 0; q < MAXT; ++q)
-#pragma unroll
-        for (int j = 0; j < SLOTS; ++j) tot[q][j] = v4f{0.f, 0.f, 0.f, 0.f};
-
-    // Store: lane (f, c) writes component c of its items' slot-j bins.
-    auto store = [&](int slice) {
-        if (f_col >= nf) return;
-        float* A = reinterpret_cast<float*>(a.A + (long long)(t0 + f_col) * a.A_tstride +
-                                            (long long)slice * a.A_pstride);
-#pragma unroll
-        for (int q = 0; q < MAXT; ++q) {
-            const int tq = wv + TC_WAVES * q;
-            if (tq >= ntiles) continue;                                   // wave-uniform
-            const TileDesc td = tiles[tq];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int ir = 4 * kq + r;
-                if (ir < td.count) {
-                    const ItemDesc& it = a.items[item_base + td.start + ir];
-#pragma unroll
-                    for (int j = 0; j < SLOTS; ++j)
-                        if ((it.writemask >> j) & 1) A[2LL * it.pos[j] + c_col] = tot[q][j][r];
-                }
-            }
-        }
-    };
-
-    const int pb = (int)(((long long)blockIdx.y * a.nP) / gridDim.y);
-    const int pe = (int)(((long long)(blockIdx.y + 1) * a.nP) / gridDim.y);
-    for (int p = pb; p < pe; ++p) {
-        if (!a.enable.on(p)) continue;
-        const int s2 = const_load(a.s2, p);
-        __syncthreads();                          // the previous plane is done with Bt, psi and s_stage
-        if (tid < 2 * NRES) {                     // flip factors per residue: exp(-2 pi i (s2-1) kt / f)
-            const int rho = tid >> 1;
-            const bool isY = (tid & 1) == 0;
-            const int k = isY ? ch->res0[rho] : ch->res1[rho];
-            const int r = isY ? a.rY : a.rX;
-            const int f = isY ? a.fY : a.fX;
-            const int kt = (2 * k < r) ? k : ((2 * k > r) ? k - r : 0);
-            int m = (int)(((long long)(s2 - 1) * kt) % f);
-            if (m < 0) m += f;
-            float sn, cs;
-            sincospif(-2.0f * (float)m / (float)f, &sn, &cs);
-            psi[tid] = make_float2(cs, sn);
-        }
-        v4f acc[MAXT][SLOTS];
-#pragma unroll
-        for (int q = 0; q < MAXT; ++q)
-#pragma unroll
-            for (int j = 0; j < SLOTS; ++j) acc[q][j] = v4f{0.f, 0.f, 0.f, 0.f};
-        const float2* Gp = a.G + item_base * SLOTS * nu * a.nP + ((long long)p * nu) * ustride;
-        // the chunk's small-FFT block of every frame, staged once per plane by
-        // global-to-LDS loads all in flight at once (awaited here; the
-        // barrier at the top of the batch loop makes it visible)
-        mac_stage_async<SLOTS>(a, cidx, p, t0, nf, s_stage);
-        wait_vmem_all();
-        for (int u0 = 0; u0 < nu; u0 += TC_UB) {
-            const int ubn = min(TC_UB, nu - u0);
-            __syncthreads();                      // psi written; the previous batch's products are done
-            // B of spectra u0 .. u0 + ubn - 1: one (P, M) pair per (spectrum,
-            // residue, pair type, frame).  Thread -> column (ub, pt), decoded
-            // once, and a share of the (residue, frame) rows.
-            {
-                constexpr int Q = TC_UB * NPT;
-                constexpr int ROWS = NRES * TC_FB;
-                const int rstep = (int)blockDim.x / Q;
-                const int r0 = tid / Q;
-                const int col = tid - r0 * Q;
-                const int pt = col % NPT, ub = col / NPT;
-                int src[2] = {-1, -1}, flip[2] = {0, 0};
-                if (r0 < rstep && ub < ubn) {
-                    const int u = u0 + ub;
-#pragma unroll
-                    for (int w = 0; w < 2; ++w) {
-                        const int off = a.uoff[u * NUSE + (w == 0 ? kPairPlain[pt] : kPairConj[pt])];
-                        const int bo = off / N, ao = off - bo * N;
-                        src[w] = off < NN ? off * NH : -1;
-                        flip[w] = (bo > c ? 1 : 0) | (ao > c ? 2 : 0);
-                    }
-                }
-                for (int rw = r0; r0 < rstep && rw < ROWS; rw += rstep) {
-                    const int f = rw % TC_FB, rho = rw / TC_FB;
-                    float4 pm = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (ub < ubn && f < nf) {
-                        const int rb0 = rho < NH ? rho : rho - NH;
-                        const float2* sf = s_stage + f * NN * NH;
-                        float2 sv[2];
-#pragma unroll
-                        for (int w = 0; w < 2; ++w) {
-                            float2 r = make_float2(0.f, 0.f);
-                            if (src[w] >= 0) {
-                                r = sf[src[w] + rb0];
-                                if (rho >= NH) r = cconj(r);
-                                if (flip[w] & 1) r = cmul(r, psi[2 * rho]);
-                                if (flip[w] & 2) r = cmul(r, psi[2 * rho + 1]);
-                            }
-                            sv[w] = r;
-                        }
-                        const float2 P = cadd(sv[0], sv[1]);
-                        const float2 d = csub(sv[0], sv[1]);
-                        pm = make_float4(P.x, P.y, -d.y, d.x);                    // M = i * d
-                    }
-                    float* b = Bt + ((ub * NRES + rho) * KS + (pt >> 1)) * 64 + 2 * (pt & 1) * 16 + 2 * f;
-                    b[0] = pm.x;                      // k row 2 (pt & 1): Re g -> P
-                    b[1] = pm.y;
-                    b[16] = pm.z;                     // k row 2 (pt & 1) + 1: Im g -> M
-                    b[17] = pm.w;
-                }
-            }
-            __syncthreads();
-            // Spectra outer, tiles inner: the loads of spectrum ub + 1 for all
-            // of this wave's tiles are in flight during the products of ub.
-            int res_q[MAXT][SLOTS];
-#pragma unroll
-            for (int q = 0; q < MAXT; ++q) {
-                const int tq = min(wv + TC_WAVES * q, ntiles - 1);
-                const TileDesc td = tiles[tq];
-#pragma unroll
-                for (int j = 0; j < SLOTS; ++j) res_q[q][j] = td.res[j];
-            }
-            auto load_u = [&](float2 (&gq)[MAXT][4], int ub) {
-#pragma unroll
-                for (int q = 0; q < MAXT; ++q) {
-                    const int it = it_of[q];
-                    load_g<SLOTS>(gq[q], Gp + (long long)(u0 + ub) * ustride, it >= 0 ? it : 0, n_items);
-                }
-            };
-            float2 gA[MAXT][4], gB[MAXT][4];
-            load_u(gA, 0);
-            auto products = [&](float2 (&gq)[MAXT][4], int ub) {
-                const float* bu = Bt + ub * NRES * KS * 64 + lane;
-#pragma unroll
-                for (int q = 0; q < MAXT; ++q) {
-                    if (wv + TC_WAVES * q >= ntiles) continue;                // wave-uniform
-                    const bool live = it_of[q] >= 0;
-#pragma unroll
-                    for (int j = 0; j < SLOTS; ++j) {
-#pragma unroll
-                        for (int s = 0; s < KS; ++s) {
-                            const int i0 = (2 * s) ^ j, i1 = (2 * s + 1) ^ j;
-                            const float sg0 = SLOTS == 4 ? (float)kQuadSG[j][i0] : 1.0f;
-                            const float sg1 = SLOTS == 4 ? (float)kQuadSG[j][i1] : 1.0f;
-                            const float2 gi = (kq >> 1) ? gq[q][i1] : gq[q][i0];
-                            const float sg = (kq >> 1) ? sg1 : sg0;
-                            const float av = live ? ((kq & 1) ? sg * gi.y : gi.x) : 0.f;
-                            const float bv = bu[(res_q[q][j] * KS + s) * 64];
-                            acc[q][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc[q][j], 0, 0, 0);
-                        }
-                    }
-                }
-            };
-            // The loads are unconditional (past the batch they re-read its
-            // last spectrum, in bounds and unused): with a branch around
-            // them the compiler's single wait before the products would
-            // have to drain the loads just issued.
-            for (int ub = 0; ub < ubn; ub += 2) {
-                load_u(gB, min(ub + 1, ubn - 1));
-                products(gA, ub);
-                load_u(gA, min(ub + 2, ubn - 1));
-                if (ub + 1 < ubn) products(gB, ub + 1);
-            }
-        }
-        // Epilogue of plane p: outer phase and 'same'-crop shift per item and
-        // slot (the same for every frame); (re, im) of a column pair meet by
-        // one lane swap.
-        const int sig = s2 - 2 + N;
-        const int c2 = (s2 - 1) / 2;
-#pragma unroll
-        for (int q = 0; q < MAXT; ++q) {
-            const int tq = wv + TC_WAVES * q;
-            if (tq >= ntiles) continue;                                       // wave-uniform
-            const TileDesc td = tiles[tq];
-#pragma unroll
-            for (int j = 0; j < SLOTS; ++j) {
-                float mine[4], other[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    mine[r] = acc[q][j][r];
-                    other[r] = __shfl_xor(mine[r], 1);
-                }
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int ir = 4 * kq + r;
-                    if (ir < td.count) {
-                        const ItemDesc& it = a.items[item_base + td.start + ir];
-                        const int m2 = it.m2[0], n2 = it.n2[0];
-                        const int outer = j == 0 ? sig * (m2 + n2)
-                                        : j == 1 ? sig * (n2 - m2)
-                                        : j == 2 ? sig * (n2 + m2) : sig * (m2 - n2);
-                        const int pos = it.pos[j];
-                        const int k0 = pos / a.rfX, k1 = pos - k0 * a.rfX;
-                        const float2 po = phase_frac_i(outer, fourN);
-                        const int e0 = (c2 * k0) % a.fY;
-                        const int e1 = (c2 * k1) % a.fX;
-                        float fr = (float)e0 / (float)a.fY + (float)e1 / (float)a.fX;
-                        fr -= rintf(fr);
-                        float sn, cs;
-                        sincospif(2.0f * fr, &sn, &cs);
-                        const float2 z = c_col == 0 ? make_float2(mine[r], other[r]) : make_float2(other[r], mine[r]);
-                        const float2 v = cmul(cmul(z, po), make_float2(cs, sn));
-                        tot[q][j][r] += c_col == 0 ? v.x : v.y;
-                    }
-                }
-            }
-        }
-        if (a.per_plane) {                        // back projection: one output per plane
-            store(p);
-#pragma unroll
-            for (int q = 0; q < MAXT; ++q)
-#pragma unroll
-                for (int j = 0; j < SLOTS; ++j) tot[q][j] = v4f{0.f, 0.f, 0.f, 0.f};
-        }
-    }
-    if (!a.per_plane) store(blockIdx.y);
+    mac_body<SLOTS, NS, PER_PLANE>(ga.a[p.g], r % p.nch, r / p.nch, p.nr, fblock);
 }
 
 // ---------------------------------------------------------------------------
 // Inverse transform, stage 1: column inverse FFTs (length fY) of the half
 // plane, keeping output rows y < Yout.  The input is the sum of nsum partial
-// accumulators A_sstride apart (the forward projection's plane ranges).
-// grid (ceil(rfX/CB), nbatch), one wave per column (blockDim = 64*CB); LDS
-// CB*fY + fY (twiddles).
+// accumulators A_sstride apart (the forward projection's plane ranges), in
+// the MAC's order: bin (k0, k1) of frame f at A[colidx * nf + f], where the
+// bins of one orbit that fall on one column are consecutive.  A column is
+// read in the order k0 = y0 + m rY, m fastest (colidx is laid out in it), so
+// that neighbouring lanes read neighbouring bins.  The output holds rows
+// [y][k1][frame of the block].
+// A workgroup takes CB columns: CB / nf columns k1 of nf frames, or CB of the
+// nf frames of one column.  grid (column blocks, planes x frame blocks), one
+// wave per column (blockDim = 64*CB); LDS CB*fY + fY (twiddles).
 // ---------------------------------------------------------------------------
+struct ColBlocks {
+    int fc, kc, nfg;                 // frames and columns per workgroup, frame groups
+    __host__ __device__ ColBlocks(int nf, int CB)
+        : fc(nf < CB ? nf : CB), kc(nf < CB ? CB / nf : 1), nfg((nf + fc - 1) / fc) {}
+    __host__ __device__ int count(int rfX) const { return (rfX + kc - 1) / kc * nfg; }
+};
 template <bool PRIME, bool BIG>
 __device__ __forceinline__ void ifft_cols_body(const IfftColArgs& a, int colblk, int batch) {
     extern __shared__ float2 lds[];
-    const int fY = a.rpY.L, rfX = a.rfX, CB = a.CB;
+    const int fY = a.rpY.L, CB = a.CB;
+    const int nfb = (a.T + a.FB - 1) / a.FB;
+    const int plane = batch / nfb, t0 = (batch - plane * nfb) * a.FB;
+    const int nf = min(a.FB, a.T - t0);
+    const ColBlocks cb(nf, CB);
+    const int f0 = colblk % cb.nfg * cb.fc, k10 = colblk / cb.nfg * cb.kc;
+    if (k10 >= a.rfX) return;                           // (a block of fewer frames has fewer column blocks)
+    const int fn = min(cb.fc, nf - f0);
+    const int ncol = fn * min(cb.kc, a.rfX - k10);
     const int cs = ifft_col_stride(fY, CB);
-    float2* C = lds;                 // [CB][cs]
+    float2* C = lds;                 // [CB][cs], column kk * fn + frame
     float2* C2 = C + CB * cs;        // BIG: [CB][cs], the second buffer of the out-of-place passes
     float2* tw = BIG ? C2 + CB * cs : C2;   // [fY]
-    const int c0 = colblk * CB;
-    const int ncol = min(CB, rfX - c0);
-    const float2* in = a.A + (long long)batch * a.A_bstride;
+    const float2* in = a.A + ((long long)plane * a.T + t0) * a.A_bstride + f0;
+    const int* idx = a.colidx + (long long)k10 * fY;
     for (int i = threadIdx.x; i < fY; i += blockDim.x) tw[i] = a.twY[i];
     constexpr int B = 8;                        // loads in flight per thread
-    for (int i0 = threadIdx.x; i0 < fY * CB; i0 += blockDim.x * B) {
+    const int total = fY * ncol;
+    const float rfn = 1.0f / (float)fn, rN = 1.0f / (float)a.N, rfY = 1.0f / (float)fY;
+    for (int i0 = threadIdx.x; i0 < total; i0 += blockDim.x * B) {
         float2 v[B];
+        int src[B], dst[B];
 #pragma unroll
         for (int u = 0; u < B; ++u) {
-            const int i = i0 + u * blockDim.x;
-            const int y = i / CB, cc = i - y * CB;
-            v[u] = make_float2(0.f, 0.f);
-            if (i < fY * CB && cc < ncol) v[u] = in[(long long)y * rfX + c0 + cc];
+            // element -> frame (fastest), entry of the column, column
+            const int i = min(i0 + u * (int)blockDim.x, total - 1);
+            int fl, m, e;
+            const int q = div_small(i, fn, rfn, fl);
+            const int kk = div_small(q, fY, rfY, e);
+            const int y0 = div_small(e, a.N, rN, m);
+            src[u] = idx[q] * nf + fl;
+            dst[u] = (kk * fn + fl) * cs + y0 + m * a.rY;
         }
+#pragma unroll
+        for (int u = 0; u < B; ++u) v[u] = in[src[u]];
         for (int q = 1; q < a.nsum; ++q) {     // partial accumulators, fixed order
 #pragma unroll
-            for (int u = 0; u < B; ++u) {
-                const int i = i0 + u * blockDim.x;
-                const int y = i / CB, cc = i - y * CB;
-                if (i < fY * CB && cc < ncol) v[u] = cadd(v[u], in[(long long)y * rfX + c0 + cc + q * a.A_sstride]);
-            }
+            for (int u = 0; u < B; ++u) v[u] = cadd(v[u], in[src[u] + q * a.A_sstride]);
         }
 #pragma unroll
-        for (int u = 0; u < B; ++u) {
-            const int i = i0 + u * blockDim.x;
-            const int y = i / CB, cc = i - y * CB;
-            if (i < fY * CB) C[cc * cs + y] = v[u];
-        }
+        for (int u = 0; u < B; ++u)
+            if (i0 + u * (int)blockDim.x < total) C[dst[u]] = v[u];
     }
     __syncthreads();
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -1198,10 +1059,15 @@ __device__ __forceinline__ void ifft_cols_body(const IfftColArgs& a, int colblk,
     }
     __syncthreads();
     const float2* Res = (BIG && (a.rpY.n & 1)) ? C2 : C;   // after an odd pass count: the second buffer
-    float2* out = a.out + (long long)batch * a.out_bstride;
+    float2* out = a.out + ((long long)plane * a.T + t0) * a.out_bstride + (long long)k10 * nf + f0;
+    const int rowst = a.rfX * nf;
     for (int i = threadIdx.x; i < a.Yout * CB; i += blockDim.x) {
         const int y = i / CB, cc = i - y * CB;
-        if (cc < ncol) out[(long long)y * rfX + c0 + cc] = Res[cc * cs + y];
+        if (cc < ncol) {
+            int fl;
+            const int kk = div_small(cc, fn, rfn, fl);
+            out[(long long)y * rowst + kk * nf + fl] = Res[cc * cs + y];
+        }
     }
 }
 template <bool PRIME, bool BIG>
@@ -1216,7 +1082,7 @@ __global__ __launch_bounds__(512) void k_ifft_cols_grouped(IfftColGrouped ga) {
     ifft_cols_body<PRIME, false>(ga.a[p.g], p.rem % p.nch, p.rem / p.nch);
 }
 
-// c2r of one row by one wave.  row: rfX = L/2+1 half-spectrum values (global);
+// c2r of one row by one wave.  row: rfX = L/2+1 half-spectrum values rs apart (global);
 // buf: LDS work area (L/2 entries for even L, L for odd L; BIG, for L above
 // 2048: buf2 is a second such area for the out-of-place passes).  For even L the
 // length-L/2 complex transform of Z[k] = E[k] + i O[k],
@@ -1228,7 +1094,7 @@ __global__ __launch_bounds__(512) void k_ifft_cols_grouped(IfftColGrouped ga) {
 template <bool PRIME, bool BIG>
 __device__ __forceinline__ float2* wave_c2r(float2* buf, float2* buf2, const float2* __restrict__ row, int L,
                                             const RadixPlan& rph, const float2* twh,
-                                            const RadixPlan& rpf, const float2* twf, int lane) {
+                                            const RadixPlan& rpf, const float2* twf, int lane, int rs) {
     // Loads are issued C2R_BATCH per lane at a time, so that their latencies
     // overlap instead of adding up.
     constexpr int B = 8;
@@ -1240,8 +1106,8 @@ __device__ __forceinline__ float2* wave_c2r(float2* buf, float2* buf2, const flo
             for (int u = 0; u < B; ++u) {
                 const int k = k0 + 64 * u;
                 if (k < L2) {
-                    xs[u] = row[k];
-                    xrs[u] = row[L2 - k];
+                    xs[u] = row[k * rs];
+                    xrs[u] = row[(L2 - k) * rs];
                 }
             }
 #pragma unroll
@@ -1270,7 +1136,7 @@ __device__ __forceinline__ float2* wave_c2r(float2* buf, float2* buf2, const flo
 #pragma unroll
             for (int u = 0; u < B; ++u) {
                 const int k = k0 + 64 * u;
-                if (k < L) vs[u] = k < rfX ? row[k] : cconj(row[L - k]);
+                if (k < L) vs[u] = k < rfX ? row[k * rs] : cconj(row[(L - k) * rs]);
             }
 #pragma unroll
             for (int u = 0; u < B; ++u) {
@@ -1297,15 +1163,29 @@ __device__ __forceinline__ float c2r_sample(const float2* buf, int L, int x) {
     return buf[x].x;
 }
 
+// Rows per workgroup of the row transforms (one wave each).
+constexpr int ROWS_PER_WG = 4;
+// Wave w of frame block tb (8 frames) -> output row and frame, frames fastest.
+struct RowFrame {
+    int y, t;
+};
+__device__ __forceinline__ RowFrame row_frame(int w, int tb, int T) {
+    const int n = min(8, T - 8 * tb), y = w / n;
+    return {y, 8 * tb + w - y * n};
+}
+
 // Forward projection, stage 2: per output row, c2r each grid group's row and
-// sum the groups in a fixed order.  One wave per (row, frame);
-// grid (ceil(Y/4), T), block 256.
+// sum the groups in a fixed order.  One wave per (row, frame), the frames of
+// a block of 8 fastest (they are interleaved in memory);
+// grid (ceil(Y * min(8, T) / RPB), ceil(T / 8)), block 64 * RPB.
 template <bool PRIME, bool BIG>
-__global__ __launch_bounds__(256) void k_ifft_rows_sum(IfftRowSumArgs a) {
+__global__ __launch_bounds__(64 * (BIG ? 2 : ROWS_PER_WG)) void k_ifft_rows_sum(IfftRowSumArgs a) {
     extern __shared__ float2 lds[];
-    constexpr int RPB = BIG ? 2 : 4;            // rows (waves) per workgroup
+    reset_smax(a.smax, a.nsmax);
+    constexpr int RPB = BIG ? 2 : ROWS_PER_WG;  // rows (waves) per workgroup
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int y = blockIdx.x * RPB + wv, t = blockIdx.y;
+    const RowFrame rf = row_frame(blockIdx.x * RPB + wv, blockIdx.y, a.T);
+    const int y = rf.y, t = rf.t;
     float2* twf = lds;                          // [maxfX]
     float2* twh = twf + a.maxfX;                // [maxfX/2]
     float2* buf = twh + a.maxfX / 2 + 1 + wv * (BIG ? 2 : 1) * a.maxfX;
@@ -1324,8 +1204,9 @@ __global__ __launch_bounds__(256) void k_ifft_rows_sum(IfftRowSumArgs a) {
             for (int i = threadIdx.x; i < L / 2; i += blockDim.x) twh[i] = G.twh[i];
         __syncthreads();
         if (y < a.Y) {
-            const float2* row = G.T + (long long)t * G.tstride + (long long)y * G.rfX;
-            const float2* res = wave_c2r<PRIME, BIG>(buf, buf2, row, L, G.rph, twh, G.rp, twf, lane);
+            const int b0 = t / G.FB * G.FB, nf = min(G.FB, a.T - b0);
+            const float2* row = G.T + (long long)b0 * G.tstride + (long long)y * G.rfX * nf + (t - b0);
+            const float2* res = wave_c2r<PRIME, BIG>(buf, buf2, row, L, G.rph, twh, G.rp, twf, lane, nf);
             const float sc = G.scale;
 #pragma unroll
             for (int q = 0; q < XPL; ++q) {
@@ -1360,21 +1241,26 @@ __global__ __launch_bounds__(256) void k_ifft_rows_sum(IfftRowSumArgs a) {
 // Backward projection, stage 2: per (row, frame, plane) c2r; then either store
 // the plane, or apply the Richardson-Lucy update in place
 // (lfdeconv.py:112-126 Prevedel: X *= Htf / v;  lfdeconv.py:151-164 standard:
-// X *= v [/ trust]; NaN -> 0 after the update).  One wave per row;
-// grid (ceil(Y/4), T, nplanes), block 256.  Twiddles of every grid group are
+// X *= v [/ trust]; NaN -> 0 after the update).  One wave per (row, frame),
+// the frames of a block of 8 fastest (they are interleaved in memory);
+// grid (ceil(Y * min(8, T) / ROWS_PER_WG), ceil(T / 8), nplanes), block 64 * ROWS_PER_WG.  Twiddles of every grid group are
 // read from global memory (they stay in the caches).
 template <bool PRIME, bool BIG>
-__global__ __launch_bounds__(256) void k_ifft_rows_plane(IfftRowPlaneArgs a) {
+__global__ __launch_bounds__(64 * ROWS_PER_WG) void k_ifft_rows_plane(IfftRowPlaneArgs a) {
     extern __shared__ float2 lds[];
+    reset_smax(a.smax, a.nsmax);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int y = blockIdx.x * 4 + wv, t = blockIdx.y;
+    const RowFrame rf = row_frame(blockIdx.x * ROWS_PER_WG + wv, blockIdx.y, a.T);
+    const int y = rf.y, t = rf.t;
     const int z = a.plane_ids[blockIdx.z];      // kernel argument (scalar load)
     const RowPlaneDesc& pd = a.pd[z];           // read in place (no private copy)
     const int L = pd.rp.L;
     float2* buf = lds + wv * (BIG ? 2 : 1) * a.wbuf;
     if (y >= a.Y) return;                       // no block-level barrier below
-    const float2* row = a.Tbuf + pd.T_off + (long long)t * pd.T_tstride + (long long)y * pd.rfX;
-    const float2* res = wave_c2r<PRIME, BIG>(buf, buf + a.wbuf, row, L, pd.rph, pd.twh, pd.rp, pd.twf, lane);
+    const int FB = pd.slots == 4 ? a.FB4 : a.FB2;
+    const int b0 = t / FB * FB, nf = min(FB, a.T - b0);
+    const float2* row = a.Tbuf + pd.T_off + (long long)b0 * pd.T_tstride + (long long)y * pd.rfX * nf + (t - b0);
+    const float2* res = wave_c2r<PRIME, BIG>(buf, buf + a.wbuf, row, L, pd.rph, pd.twh, pd.rp, pd.twf, lane, nf);
     buf = const_cast<float2*>(res);
     const float sc = pd.scale;
     const long long o = (((long long)z * a.T + t) * a.Y + y) * a.X;
@@ -1524,7 +1410,7 @@ bool plan_has_prime(const RadixPlan& rp) {
 static bool has_prime(const RadixPlan& rp) { return plan_has_prime(rp); }
 
 size_t small_fft_lds(int rY, int rX) {
-    return ((size_t)(rY + 1) * (rX / 2 + 1) + 2 * (size_t)(rY + rX)) * sizeof(float2);
+    return ((size_t)(rY + 1) * (rX / 2 + 1) + 2 * (size_t)(rY + rX) + 1) * sizeof(float2);
 }
 // Reduced grids above 128 points take the 256-point wave transforms.
 bool small_fft_big(int rY, int rX) { return rY > 128 || rX > 128; }
@@ -1555,89 +1441,73 @@ hipError_t launch_psf_cols(const PsfColArgs& a, int nu, hipStream_t s) {
     else hipLaunchKernelGGL(k_psf_cols<false>, dim3((a.rfX + a.CB - 1) / a.CB, nu), dim3(FFT_THREADS), lds, s, a);
     return hipGetLastError();
 }
+size_t spec_pack_lds(int nu, int slots) {
+    return (size_t)nu * PACK_ITEMS * slots * sizeof(float2) + 8 * PACK_ITEMS * sizeof(float);
+}
 hipError_t launch_spec_pack(const SpecPackArgs& a, int nchunks, hipStream_t s) {
-    hipLaunchKernelGGL(k_spec_pack, dim3(nchunks, a.nu), dim3(FLF_CHUNK_MAX), 0, s, a);
+    const size_t lds = spec_pack_lds(a.nu, a.slots);
+    hipLaunchKernelGGL(k_spec_pack, dim3((FLF_CHUNK_MAX + PACK_ITEMS - 1) / PACK_ITEMS, nchunks), dim3(256), lds, s, a);
     return hipGetLastError();
 }
-size_t mac_tc_lds(int slots, int N) {
-    const int nres = slots == 4 ? 8 : 4;
-    return (size_t)TC_UB * nres * (slots / 2) * 64 * sizeof(float) + 2 * (size_t)nres * sizeof(float2) +
-           (size_t)TC_FB * N * N * (nres / 2) * sizeof(float2);
-}
-int mac_row_stride(int slots, int nu) {
-    const int n = nu * (slots == 4 ? 4 : 2);
-    return n + ((1 - n % 16) + 16) % 16;
-}
-size_t mac_lds(int slots, int nu, int N, int fb) {
-    const int nres = slots == 4 ? 8 : 4;
-    return (size_t)fb * nres * mac_row_stride(slots, nu) * sizeof(float4) +
-           ((size_t)fb * N * N * (nres / 2) + 2 * nres) * sizeof(float2);
-}
-template <int SLOTS, int IPT>
-static void launch_mac_fb(const MacArgs& a, int fb, dim3 grid, dim3 block, size_t lds, hipStream_t s) {
-    if (fb == 1) hipLaunchKernelGGL((k_mac<SLOTS, IPT, 1>), grid, block, lds, s, a);
-    else if (fb == 2) hipLaunchKernelGGL((k_mac<SLOTS, IPT, 2>), grid, block, lds, s, a);
-    else if (fb == 3) hipLaunchKernelGGL((k_mac<SLOTS, IPT, 3>), grid, block, lds, s, a);
-    else hipLaunchKernelGGL((k_mac<SLOTS, IPT, 4>), grid, block, lds, s, a);
-}
-hipError_t launch_mac(const MacArgs& a, int slots, int ipt, int fb, int nchunks, int nplanes_grid, bool mfma,
-                      hipStream_t s) {
-    if (fb < 1 || fb > 4 || (ipt != 1 && ipt != 2 && ipt != 4) || a.T < 1 || a.rs != mac_row_stride(slots, a.nu))
-        return hipErrorInvalidValue;
-    const size_t lds = mac_lds(slots, a.nu, a.N, fb);
-    dim3 grid(nchunks * ((a.T + fb - 1) / fb), nplanes_grid);
-    if (mfma && a.tiles) {
-        // matrix-core kernel: TC_FB frames per workgroup
-        dim3 tgrid(nchunks * ((a.T + TC_FB - 1) / TC_FB), nplanes_grid);
-        const size_t tlds = mac_tc_lds(slots, a.N);
-        if (slots == 4) hipLaunchKernelGGL((k_mac_tc<4>), tgrid, dim3(64 * TC_WAVES), tlds, s, a);
-        else hipLaunchKernelGGL((k_mac_tc<2>), tgrid, dim3(64 * TC_WAVES), tlds, s, a);
-        return hipGetLastError();
-    }
-    dim3 block(FLF_CHUNK_MAX);                   // ipt 2 / 4: lane groups share ipt items
+// Slots per matrix instruction for T frames: as many as leave no column that
+// these frames could fill empty (4 slots x 2 frames, 2 x 4, 1 x 8).
+int mac_slots_shared(int slots, int T) { return T > 4 ? 1 : (T > 2 || slots == 2 ? 2 : 4); }
+int mac_frames(int slots, int T) { return FLF_MAC_FB / mac_slots_shared(slots, T); }
+template <class F>
+static auto mac_variant(int slots, int ns, bool per_plane, F f) {
+    using std::integral_constant;
+    auto go = [&](auto s, auto n) {
+        return per_plane ? f(s, n, std::true_type{}) : f(s, n, std::false_type{});
+    };
     if (slots == 4) {
-        if (ipt == 1) launch_mac_fb<4, 1>(a, fb, grid, block, lds, s);
-        else if (ipt == 2) launch_mac_fb<4, 2>(a, fb, grid, block, lds, s);
-        else launch_mac_fb<4, 4>(a, fb, grid, block, lds, s);
-    } else {
-        if (ipt == 1) launch_mac_fb<2, 1>(a, fb, grid, block, lds, s);
-        else if (ipt == 2) launch_mac_fb<2, 2>(a, fb, grid, block, lds, s);
-        else launch_mac_fb<2, 4>(a, fb, grid, block, lds, s);
+        if (ns == 4) return go(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+        if (ns == 2) return go(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+        return go(integral_constant<int, 4>{}, integral_constant<int, 1>{});
     }
+    if (ns == 2) return go(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+    return go(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+}
+size_t mac_lds(int slots, int T) {
+    return mac_variant(slots, mac_slots_shared(slots, T), false, [](auto s, auto n, auto) { return MacShape<s.value, n.value>::LDS; });
+}
+static bool mac_args_ok(const MacArgs& a, int slots) {
+    return (slots == 2 || slots == 4) && a.T >= 1 && a.kg == (slots == 4 ? a.nu : (a.nu + 1) / 2);
+}
+hipError_t launch_mac(const MacArgs& a, int slots, int nchunks, int nplanes_grid, hipStream_t s) {
+    if (!mac_args_ok(a, slots)) return hipErrorInvalidValue;
+    const int fb = mac_frames(slots, a.T);
+    const dim3 grid(nchunks * ((a.T + fb - 1) / fb), nplanes_grid), block(MAC_THREADS);
+    mac_variant(slots, mac_slots_shared(slots, a.T), a.per_plane != 0, [&](auto sl, auto ns, auto pp) {
+        hipLaunchKernelGGL((k_mac<sl.value, ns.value, pp.value>), grid, block, (MacShape<sl.value, ns.value>::LDS), s, a);
+    });
     return hipGetLastError();
 }
-template <int SLOTS, int IPT>
-static void launch_mac_grouped_fb(const MacGrouped& ga, int fb, dim3 grid, dim3 block, size_t lds, hipStream_t s) {
-    if (fb == 1) hipLaunchKernelGGL((k_mac_grouped<SLOTS, IPT, 1>), grid, block, lds, s, ga);
-    else if (fb == 2) hipLaunchKernelGGL((k_mac_grouped<SLOTS, IPT, 2>), grid, block, lds, s, ga);
-    else if (fb == 3) hipLaunchKernelGGL((k_mac_grouped<SLOTS, IPT, 3>), grid, block, lds, s, ga);
-    else hipLaunchKernelGGL((k_mac_grouped<SLOTS, IPT, 4>), grid, block, lds, s, ga);
-}
-hipError_t launch_mac_grouped(const MacGrouped& ga, int slots, int ipt, int fb, int nfb, size_t lds, hipStream_t s) {
+hipError_t launch_mac_grouped(const MacGrouped& ga, int slots, hipStream_t s) {
     const GroupedGrid& gg = ga.gg;
-    if (fb < 1 || fb > 4 || (ipt != 1 && ipt != 2 && ipt != 4) || (slots != 2 && slots != 4) || nfb < 1 || gg.ngroups < 1 ||
-        gg.ngroups > FLF_MAX_GROUPS)
-        return hipErrorInvalidValue;
-    if (ga.nfb != nfb) return hipErrorInvalidValue;
-    for (int k = 0; k < gg.ngroups; ++k)
-        if (gg.start[k + 1] - gg.start[k] < gg.nchunks[k] * gg.nranges[k] * nfb) return hipErrorInvalidValue;
-    dim3 grid(gg.start[gg.ngroups]);
-    dim3 block(FLF_CHUNK_MAX);
-    if (slots == 4) {
-        if (ipt == 1) launch_mac_grouped_fb<4, 1>(ga, fb, grid, block, lds, s);
-        else if (ipt == 2) launch_mac_grouped_fb<4, 2>(ga, fb, grid, block, lds, s);
-        else launch_mac_grouped_fb<4, 4>(ga, fb, grid, block, lds, s);
-    } else {
-        if (ipt == 1) launch_mac_grouped_fb<2, 1>(ga, fb, grid, block, lds, s);
-        else if (ipt == 2) launch_mac_grouped_fb<2, 2>(ga, fb, grid, block, lds, s);
-        else launch_mac_grouped_fb<2, 4>(ga, fb, grid, block, lds, s);
+    if (gg.ngroups < 1 || gg.ngroups > FLF_MAX_GROUPS) return hipErrorInvalidValue;
+    const int T = ga.a[0].T, fb = mac_frames(slots, T);
+    if (ga.nfb != (T + fb - 1) / fb) return hipErrorInvalidValue;
+    for (int k = 0; k < gg.ngroups; ++k) {
+        if (gg.start[k + 1] - gg.start[k] < gg.nchunks[k] * gg.nranges[k] * ga.nfb) return hipErrorInvalidValue;
+        if (!mac_args_ok(ga.a[k], slots) || ga.a[k].per_plane != ga.a[0].per_plane || ga.a[k].T != T) return hipErrorInvalidValue;
     }
+    const dim3 grid(gg.start[gg.ngroups]), block(MAC_THREADS);
+    mac_variant(slots, mac_slots_shared(slots, T), ga.a[0].per_plane != 0, [&](auto sl, auto ns, auto pp) {
+        hipLaunchKernelGGL((k_mac_grouped<sl.value, ns.value, pp.value>), grid, block, (MacShape<sl.value, ns.value>::LDS), s, ga);
+    });
     return hipGetLastError();
 }
 // Transforms longer than 2048 points run out of place (two LDS buffers).
 bool wave_big(int L) { return L > 2048; }
 size_t ifft_cols_lds(int CB, int fY) {
     return ((size_t)CB * ifft_col_stride(fY, CB) * (wave_big(fY) ? 2 : 1) + fY) * sizeof(float2);
+}
+// Column blocks of a call: those of a full block of frames, or of the last one
+// where fewer frames make more of them.
+int ifft_col_blocks(const IfftColArgs& a) {
+    int n = 0;
+    for (int t0 = 0; t0 < a.T; t0 += a.FB) n = std::max(n, ColBlocks(std::min(a.FB, a.T - t0), a.CB).count(a.rfX));
+    return n;
 }
 hipError_t launch_ifft_cols_grouped(const IfftColGrouped& ga, int CB, bool prime, size_t lds, hipStream_t s) {
     const GroupedGrid& gg = ga.gg;
@@ -1648,7 +1518,7 @@ hipError_t launch_ifft_cols_grouped(const IfftColGrouped& ga, int CB, bool prime
 }
 hipError_t launch_ifft_cols(const IfftColArgs& a, int nbatch, hipStream_t s) {
     size_t lds = ifft_cols_lds(a.CB, a.rpY.L);
-    const dim3 grid((a.rfX + a.CB - 1) / a.CB, nbatch), block(64 * a.CB);
+    const dim3 grid(ifft_col_blocks(a), nbatch), block(64 * a.CB);
     const bool big = wave_big(a.rpY.L);
     if (has_prime(a.rpY)) {
         if (big) hipLaunchKernelGGL((k_ifft_cols<true, true>), grid, block, lds, s, a);
@@ -1663,18 +1533,20 @@ hipError_t launch_ifft_cols(const IfftColArgs& a, int nbatch, hipStream_t s) {
 // longer than 2048, which take two waves per workgroup instead of four).
 size_t ifft_rows_sum_lds(int maxfX) {
     const bool big = wave_big(maxfX);
-    return ((size_t)maxfX + maxfX / 2 + 1 + (big ? 2 * 2 : 4) * (size_t)maxfX) * sizeof(float2);
+    return ((size_t)maxfX + maxfX / 2 + 1 + (big ? 2 * 2 : ROWS_PER_WG) * (size_t)maxfX) * sizeof(float2);
 }
+static int row_blocks(int Y, int T, int rows) { return (Y * std::min(8, T) + rows - 1) / rows; }
 hipError_t launch_ifft_rows_sum(const IfftRowSumArgs& a, int Y, int T, hipStream_t s) {
+    if (a.T != T) return hipErrorInvalidValue;
     size_t lds = ifft_rows_sum_lds(a.maxfX);
     bool prime = false;
     for (int g = 0; g < a.ngroups; ++g) prime = prime || (a.grp[g].active && (has_prime(a.grp[g].rp) || has_prime(a.grp[g].rph)));
     if (wave_big(a.maxfX)) {
-        const dim3 grid((Y + 1) / 2, T), block(128);
+        const dim3 grid(row_blocks(Y, T, 2), (T + 7) / 8), block(128);
         if (prime) hipLaunchKernelGGL((k_ifft_rows_sum<true, true>), grid, block, lds, s, a);
         else hipLaunchKernelGGL((k_ifft_rows_sum<false, true>), grid, block, lds, s, a);
     } else {
-        const dim3 grid((Y + 3) / 4, T), block(256);
+        const dim3 grid(row_blocks(Y, T, ROWS_PER_WG), (T + 7) / 8), block(64 * ROWS_PER_WG);
         if (prime) hipLaunchKernelGGL((k_ifft_rows_sum<true, false>), grid, block, lds, s, a);
         else hipLaunchKernelGGL((k_ifft_rows_sum<false, false>), grid, block, lds, s, a);
     }
@@ -1682,10 +1554,10 @@ hipError_t launch_ifft_rows_sum(const IfftRowSumArgs& a, int Y, int T, hipStream
 }
 // c2r of an even length runs as a half-length complex FFT in place.
 int c2r_wave_buffer(int fX) { return (fX & 1) ? fX : fX / 2; }
-size_t ifft_rows_plane_lds(int wbuf, bool big) { return 4 * (size_t)wbuf * (big ? 2 : 1) * sizeof(float2); }
+size_t ifft_rows_plane_lds(int wbuf, bool big) { return ROWS_PER_WG * (size_t)wbuf * (big ? 2 : 1) * sizeof(float2); }
 hipError_t launch_ifft_rows_plane(const IfftRowPlaneArgs& a, int nplanes, hipStream_t s) {
     size_t lds = ifft_rows_plane_lds(a.wbuf, a.big != 0);
-    const dim3 grid((a.Y + 3) / 4, a.T, nplanes), block(256);
+    const dim3 grid(row_blocks(a.Y, a.T, ROWS_PER_WG), (a.T + 7) / 8, nplanes), block(64 * ROWS_PER_WG);
     if (a.prime) {
         if (a.big) hipLaunchKernelGGL((k_ifft_rows_plane<true, true>), grid, block, lds, s, a);
         else hipLaunchKernelGGL((k_ifft_rows_plane<true, false>), grid, block, lds, s, a);
@@ -1711,24 +1583,18 @@ hipError_t configure_kernels(size_t max_lds) {
                         (const void*)k_ifft_rows_sum<false, true>, (const void*)k_ifft_rows_sum<true, true>,
                         (const void*)k_ifft_rows_plane<false, false>, (const void*)k_ifft_rows_plane<true, false>,
                         (const void*)k_ifft_rows_plane<false, true>, (const void*)k_ifft_rows_plane<true, true>,
-                        (const void*)k_mac<4, 1, 1>, (const void*)k_mac<4, 1, 2>, (const void*)k_mac<4, 1, 3>,
-                        (const void*)k_mac<4, 1, 4>, (const void*)k_mac<4, 2, 1>, (const void*)k_mac<4, 2, 2>,
-                        (const void*)k_mac<4, 2, 3>, (const void*)k_mac<4, 2, 4>, (const void*)k_mac<2, 1, 1>,
-                        (const void*)k_mac<2, 1, 2>, (const void*)k_mac<2, 1, 3>, (const void*)k_mac<2, 1, 4>,
-                        (const void*)k_mac<2, 2, 1>, (const void*)k_mac<2, 2, 2>, (const void*)k_mac<2, 2, 3>,
-                        (const void*)k_mac<2, 2, 4>,
-                        (const void*)k_mac_tc<4>, (const void*)k_mac_tc<2>,
+                        (const void*)k_spec_pack,
                         (const void*)k_small_fft_grouped, (const void*)k_ifft_cols_grouped<false>,
-                        (const void*)k_ifft_cols_grouped<true>,
-                        (const void*)k_mac_grouped<4, 1, 1>, (const void*)k_mac_grouped<4, 1, 2>,
-                        (const void*)k_mac_grouped<4, 1, 3>, (const void*)k_mac_grouped<4, 1, 4>,
-                        (const void*)k_mac_grouped<4, 2, 1>, (const void*)k_mac_grouped<4, 2, 2>,
-                        (const void*)k_mac_grouped<4, 2, 3>, (const void*)k_mac_grouped<4, 2, 4>,
-                        (const void*)k_mac_grouped<2, 1, 1>, (const void*)k_mac_grouped<2, 1, 2>,
-                        (const void*)k_mac_grouped<2, 1, 3>, (const void*)k_mac_grouped<2, 1, 4>,
-                        (const void*)k_mac_grouped<2, 2, 1>, (const void*)k_mac_grouped<2, 2, 2>,
-                        (const void*)k_mac_grouped<2, 2, 3>, (const void*)k_mac_grouped<2, 2, 4>};
-    for (const void* k : ks) {
+                        (const void*)k_ifft_cols_grouped<true>};
+    std::vector<const void*> all(std::begin(ks), std::end(ks));
+    for (int slots : {2, 4})
+        for (int ns = 1; ns <= slots; ns *= 2)
+            for (bool pp : {false, true})
+                mac_variant(slots, ns, pp, [&](auto sl, auto n, auto p) {
+                    all.push_back((const void*)k_mac<sl.value, n.value, p.value>);
+                    all.push_back((const void*)k_mac_grouped<sl.value, n.value, p.value>);
+                });
+    for (const void* k : all) {
         hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_lds);
         if (e != hipSuccess) return e;
     }

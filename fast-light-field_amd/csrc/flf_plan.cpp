@@ -27,6 +27,7 @@
 #include "flf_plan.h"
 
 #include <algorithm>
+#include <array>
 #include <map>
 
 namespace flf {
@@ -97,12 +98,10 @@ static int alias2(int x, int r, int N) {
     return (2 * m + 1) % (2 * N);
 }
 
-std::string build_grid_tables(int N, int fY, int fX, GridTables& gt, int items_per_thread) {
+std::string build_grid_tables(int N, int fY, int fX, GridTables& gt) {
     if (N % 2 == 0 || N < 3 || N > FLF_MAX_N) return "Nnum must be odd and in [3, 31]";
     if (fY % N || fX % N) return "Fourier grid must be a multiple of Nnum";
-    if (items_per_thread < 1 || items_per_thread > 4) return "items per thread must be 1..4";
     gt = GridTables();
-    gt.ipt = items_per_thread;
     gt.fY = fY;
     gt.fX = fX;
     gt.rY = fY / N;
@@ -151,6 +150,15 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt, int items_p
         }
     }
     if (present != NN) return "internal: uses do not cover every offset once";
+    // Pair types: the two uses that read the same slot of an item, one plain
+    // and one conjugated (k_mac).
+    const int plain[4] = {0, 2, 4, 7}, conj[4] = {1, 3, 5, 6};
+    for (int u = 0; u < gt.nu; ++u)
+        for (int pt = 0; pt < gt.slots; ++pt)
+            for (int w = 0; w < 2; ++w) {
+                const int off = gt.uoff[u * gt.nuse + (w == 0 ? plain[pt] : conj[pt])];
+                gt.pairs.push_back(off < NN ? off * 8 + (off / N > c ? 1 : 0) + (off % N > c ? 2 : 0) : 4);
+            }
 
     const int rY = gt.rY, rX = gt.rX, rfX = gt.rfX;
     auto canon = [&](int k0, int k1) -> long long {
@@ -201,10 +209,10 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt, int items_p
                 res = {{k0, k1}, {n0, k1}, {n0, n1}, {k0, n1}};
             }
         }
-        std::vector<ItemDesc> its;
-        its.reserve(bases.size());
-        for (auto& bp : bases) {
-            int p0 = bp.first, p1 = bp.second;
+        // An item may take the base of its transposed bin (square: slots 2, 3,
+        // 0, 1) or of its negated row (non-square: slots 1, 0) just as well;
+        // its class is then the partner of its own.
+        auto make_item = [&](int p0, int p1, ItemDesc& it) -> const char* {
             int K0[4], K1[4];
             K0[0] = p0; K1[0] = p1;
             K0[1] = (fY - p0) % fY; K1[1] = p1;
@@ -212,7 +220,7 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt, int items_p
                 K0[2] = p1; K1[2] = p0;
                 K0[3] = (fY - p1) % fY; K1[3] = p0;
             }
-            ItemDesc it{};
+            it = ItemDesc{};
             it.writemask = 0;
             for (int j = 0; j < 4; ++j) {
                 if (j >= gt.slots) {
@@ -233,66 +241,82 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt, int items_p
                 it.m2[j] = (unsigned char)alias2(K0[j], rY, N);
                 it.n2[j] = (unsigned char)alias2(K1[j], rX, N);
             }
+            return nullptr;
+        };
+        std::vector<ItemDesc> its;
+        its.reserve(bases.size());
+        typedef std::array<unsigned char, 4> Class;
+        auto class_of = [](const ItemDesc& it) { return Class{it.res[0], it.res[1], it.res[2], it.res[3]}; };
+        std::map<Class, int> size;
+        for (auto& bp : bases) {
+            ItemDesc it;
+            if (const char* e = make_item(bp.first, bp.second, it)) return e;
             its.push_back(it);
+            ++size[class_of(it)];
+        }
+        // Tiles hold FLF_TILE items of one class: a class's items past its last
+        // full tile move to the partner class if they fit into the open tile
+        // there (at N = 15 one class of 36 and its partner of 28 become two of
+        // 32: 8 tiles per orbit instead of 9, one workgroup instead of two).
+        for (auto& kv : size) {
+            const int rest = kv.second % FLF_TILE;
+            if (kv.second <= FLF_TILE || rest == 0) continue;
+            int left = rest;
+            bool fits = false;
+            for (size_t q = its.size(); q-- > 0 && left > 0;) {
+                if (class_of(its[q]) != kv.first) continue;
+                ItemDesc alt;
+                const int p0 = bases[q].first, p1 = bases[q].second;
+                if (const char* e = make_item(gt.square ? p1 : (fY - p0) % fY, gt.square ? p0 : p1, alt)) return e;
+                const Class other = class_of(alt);
+                if (other == kv.first) break;
+                if (left == rest) {
+                    auto f = size.find(other);
+                    fits = f != size.end() && f->second % FLF_TILE != 0 && f->second % FLF_TILE + rest <= FLF_TILE;
+                }
+                if (!fits) break;
+                its[q] = alt;
+                ++size[other];
+                --kv.second;
+                --left;
+            }
         }
         gt.max_res = std::max(gt.max_res, (int)res.size());
-        gt.real_items += (long long)its.size();
-        // Order by residue tuple (residue class): the matrix-core MAC works on
-        // tiles of one class, and runs of ipt items share their residues.  For
-        // ipt > 1, pad every class to a multiple of ipt with non-writing copies.
-        const int ipt = gt.ipt;
+        // Order by residue tuple (residue class): the MAC works on tiles of one
+        // class, one per wave.
         std::stable_sort(its.begin(), its.end(), [](const ItemDesc& x, const ItemDesc& y) {
             for (int j = 0; j < 4; ++j)
                 if (x.res[j] != y.res[j]) return x.res[j] < y.res[j];
             return false;
         });
-        if (ipt > 1) {
-            std::vector<ItemDesc> padded;
-            size_t i0 = 0;
-            while (i0 < its.size()) {
-                size_t i1 = i0;
-                while (i1 < its.size() && std::equal(its[i1].res, its[i1].res + 4, its[i0].res)) ++i1;
-                for (size_t q = i0; q < i1; ++q) padded.push_back(its[q]);
-                size_t n = i1 - i0;
-                while (n % ipt) {
-                    ItemDesc d = its[i0];
-                    d.writemask = 0;
-                    padded.push_back(d);
-                    ++n;
-                }
-                i0 = i1;
-            }
-            its.swap(padded);
-        }
-        const size_t cmax = (size_t)(FLF_CHUNK_MAX / ipt) * ipt;
-        for (size_t s = 0; s < its.size(); s += cmax) {
+        // Tiles: runs of one residue class, at most FLF_TILE items each; at
+        // most FLF_CHUNK_TILES of them (and FLF_CHUNK_MAX items) per chunk.
+        size_t s = 0;
+        while (s < its.size()) {
             ChunkDesc ch{};
             ch.item_base = (long long)gt.items.size();
-            ch.n_items = (int)std::min<size_t>(cmax, its.size() - s);
             ch.n_res = (int)res.size();
             for (int q = 0; q < FLF_MAX_RES; ++q) {
                 ch.res0[q] = q < ch.n_res ? res[q].first : 0;
                 ch.res1[q] = q < ch.n_res ? res[q].second : 0;
             }
-            gt.items.insert(gt.items.end(), its.begin() + s, its.begin() + s + ch.n_items);
-            // Tiles: runs of one residue class, at most FLF_TILE items each.
             ch.tile_base = (int)gt.tiles.size();
-            int i0 = 0;
-            while (i0 < ch.n_items) {
-                const ItemDesc& first = its[s + i0];
-                int i1 = i0;
-                while (i1 < ch.n_items && i1 - i0 < FLF_TILE &&
-                       std::equal(its[s + i1].res, its[s + i1].res + 4, first.res))
-                    ++i1;
+            while (s < its.size() && ch.n_tiles < FLF_CHUNK_TILES) {
+                const ItemDesc& first = its[s];
+                size_t e = s;
+                while (e < its.size() && e - s < FLF_TILE && std::equal(its[e].res, its[e].res + 4, first.res)) ++e;
+                if (ch.n_items + (int)(e - s) > FLF_CHUNK_MAX) break;
                 TileDesc td{};
-                td.start = i0;
-                td.count = i1 - i0;
+                td.start = ch.n_items;
+                td.count = (int)(e - s);
                 for (int j = 0; j < 4; ++j) td.res[j] = first.res[j];
                 gt.tiles.push_back(td);
-                i0 = i1;
+                gt.items.insert(gt.items.end(), its.begin() + s, its.begin() + e);
+                ch.n_items += td.count;
+                ch.n_tiles += 1;
+                s = e;
             }
-            ch.n_tiles = (int)gt.tiles.size() - ch.tile_base;
-            if (ch.n_tiles > FLF_MAX_TILES) return "internal: too many residue-class tiles in a chunk";
+            gt.max_items = std::max(gt.max_items, ch.n_items);
             gt.chunks.push_back(ch);
         }
     }
@@ -306,6 +330,24 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt, int items_p
             }
     for (auto v : hit)
         if (!v) return "internal: bin not covered";
+    gt.wpos.assign(gt.items.size() * 4, 0xffff);
+    gt.colidx.assign((size_t)fY * rfX, 0);
+    std::vector<std::array<int, 3>> bins;                        // (k1, k0, item * 4 + slot) of one chunk
+    for (auto& ch : gt.chunks) {
+        bins.clear();
+        for (int i = 0; i < ch.n_items; ++i) {
+            const ItemDesc& it = gt.items[ch.item_base + i];
+            for (int j = 0; j < gt.slots; ++j)
+                if ((it.writemask >> j) & 1)
+                    bins.push_back({it.pos[j] % rfX, it.pos[j] / rfX, (int)(ch.item_base + i) * 4 + j});
+        }
+        std::sort(bins.begin(), bins.end());
+        for (size_t q = 0; q < bins.size(); ++q) {
+            const int k1 = bins[q][0], k0 = bins[q][1];
+            gt.wpos[bins[q][2]] = (unsigned short)q;
+            gt.colidx[(size_t)k1 * fY + (size_t)(k0 % rY) * N + k0 / rY] = (int)(ch.item_base * gt.slots + q);
+        }
+    }
     return "";
 }
 

@@ -30,21 +30,25 @@ struct GridTables {
     int slots = 0;               // 4 (square) or 2
     int nu = 0;                  // stored spectra per plane: h(h+1)/2 or h*h
     int max_res = 0;             // largest residue list of any chunk
-    int ipt = 1;                 // items per MAC thread
-    long long real_items = 0;    // items excluding padding copies
+    int max_items = 0;           // items of the largest chunk
     std::vector<int> u_bu, u_au; // stored spectrum u -> quadrant (b, a) (b > a: transposed)
     std::vector<int> uoff;       // [nu][uses]: offset b*N+a of each use of u, N*N if absent
     int nuse = 0;                // uses per stored spectrum: 8 (quads) or 4 (pairs)
+    // [nu][slots][2]: the plain and the conjugated use of each pair type, as
+    // offset * 8 + flags (1: row flipped, 2: column flipped), 4 if absent.
+    std::vector<int> pairs;
     std::vector<ChunkDesc> chunks;
     std::vector<ItemDesc> items;
     std::vector<TileDesc> tiles;
+    // Accumulator order: chunk by chunk (item_base * slots bins before it), a
+    // chunk's bins by (k1, k0).  wpos: [item][4], the place of each slot's bin
+    // within its chunk, 0xffff where the item does not write it.  colidx:
+    // [k1][y0][m], the place of bin (y0 + m rY, k1) in the whole order.
+    std::vector<unsigned short> wpos;
+    std::vector<int> colidx;
 };
 
 // Builds the tables; returns an empty string or an error message.
-// items_per_thread > 1 groups the items of each chunk so that every run of
-// items_per_thread consecutive items shares its residues (one MAC thread
-// handles such a run); classes whose size is not a multiple are padded with
-// copies that never write.
-std::string build_grid_tables(int N, int fY, int fX, GridTables& gt, int items_per_thread = 1);
+std::string build_grid_tables(int N, int fY, int fX, GridTables& gt);
 
 }  // namespace flf

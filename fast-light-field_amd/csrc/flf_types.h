@@ -8,8 +8,9 @@
 #define FLF_MAX_FOURIER 16384  // Fourier grid length per axis (keeps phase products in 32 bits)
 #define FLF_MAX_N 31           // largest supported Nnum (s-table = N*N entries)
 #define FLF_PRIME_RADIX_MAX 31 // largest odd prime radix of a transform (a prime factor of Nnum)
-#define FLF_TILE 16            // items per matrix-core tile (one residue class)
-#define FLF_MAX_TILES 24       // tiles per chunk: <= FLF_CHUNK_MAX / FLF_TILE + FLF_MAX_RES
+#define FLF_TILE 32            // items per tile of a MAC wave (one residue class)
+#define FLF_CHUNK_TILES 8      // tiles per chunk: one per wave of a MAC workgroup
+#define FLF_MAC_FB 8           // frames per MAC workgroup (16 matrix columns of Re, Im)
 
 struct RadixPlan {
     int L;                      // transform length
@@ -29,7 +30,7 @@ struct ChunkDesc {
 };
 
 // A run of at most FLF_TILE consecutive items of one chunk that share their
-// slot residues (one residue class): the unit of the matrix-core MAC.
+// slot residues (one residue class): one MAC wave's share of the chunk.
 struct TileDesc {
     int start;                  // first item, relative to the chunk
     int count;                  // items in the tile (<= FLF_TILE)

@@ -5,31 +5,25 @@ CalibrateBlockFactors, projector.py:628-675).
 
 Plan options come first, each candidate a fresh plan (spectra recomputed):
 the pass order of every FFT (``radix_order``: largest radices first,
-reversed, without radix 8, odd radices first) and the items per MAC thread
-(``mac_ipt``).  Then the launch shapes: the matrix-core MAC (``mac_mfma``,
-8 frames per workgroup; only when a call holds several frames), one dispatch per stage for all grid
-groups or one per group (``grouped_launch``), the forward MAC's plane ranges
-(``fwd_split``), the frames per MAC workgroup (``mac_frames``, only when a
-call holds several frames), the columns per column-transform workgroup
-(``ifft_col_batch``) and the planes per back-projection MAC workgroup
-(``bwd_planes``).  ``bwd_frame_group`` is not searched: at 32 x 1455^2 it
-saves about 5% of the back-projection MAC but multiplies that launch's HBM
-reads several times over, for a whole-step difference within run-to-run
-noise.  Each option is searched with the others fixed (coordinate
+reversed, without radix 8, odd radices first).  Then the launch shapes: one
+dispatch per stage for all grid groups or one per group
+(``grouped_launch``), the forward MAC's plane ranges (``fwd_split``), the
+columns per column-transform workgroup (``ifft_col_batch``) and the planes
+per back-projection MAC workgroup (``bwd_planes``).  ``mac_frames`` keeps its
+default (no kernel depends on it any more); ``bwd_frame_group`` only orders
+the dispatch and is not searched.  Each option is searched with the others fixed (coordinate
 descent, one pass); results depend on them only through FP32 rounding.
 """
 import torch
 
 PLAN_CANDIDATES = {
     "radix_order": [0, 1, 2, 3],
-    "mac_ipt": [2, 4, 1],
 }
 
 CANDIDATES = {
-    "mac_mfma": [0, 1],
     "grouped_launch": [1, 0],
     "fwd_split": [1, 2, 3, 4],
-    "mac_frames": [1, 2, 3, 4],
+    "mac_frames": [2],
     "ifft_col_batch": [2, 4, 8],
     "bwd_planes": [1, 2, 3, 4],
 }
@@ -91,7 +85,7 @@ def tune(projector, hMatrix, frames, Y, X, reps=3, log=None, plan_options=True):
         for name, values in PLAN_CANDIDATES.items():
             search(name, values, True)
     for name, values in CANDIDATES.items():
-        if name in ("mac_frames", "mac_mfma") and frames < 2:
+        if name == "mac_frames" and frames < 2:
             continue
         search(name, values, False)
     del vol, img

@@ -102,17 +102,18 @@ int flf_set_frame_dims(flf_ctx* ctx, const int* dims, int T, void* stream);
  * SetNumThreadsToUse / SetPlanningMode, py_light_field.cpp:216-241, are its
  * tuning knobs).  Names and values:
  *   "fwd_split"      0 (automatic) or 1..4 plane ranges of the forward MAC
- *   "mac_frames"     1..4 frames per MAC workgroup (upper bound)
- *   "mac_mfma"       0/1: matrix-core MAC (FP32 MFMA, 8 frames per
- *                    workgroup) for calls of >= 2 frames
- *   "bwd_planes"     1..8 planes per back-projection MAC workgroup
+ *   "mac_frames"     1..4 and "mac_mfma" 0/1: values of earlier
+ *                    multiply-accumulate kernels, accepted and kept; the
+ *                    matrix-core kernel takes up to 8 frames per workgroup
+ *   "bwd_planes"     1..8 planes per back-projection MAC workgroup (until it
+ *                    is set: 1 to 3 by the size of the projection)
  *   "bwd_frame_group" 0..64 frame blocks of a chunk the back-projection MAC
  *                    dispatches side by side (0: all; bit-identical results)
  *   "ifft_col_batch" 1..8 columns per column-transform workgroup (after plan)
  *   "grouped_launch" 0/1 (default 1): the small FFTs, the multiply-accumulate
  *                    and the column transforms of all Fourier-grid groups of
  *                    a projection go out as one dispatch each (bit-identical
- *                    results); not with group_streams or mac_mfma
+ *                    results); not with group_streams
  *   "group_streams"  0/1 (default 0): the Fourier-grid groups of a projection
  *                    run side by side on library-owned streams, forked from
  *                    and joined back to the caller's stream by events (one
@@ -122,7 +123,7 @@ int flf_set_frame_dims(flf_ctx* ctx, const int* dims, int T, void* stream);
  *   "radix_order"    0..3 pass order of every FFT: 0 largest radices first,
  *                    1 reversed, 2 no radix 8 (wave-level transforms), 3 odd
  *                    radices first (wave-level); a prime pass stays last
- *   "mac_ipt"        1, 2 or 4 items per MAC lane group (2 / 4: lane pairs / quads share them)
+ *   "mac_ipt"        1, 2 or 4: as mac_frames
  * Results do not depend on them beyond FP32 rounding (group_streams: not at
  * all).  flfhip.autotune picks them by timing. */
 int flf_set_option(flf_ctx* ctx, const char* name, int value);
