@@ -28,7 +28,6 @@
 
 #include <algorithm>
 #include <array>
-#include <map>
 
 namespace flf {
 
@@ -161,20 +160,23 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt) {
             }
 
     const int rY = gt.rY, rX = gt.rX, rfX = gt.rfX;
-    auto canon = [&](int k0, int k1) -> long long {
-        long long best = -1;
-        int a0[2] = {k0 % rY, (rY - k0 % rY) % rY};
-        int a1[2] = {k1 % rX, (rX - k1 % rX) % rX};
-        for (int i = 0; i < 2; ++i)
-            for (int j = 0; j < 2; ++j) {
-                long long v = (long long)a0[i] * rX + a1[j];
-                if (best < 0 || v < best) best = v;
-                if (gt.square) {
-                    long long w = (long long)a1[j] * rX + a0[i];
-                    if (w < best) best = w;
-                }
-            }
-        return best;
+    // Residue, its negative and the half-unit alias of every coordinate.
+    struct Axis { std::vector<int> res, neg; std::vector<unsigned char> al; };
+    auto axis = [N](int f, int r) {
+        Axis ax;
+        for (int k = 0; k < f; ++k) {
+            ax.res.push_back(k % r);
+            ax.neg.push_back((r - k % r) % r);
+            ax.al.push_back((unsigned char)alias2(k, r, N));
+        }
+        return ax;
+    };
+    const Axis aY = axis(fY, rY), aX = axis(fX, rX);
+    // Orbit of a base: the least index among its residue's images (mirroring an
+    // axis and, square grids, swapping the two).
+    auto canon = [&](int p0, int p1) {
+        const int a0 = std::min(aY.res[p0], aY.neg[p0]), a1 = std::min(aX.res[p1], aX.neg[p1]);
+        return gt.square ? std::min(a0, a1) * rX + std::max(a0, a1) : a0 * rX + a1;
     };
 
     // Collect item bases per orbit (ordered by orbit key for determinism).
@@ -183,11 +185,11 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt) {
         const int half = fY / 2;
         for (int p0 = 0; p0 <= half; ++p0)
             for (int p1 = 0; p1 <= p0; ++p1)
-                orbit_items[canon(p0 % rY, p1 % rX)].push_back({p0, p1});
+                orbit_items[canon(p0, p1)].push_back({p0, p1});
     } else {
         for (int p0 = 0; p0 <= fY / 2; ++p0)
             for (int p1 = 0; p1 <= fX / 2; ++p1)
-                orbit_items[canon(p0 % rY, p1 % rX)].push_back({p0, p1});
+                orbit_items[canon(p0, p1)].push_back({p0, p1});
     }
 
     gt.max_res = 0;
@@ -200,6 +202,7 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt) {
         // S at the first half only; the MAC gets the second half by
         // conjugation (S(-k) = conj S(k) for real input).
         std::vector<std::pair<int, int>> res;
+        std::array<int, 8> rkey;                                 // res as k0 * rX + k1
         {
             const int k0 = bases[0].first % rY, k1 = bases[0].second % rX;
             const int n0 = (rY - k0) % rY, n1 = (rX - k1) % rX;
@@ -208,6 +211,7 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt) {
             } else {
                 res = {{k0, k1}, {n0, k1}, {n0, n1}, {k0, n1}};
             }
+            for (size_t q = 0; q < res.size(); ++q) rkey[q] = res[q].first * rX + res[q].second;
         }
         // An item may take the base of its transposed bin (square: slots 2, 3,
         // 0, 1) or of its negated row (non-square: slots 1, 0) just as well;
@@ -232,28 +236,39 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt) {
                 bool dup = false;
                 for (int i = 0; i < j; ++i) dup |= (it.pos[i] == it.pos[j]);
                 if (!dup) it.writemask |= (1 << j);
-                std::pair<int, int> rr(K0[j] % rY, K1[j] % rX);
-                int ri = -1;
-                for (size_t q = 0; q < res.size() && ri < 0; ++q)
-                    if (res[q] == rr) ri = (int)q;
-                if (ri < 0) return "internal: slot residue outside its orbit";
+                const int rr = aY.res[K0[j]] * rX + aX.res[K1[j]], nr = (int)res.size();
+                int ri = 0;
+                while (ri < nr && rkey[ri] != rr) ++ri;
+                if (ri == nr) return "internal: slot residue outside its orbit";
                 it.res[j] = (unsigned char)ri;
-                it.m2[j] = (unsigned char)alias2(K0[j], rY, N);
-                it.n2[j] = (unsigned char)alias2(K1[j], rX, N);
+                it.m2[j] = aY.al[K0[j]];
+                it.n2[j] = aX.al[K1[j]];
             }
             return nullptr;
         };
         std::vector<ItemDesc> its;
         its.reserve(bases.size());
-        typedef std::array<unsigned char, 4> Class;
-        auto class_of = [](const ItemDesc& it) { return Class{it.res[0], it.res[1], it.res[2], it.res[3]}; };
-        std::map<Class, int> size;
+        // Classes (residue tuples, ascending) and their sizes: at most 8.
+        typedef std::pair<unsigned, int> Class;
+        auto class_of = [](const ItemDesc& it) {
+            return (unsigned)it.res[0] << 24 | (unsigned)it.res[1] << 16 | (unsigned)it.res[2] << 8 | it.res[3];
+        };
+        std::vector<Class> size;
+        auto find = [&size](unsigned c) {
+            return std::find_if(size.begin(), size.end(), [c](const Class& x) { return x.first == c; });
+        };
         for (auto& bp : bases) {
             ItemDesc it;
             if (const char* e = make_item(bp.first, bp.second, it)) return e;
             its.push_back(it);
-            ++size[class_of(it)];
+            const unsigned c = class_of(it);
+            auto f = find(c);
+            if (f == size.end())
+                size.push_back({c, 1});
+            else
+                ++f->second;
         }
+        std::sort(size.begin(), size.end());
         // Tiles hold FLF_TILE items of one class: a class's items past its last
         // full tile move to the partner class if they fit into the open tile
         // there (at N = 15 one class of 36 and its partner of 28 become two of
@@ -268,15 +283,15 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt) {
                 ItemDesc alt;
                 const int p0 = bases[q].first, p1 = bases[q].second;
                 if (const char* e = make_item(gt.square ? p1 : (fY - p0) % fY, gt.square ? p0 : p1, alt)) return e;
-                const Class other = class_of(alt);
+                const unsigned other = class_of(alt);
                 if (other == kv.first) break;
                 if (left == rest) {
-                    auto f = size.find(other);
+                    auto f = find(other);
                     fits = f != size.end() && f->second % FLF_TILE != 0 && f->second % FLF_TILE + rest <= FLF_TILE;
                 }
                 if (!fits) break;
                 its[q] = alt;
-                ++size[other];
+                ++find(other)->second;
                 --kv.second;
                 --left;
             }
@@ -284,11 +299,12 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt) {
         gt.max_res = std::max(gt.max_res, (int)res.size());
         // Order by residue tuple (residue class): the MAC works on tiles of one
         // class, one per wave.
-        std::stable_sort(its.begin(), its.end(), [](const ItemDesc& x, const ItemDesc& y) {
-            for (int j = 0; j < 4; ++j)
-                if (x.res[j] != y.res[j]) return x.res[j] < y.res[j];
-            return false;
-        });
+        std::vector<ItemDesc> sorted;
+        sorted.reserve(its.size());
+        for (const Class& c : size)
+            for (const ItemDesc& it : its)
+                if (class_of(it) == c.first) sorted.push_back(it);
+        its.swap(sorted);
         // Tiles: runs of one residue class, at most FLF_TILE items each; at
         // most FLF_CHUNK_TILES of them (and FLF_CHUNK_MAX items) per chunk.
         size_t s = 0;
@@ -320,34 +336,34 @@ std::string build_grid_tables(int N, int fY, int fX, GridTables& gt) {
             gt.chunks.push_back(ch);
         }
     }
-    // Coverage check: every half-plane bin written exactly once.
-    std::vector<unsigned char> hit((size_t)fY * rfX, 0);
-    for (auto& it : gt.items)
+    // The item slot that writes each half-plane bin, exactly one, then the bins'
+    // places within their chunks: counted over the bins in (k1, k0) order.
+    std::vector<int> owner((size_t)fY * rfX, -1), chunk_of(gt.items.size());
+    std::vector<int> row(fY);
+    for (size_t i = 0; i < gt.items.size(); ++i) {
+        const ItemDesc& it = gt.items[i];
         for (int j = 0; j < gt.slots; ++j)
             if ((it.writemask >> j) & 1) {
-                if (hit[it.pos[j]]) return "internal: bin written twice";
-                hit[it.pos[j]] = 1;
+                const int k0 = it.pos[j] / rfX, k1 = it.pos[j] - k0 * rfX;
+                int& o = owner[(size_t)k1 * fY + k0];
+                if (o >= 0) return "internal: bin written twice";
+                o = (int)i * 4 + j;
             }
-    for (auto v : hit)
-        if (!v) return "internal: bin not covered";
+    }
+    for (size_t c = 0; c < gt.chunks.size(); ++c)
+        std::fill_n(chunk_of.begin() + gt.chunks[c].item_base, gt.chunks[c].n_items, (int)c);
+    for (int k0 = 0; k0 < fY; ++k0) row[k0] = (k0 % rY) * N + k0 / rY;
     gt.wpos.assign(gt.items.size() * 4, 0xffff);
     gt.colidx.assign((size_t)fY * rfX, 0);
-    std::vector<std::array<int, 3>> bins;                        // (k1, k0, item * 4 + slot) of one chunk
-    for (auto& ch : gt.chunks) {
-        bins.clear();
-        for (int i = 0; i < ch.n_items; ++i) {
-            const ItemDesc& it = gt.items[ch.item_base + i];
-            for (int j = 0; j < gt.slots; ++j)
-                if ((it.writemask >> j) & 1)
-                    bins.push_back({it.pos[j] % rfX, it.pos[j] / rfX, (int)(ch.item_base + i) * 4 + j});
+    std::vector<int> used(gt.chunks.size(), 0);
+    for (int k1 = 0; k1 < rfX; ++k1)
+        for (int k0 = 0; k0 < fY; ++k0) {
+            const int o = owner[(size_t)k1 * fY + k0];
+            if (o < 0) return "internal: bin not covered";
+            const int c = chunk_of[o >> 2], q = used[c]++;
+            gt.wpos[o] = (unsigned short)q;
+            gt.colidx[(size_t)k1 * fY + row[k0]] = (int)(gt.chunks[c].item_base * gt.slots + q);
         }
-        std::sort(bins.begin(), bins.end());
-        for (size_t q = 0; q < bins.size(); ++q) {
-            const int k1 = bins[q][0], k0 = bins[q][1];
-            gt.wpos[bins[q][2]] = (unsigned short)q;
-            gt.colidx[(size_t)k1 * fY + (size_t)(k0 % rY) * N + k0 / rY] = (int)(ch.item_base * gt.slots + q);
-        }
-    }
     return "";
 }
 
