@@ -619,33 +619,33 @@ int run_backward(flf_ctx* ctx, const float* img, float* vol, const float* Htf, c
     const int rj = join_groups(ctx, fk);
     if (rc) return rc;
     if (rj) return rj;
-    // every plane's row transform (and RL update) in one launch on st
-    std::vector<int> ids;
-    int wbuf = 0, prime = 0, big = 0;
-    for (int z = 0; z < ctx->nz; ++z)
-        if (sel[z]) {
-            ids.push_back(z);
+    // The planes' row transforms (and RL update) on st: one launch for the rows
+    // of even length, one for those of odd length, whose full-length
+    // transforms take twice the registers.
+    for (int odd = 0; odd < 2; ++odd) {
+        IfftRowPlaneArgs r{};
+        int np = 0;
+        for (int z = 0; z < ctx->nz; ++z) {
             const Group& gz = ctx->groups[ctx->group_of[z]];
-            wbuf = std::max(wbuf, c2r_wave_buffer(gz.gt.fX));
-            if (wave_big(gz.gt.fX)) big = 1;
-            if (plan_has_prime(gz.rpXw) || plan_has_prime(gz.rpXhw)) prime = 1;
+            if (!sel[z] || (gz.gt.fX & 1) != odd) continue;
+            r.plane_ids[np++] = (unsigned short)z;
+            r.wbuf = std::max(r.wbuf, c2r_wave_buffer(gz.gt.fX));
+            if (wave_big(gz.gt.fX)) r.big = 1;
+            if (plan_has_prime(gz.rpXw) || plan_has_prime(gz.rpXhw)) r.prime = 1;
         }
-    if (ids.empty()) return FLF_OK;
-    IfftRowPlaneArgs r{};
-    r.smax = ctx->d_smax_bwd;
-    r.nsmax = (int)ctx->groups.size() * ctx->Tcap * FLF_SMAX_WAYS;
-    r.pd = ctx->d_rowdesc;
-    for (size_t i = 0; i < ids.size(); ++i) r.plane_ids[i] = (unsigned short)ids[i];
-    r.Tbuf = ctx->d_T_bwd;
-    r.vol = vol; r.Htf = Htf; r.trust = trust;
-    r.mode = mode; r.T = ctx->T; r.Y = ctx->Y; r.X = ctx->X;
-    r.FB4 = mac_frames(4, ctx->T);
-    r.FB2 = mac_frames(2, ctx->T);
-    r.wbuf = wbuf;
-    r.prime = prime;
-    r.big = big;
-    r.fdims = frame_dims(ctx);
-    HIPCHK(launch_ifft_rows_plane(r, (int)ids.size(), st));
+        if (np == 0) continue;
+        r.smax = ctx->d_smax_bwd;
+        r.nsmax = (int)ctx->groups.size() * ctx->Tcap * FLF_SMAX_WAYS;
+        r.pd = ctx->d_rowdesc;
+        r.Tbuf = ctx->d_T_bwd;
+        r.vol = vol; r.Htf = Htf; r.trust = trust;
+        r.mode = mode; r.T = ctx->T; r.Y = ctx->Y; r.X = ctx->X;
+        r.FB4 = mac_frames(4, ctx->T);
+        r.FB2 = mac_frames(2, ctx->T);
+        r.odd = odd;
+        r.fdims = frame_dims(ctx);
+        HIPCHK(launch_ifft_rows_plane(r, np, st));
+    }
     return FLF_OK;
 }
 
@@ -1125,6 +1125,7 @@ int run_forward(flf_ctx* ctx, const float* vol, const float* vol2, float* img, c
         rs.grp[gi].twf = g.twX;
         rs.grp[gi].twh = g.twXh;
         if (any) rs.maxfX = std::max(rs.maxfX, gt.fX);
+        if (any) rs.wbuf = std::max(rs.wbuf, c2r_wave_buffer(gt.fX));
     }
     GroupFork fk;
     rc = fork_groups(ctx, st, nactive, fk);

@@ -155,6 +155,7 @@ struct IfftRowSumArgs {
     int nsmax;
     int ngroups;
     int maxfX;
+    int wbuf;                    // c2r_wave_buffer, max over the active groups
     int X, Y, T;
     float* img;                  // forward image, or null (not stored)
     long long img_tstride;
@@ -190,6 +191,7 @@ struct IfftRowPlaneArgs {
     int wbuf;                    // per-wave LDS buffer (float2): max over planes of fX/2 (even) or fX
     const int2* fdims;           // per frame valid size; outside it the volume is set to 0
     int prime;                   // some plane's row plan ends with an odd prime radix above 5
+    int odd;                     // some plane's rows have an odd length
     int big;                     // some plane's rows are longer than 2048 (out-of-place transforms)
 };
 

@@ -1091,14 +1091,14 @@ __global__ __launch_bounds__(512) void k_ifft_cols_grouped(IfftColGrouped ga) {
 // extension and a full-length transform.  The imaginary parts of X[0] and
 // X[L/2] are dropped, as a c2r transform does.  Returns with the result in
 // buf (interleaved real samples for even L, real parts for odd L).
-template <bool PRIME, bool BIG>
+template <bool PRIME, bool BIG, bool ODD>
 __device__ __forceinline__ float2* wave_c2r(float2* buf, float2* buf2, const float2* __restrict__ row, int L,
                                             const RadixPlan& rph, const float2* twh,
                                             const RadixPlan& rpf, const float2* twf, int lane, int rs) {
     // Loads are issued C2R_BATCH per lane at a time, so that their latencies
     // overlap instead of adding up.
     constexpr int B = 8;
-    if ((L & 1) == 0) {
+    if (!ODD || (L & 1) == 0) {
         const int L2 = L / 2;
         for (int k0 = lane; k0 < L2; k0 += 64 * B) {
             float2 xs[B], xrs[B];
@@ -1155,6 +1155,35 @@ __device__ __forceinline__ float2* wave_c2r(float2* buf, float2* buf2, const flo
     }
 }
 
+// The same transform of a row that lies in buf already (rfX values, natural
+// order), in place: a lane takes both values of a pair (k, L/2 - k), whose
+// results E + i O and conj(E) + i conj(O) replace them.  twd: the length-L
+// table for the pre-twiddle (global memory, even L); tab: the table of the
+// transform itself (LDS).
+template <bool PRIME, bool ODD>
+__device__ __forceinline__ void wave_c2r_in_place(float2* buf, int L, const RadixPlan& rph, const RadixPlan& rpf,
+                                                  const float2* __restrict__ twd, const float2* tab, int lane) {
+    if (!ODD || (L & 1) == 0) {
+        const int L2 = L / 2;
+        for (int k = lane; 2 * k <= L2; k += 64) {
+            float2 x = buf[k], xr = cconj(buf[L2 - k]);
+            if (k == 0) { x.y = 0.f; xr.y = 0.f; }
+            const float2 E = cadd(x, xr), O = cmul(csub(x, xr), cconj(twd[k]));
+            buf[k] = make_float2(E.x - O.y, E.y + O.x);                        // E + i O
+            if (2 * k < L2 && k > 0) buf[L2 - k] = make_float2(E.x + O.y, O.x - E.y);   // conj(E) + i conj(O)
+        }
+        wave_sync();
+        wave_fft<1024, PRIME>(buf, 1, rph, tab, true, lane);
+    } else {
+        for (int k = lane; 2 * k < L; k += 64) {
+            if (k == 0) buf[0].y = 0.f;
+            else buf[L - k] = cconj(buf[k]);
+        }
+        wave_sync();
+        wave_fft<2048, PRIME>(buf, 1, rpf, tab, true, lane);
+    }
+}
+
 __device__ __forceinline__ float c2r_sample(const float2* buf, int L, int x) {
     if ((L & 1) == 0) {
         const float2 v = buf[x >> 1];
@@ -1163,7 +1192,8 @@ __device__ __forceinline__ float c2r_sample(const float2* buf, int L, int x) {
     return buf[x].x;
 }
 
-// Rows per workgroup of the row transforms (one wave each).
+// Rows per workgroup of the row transforms that read rows from memory directly
+// (one frame, or rows longer than 2048; one wave each).
 constexpr int ROWS_PER_WG = 4;
 // Wave w of frame block tb (8 frames) -> output row and frame, frames fastest.
 struct RowFrame {
@@ -1174,11 +1204,87 @@ __device__ __forceinline__ RowFrame row_frame(int w, int tb, int T) {
     return {y, 8 * tb + w - y * n};
 }
 
+// Several frames: rows staged through LDS.  The frames of a block lie
+// interleaved, so a wave that reads its own row takes 8 of every 8 n bytes
+// (n frames) and each of its loads touches 64 lines.  Here a workgroup of
+// ROW_WAVES waves takes ROW_WAVES / n rows of the n frames of a block, one
+// contiguous run of memory, and spreads it over the waves' LDS buffers.
+// Bound: memory and the passes' latency.  8 frames of 1455^2 x 41 planes, stored
+// (6 GB) / with the update (11.6 GB): 3.55 / 6.65 -> 2.29 / 3.08 ms (2.42 / 4.52
+// from rows apart, as one frame has them; that order costs the column
+// transform its runs).  Even lengths alone: 75 registers instead of 127 (odd
+// lengths take full-length transforms), 6 waves per SIMD instead of 4.
+constexpr int ROW_WAVES = 8;
+struct RowSet {
+    int t0, n, y0, rows;          // frames t0 .. t0 + n - 1, rows y0 .. y0 + rows - 1
+};
+__device__ __forceinline__ RowSet row_set(int blk, int tb, int T, int Y) {
+    RowSet r;
+    r.t0 = 8 * tb;
+    r.n = min(8, T - r.t0);
+    const int R = ROW_WAVES / r.n;
+    r.y0 = blk * R;
+    r.rows = min(R, Y - r.y0);    // <= 0: past the end (a block of fewer frames has fewer workgroups)
+    return r;
+}
+// Buffer stride (float2): the values of one k and the n frames fall on
+// distinct banks, with the 32 / n neighbours that a half wave writes along.
+__host__ __device__ inline int row_stage_stride(int wbuf, int n) {
+    const int want = 32 / n % 32, len = wbuf + 1;
+    return len + ((want - len) % 32 + 32) % 32;
+}
+// src: the run's first value; element q = ((row, k), frame) goes to the buffer
+// of wave row * n + frame, entry k.
+__device__ __forceinline__ void stage_rows(float2* buf, int bs, const float2* __restrict__ src, const RowSet& r, int rfX) {
+    constexpr int B = 8;                        // loads in flight per thread
+    const int total = r.rows * rfX * r.n;
+    const float rn = 1.0f / (float)r.n, rrf = 1.0f / (float)rfX;
+    for (int i0 = threadIdx.x; i0 < total; i0 += 64 * ROW_WAVES * B) {
+        float2 v[B];
+#pragma unroll
+        for (int u = 0; u < B; ++u) v[u] = src[min(i0 + u * 64 * ROW_WAVES, total - 1)];
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            const int i = i0 + u * 64 * ROW_WAVES;
+            int f, k;
+            const int row = div_small(div_small(i, r.n, rn, f), rfX, rrf, k);
+            if (i < total) buf[(row * r.n + f) * bs + k] = v[u];
+        }
+    }
+}
+__device__ __forceinline__ void stage_table(float2* tab, int L, const float2* __restrict__ twh, const float2* __restrict__ twf) {
+    const int n = (L & 1) ? L : L / 2;
+    const float2* t = (L & 1) ? twf : twh;
+    for (int i = threadIdx.x; i < n; i += 64 * ROW_WAVES) tab[i] = t[i];
+}
+
+template <int XPL>
+__device__ __forceinline__ void store_row_sum(const IfftRowSumArgs& a, const float* acc, int y, int t, int lane) {
+    const int Yv = a.fdims ? a.fdims[t].x : a.Y, Xv = a.fdims ? a.fdims[t].y : a.X;
+    const long long ro = (long long)t * a.img_tstride + (long long)y * a.X;
+    if (a.img) {
+#pragma unroll
+        for (int q = 0; q < XPL; ++q) {
+            const int x = lane + 64 * q;
+            if (x < a.X) a.img[ro + x] = (y < Yv && x < Xv) ? acc[q] : 0.f;
+        }
+    }
+    if (a.ratio) {
+        // standard RL's error image im / HX (lfdeconv.py:191) with IEEE
+        // division: 0/0 gives NaN and x/0 inf, as in numpy
+#pragma unroll
+        for (int q = 0; q < XPL; ++q) {
+            const int x = lane + 64 * q;
+            if (x < a.X) a.ratio[ro + x] = (y < Yv && x < Xv) ? a.im[ro + x] / acc[q] : 0.f;
+        }
+    }
+}
+
 // Forward projection, stage 2: per output row, c2r each grid group's row and
 // sum the groups in a fixed order.  One wave per (row, frame), the frames of
 // a block of 8 fastest (they are interleaved in memory);
 // grid (ceil(Y * min(8, T) / RPB), ceil(T / 8)), block 64 * RPB.
-template <bool PRIME, bool BIG>
+template <bool PRIME, bool BIG, bool ODD>
 __global__ __launch_bounds__(64 * (BIG ? 2 : ROWS_PER_WG)) void k_ifft_rows_sum(IfftRowSumArgs a) {
     extern __shared__ float2 lds[];
     reset_smax(a.smax, a.nsmax);
@@ -1206,7 +1312,7 @@ __global__ __launch_bounds__(64 * (BIG ? 2 : ROWS_PER_WG)) void k_ifft_rows_sum(
         if (y < a.Y) {
             const int b0 = t / G.FB * G.FB, nf = min(G.FB, a.T - b0);
             const float2* row = G.T + (long long)b0 * G.tstride + (long long)y * G.rfX * nf + (t - b0);
-            const float2* res = wave_c2r<PRIME, BIG>(buf, buf2, row, L, G.rph, twh, G.rp, twf, lane, nf);
+            const float2* res = wave_c2r<PRIME, BIG, ODD>(buf, buf2, row, L, G.rph, twh, G.rp, twf, lane, nf);
             const float sc = G.scale;
 #pragma unroll
             for (int q = 0; q < XPL; ++q) {
@@ -1216,25 +1322,98 @@ __global__ __launch_bounds__(64 * (BIG ? 2 : ROWS_PER_WG)) void k_ifft_rows_sum(
             wave_sync();
         }
     }
-    if (y < a.Y) {
-        const int Yv = a.fdims ? a.fdims[t].x : a.Y, Xv = a.fdims ? a.fdims[t].y : a.X;
-        const long long ro = (long long)t * a.img_tstride + (long long)y * a.X;
-        if (a.img) {
+    if (y < a.Y) store_row_sum<XPL>(a, acc, y, t, lane);
+}
+
+// The same for several frames, rows staged through LDS (see stage_rows);
+// grid (ceil(Y / (ROW_WAVES / n)), ceil(T / 8)), block 64 * ROW_WAVES.
+template <bool PRIME, bool ODD>
+__global__ __launch_bounds__(64 * ROW_WAVES) void k_ifft_rows_sum_staged(IfftRowSumArgs a) {
+    extern __shared__ float2 lds[];
+    reset_smax(a.smax, a.nsmax);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const RowSet r = row_set(blockIdx.x, blockIdx.y, a.T, a.Y);
+    if (r.rows <= 0) return;
+    const int bs = row_stage_stride(a.wbuf, r.n);
+    float2* tab = lds;                          // [wbuf]
+    float2* bufs = lds + a.wbuf;                // [ROW_WAVES][bs]
+    float2* buf = bufs + wv * bs;
+    const int row = wv / r.n, y = r.y0 + row, t = r.t0 + wv - row * r.n;
+    const bool busy = row < r.rows;
+    constexpr int XPL = 2048 / 64;
+    float acc[XPL];
+#pragma unroll
+    for (int q = 0; q < XPL; ++q) acc[q] = 0.f;
+    for (int g = 0; g < a.ngroups; ++g) {
+        const IfftRowGroup& G = a.grp[g];
+        if (!G.active) continue;
+        const int L = G.rp.L;
+        __syncthreads();
+        stage_table(tab, L, G.twh, G.twf);
+        stage_rows(bufs, bs, G.T + (long long)r.t0 * G.tstride + (long long)r.y0 * G.rfX * r.n, r, G.rfX);
+        __syncthreads();
+        if (busy) {
+            wave_c2r_in_place<PRIME, ODD>(buf, L, G.rph, G.rp, G.twf, tab, lane);
+            const float sc = G.scale;
 #pragma unroll
             for (int q = 0; q < XPL; ++q) {
                 const int x = lane + 64 * q;
-                if (x < a.X) a.img[ro + x] = (y < Yv && x < Xv) ? acc[q] : 0.f;
+                if (x < a.X) acc[q] += c2r_sample(buf, L, x) * sc;
             }
         }
-        if (a.ratio) {
-            // standard RL's error image im / HX (lfdeconv.py:191) with IEEE
-            // division: 0/0 gives NaN and x/0 inf, as in numpy
+    }
+    if (busy) store_row_sum<XPL>(a, acc, y, t, lane);
+}
+
+// One row's samples to the volume: stored, or the Richardson-Lucy update.  Two
+// samples per lane and step, as they lie in buf for even lengths (rows of an
+// odd X start on 4-byte boundaries; 8-byte accesses need no more).
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ float rl_update(int mode, float v, float xo, float hd, bool trust) {
+    if (mode == 0) return v;
+    float xn;
+    if (mode == 1) {
+        xn = xo * (hd / v);
+    } else {
+        xn = xo * v;
+        if (trust) xn = xn / hd;
+    }
+    return __builtin_isnan(xn) ? 0.f : xn;
+}
+__device__ __forceinline__ void update_row(const IfftRowPlaneArgs& a, const float2* buf, const RowPlaneDesc& pd, int z,
+                                           int t, int y, int lane) {
+    const int L = pd.rp.L, X2 = a.X / 2;
+    const float sc = pd.scale;
+    const long long o = (((long long)z * a.T + t) * a.Y + y) * a.X;
+    const int Yv = a.fdims ? a.fdims[t].x : a.Y, Xv = a.fdims ? a.fdims[t].y : a.X;
+    float* vol = a.vol + o;
+    const bool tr = a.mode == 2 && a.trust;
+    const float* hs = a.mode == 1 ? a.Htf + o : tr ? a.trust + ((long long)z * a.Y + y) * a.X : nullptr;
+    constexpr int B = 4;                        // pairs in flight per lane
+    for (int k0 = lane; k0 < X2; k0 += 64 * B) {
+        f2u xo[B], hd[B];
 #pragma unroll
-            for (int q = 0; q < XPL; ++q) {
-                const int x = lane + 64 * q;
-                if (x < a.X) a.ratio[ro + x] = (y < Yv && x < Xv) ? a.im[ro + x] / acc[q] : 0.f;
+        for (int u = 0; u < B; ++u) {
+            const int x = 2 * min(k0 + 64 * u, X2 - 1);
+            xo[u] = a.mode != 0 ? *(const f2u*)(vol + x) : f2u{0.f, 0.f};
+            hd[u] = hs ? *(const f2u*)(hs + x) : f2u{1.f, 1.f};
+        }
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            const int k = k0 + 64 * u, x = 2 * k;
+            if (k < X2) {
+                float2 v = (L & 1) ? make_float2(buf[x].x, buf[x + 1].x) : buf[k];
+                f2u r;
+                r.x = y < Yv && x < Xv ? rl_update(a.mode, v.x * sc, xo[u].x, hd[u].x, tr) : 0.f;
+                r.y = y < Yv && x + 1 < Xv ? rl_update(a.mode, v.y * sc, xo[u].y, hd[u].y, tr) : 0.f;
+                *(f2u*)(vol + x) = r;
             }
         }
+    }
+    if ((a.X & 1) && lane == 0) {
+        const int x = a.X - 1;
+        const float xo = a.mode != 0 ? vol[x] : 0.f, hd = hs ? hs[x] : 1.f;
+        vol[x] = y < Yv && x < Xv ? rl_update(a.mode, c2r_sample(buf, L, x) * sc, xo, hd, tr) : 0.f;
     }
 }
 
@@ -1245,7 +1424,7 @@ __global__ __launch_bounds__(64 * (BIG ? 2 : ROWS_PER_WG)) void k_ifft_rows_sum(
 // the frames of a block of 8 fastest (they are interleaved in memory);
 // grid (ceil(Y * min(8, T) / ROWS_PER_WG), ceil(T / 8), nplanes), block 64 * ROWS_PER_WG.  Twiddles of every grid group are
 // read from global memory (they stay in the caches).
-template <bool PRIME, bool BIG>
+template <bool PRIME, bool BIG, bool ODD>
 __global__ __launch_bounds__(64 * ROWS_PER_WG) void k_ifft_rows_plane(IfftRowPlaneArgs a) {
     extern __shared__ float2 lds[];
     reset_smax(a.smax, a.nsmax);
@@ -1260,44 +1439,32 @@ __global__ __launch_bounds__(64 * ROWS_PER_WG) void k_ifft_rows_plane(IfftRowPla
     const int FB = pd.slots == 4 ? a.FB4 : a.FB2;
     const int b0 = t / FB * FB, nf = min(FB, a.T - b0);
     const float2* row = a.Tbuf + pd.T_off + (long long)b0 * pd.T_tstride + (long long)y * pd.rfX * nf + (t - b0);
-    const float2* res = wave_c2r<PRIME, BIG>(buf, buf + a.wbuf, row, L, pd.rph, pd.twh, pd.rp, pd.twf, lane, nf);
-    buf = const_cast<float2*>(res);
-    const float sc = pd.scale;
-    const long long o = (((long long)z * a.T + t) * a.Y + y) * a.X;
-    const int Yv = a.fdims ? a.fdims[t].x : a.Y, Xv = a.fdims ? a.fdims[t].y : a.X;
-    constexpr int B = 8;                        // loads in flight per lane
-    for (int x0 = lane; x0 < a.X; x0 += 64 * B) {
-        float v[B], xo[B], hd[B];
-#pragma unroll
-        for (int u = 0; u < B; ++u) {
-            const int x = x0 + 64 * u;
-            if (x < a.X) {
-                v[u] = c2r_sample(buf, L, x) * sc;
-                if (a.mode != 0) xo[u] = a.vol[o + x];
-                if (a.mode == 1) hd[u] = a.Htf[o + x];
-                else if (a.mode == 2) hd[u] = a.trust ? a.trust[((long long)z * a.Y + y) * a.X + x] : 1.f;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < B; ++u) {
-            const int x = x0 + 64 * u;
-            if (x < a.X && (y >= Yv || x >= Xv)) {
-                a.vol[o + x] = 0.f;                 // outside this frame's valid region
-            } else if (x < a.X) {
-                if (a.mode == 0) {
-                    a.vol[o + x] = v[u];
-                } else if (a.mode == 1) {
-                    const float r = hd[u] / v[u];
-                    const float xn = xo[u] * r;
-                    a.vol[o + x] = __builtin_isnan(xn) ? 0.f : xn;
-                } else {
-                    float xn = xo[u] * v[u];
-                    if (a.trust) xn = xn / hd[u];
-                    a.vol[o + x] = __builtin_isnan(xn) ? 0.f : xn;
-                }
-            }
-        }
-    }
+    const float2* res = wave_c2r<PRIME, BIG, ODD>(buf, buf + a.wbuf, row, L, pd.rph, pd.twh, pd.rp, pd.twf, lane, nf);
+    update_row(a, res, pd, z, t, y, lane);
+}
+
+// The same for several frames, rows staged through LDS (see stage_rows);
+// grid (ceil(Y / (ROW_WAVES / n)), ceil(T / 8), nplanes), block 64 * ROW_WAVES.
+template <bool PRIME, bool ODD>
+__global__ __launch_bounds__(64 * ROW_WAVES) void k_ifft_rows_plane_staged(IfftRowPlaneArgs a) {
+    extern __shared__ float2 lds[];
+    reset_smax(a.smax, a.nsmax);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const RowSet r = row_set(blockIdx.x, blockIdx.y, a.T, a.Y);
+    if (r.rows <= 0) return;
+    const int z = a.plane_ids[blockIdx.z];
+    const RowPlaneDesc& pd = a.pd[z];
+    const int L = pd.rp.L, bs = row_stage_stride(a.wbuf, r.n);
+    float2* tab = lds;                          // [wbuf]
+    float2* bufs = lds + a.wbuf;                // [ROW_WAVES][bs]
+    stage_table(tab, L, pd.twh, pd.twf);
+    stage_rows(bufs, bs, a.Tbuf + pd.T_off + (long long)r.t0 * pd.T_tstride + (long long)r.y0 * pd.rfX * r.n, r, pd.rfX);
+    __syncthreads();
+    const int row = wv / r.n;
+    if (row >= r.rows) return;                  // no block-level barrier below
+    float2* buf = bufs + wv * bs;
+    wave_c2r_in_place<PRIME, ODD>(buf, L, pd.rph, pd.rp, pd.twf, tab, lane);
+    update_row(a, buf, pd, z, r.t0 + wv - row * r.n, r.y0 + row, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -1536,35 +1703,67 @@ size_t ifft_rows_sum_lds(int maxfX) {
     return ((size_t)maxfX + maxfX / 2 + 1 + (big ? 2 * 2 : ROWS_PER_WG) * (size_t)maxfX) * sizeof(float2);
 }
 static int row_blocks(int Y, int T, int rows) { return (Y * std::min(8, T) + rows - 1) / rows; }
+// Staged rows: the transform's table and one buffer per wave (149 KB at most,
+// rows of 2047).
+static size_t row_stage_lds(int wbuf, int T) {
+    int bs = 0;
+    for (int n : {std::min(8, T), T > 8 && T % 8 ? T % 8 : std::min(8, T)}) bs = std::max(bs, row_stage_stride(wbuf, n));
+    return ((size_t)wbuf + (size_t)ROW_WAVES * bs) * sizeof(float2);
+}
+// Workgroups over the rows: a block of n frames takes ROW_WAVES / n rows each.
+static int row_stage_blocks(int Y, int T) {
+    const int R = ROW_WAVES / std::min(8, T);
+    return (Y + R - 1) / R;
+}
+// Calls f with a flag as a compile-time constant.
+template <class F>
+static void with_bool(bool b, F f) {
+    if (b) f(std::true_type{});
+    else f(std::false_type{});
+}
 hipError_t launch_ifft_rows_sum(const IfftRowSumArgs& a, int Y, int T, hipStream_t s) {
     if (a.T != T) return hipErrorInvalidValue;
-    size_t lds = ifft_rows_sum_lds(a.maxfX);
-    bool prime = false;
-    for (int g = 0; g < a.ngroups; ++g) prime = prime || (a.grp[g].active && (has_prime(a.grp[g].rp) || has_prime(a.grp[g].rph)));
-    if (wave_big(a.maxfX)) {
-        const dim3 grid(row_blocks(Y, T, 2), (T + 7) / 8), block(128);
-        if (prime) hipLaunchKernelGGL((k_ifft_rows_sum<true, true>), grid, block, lds, s, a);
-        else hipLaunchKernelGGL((k_ifft_rows_sum<false, true>), grid, block, lds, s, a);
-    } else {
-        const dim3 grid(row_blocks(Y, T, ROWS_PER_WG), (T + 7) / 8), block(64 * ROWS_PER_WG);
-        if (prime) hipLaunchKernelGGL((k_ifft_rows_sum<true, false>), grid, block, lds, s, a);
-        else hipLaunchKernelGGL((k_ifft_rows_sum<false, false>), grid, block, lds, s, a);
+    bool prime = false, odd = false;
+    for (int g = 0; g < a.ngroups; ++g) {
+        if (!a.grp[g].active) continue;
+        prime = prime || has_prime(a.grp[g].rp) || has_prime(a.grp[g].rph);
+        odd = odd || (a.grp[g].rp.L & 1);
     }
+    const bool big = wave_big(a.maxfX);
+    with_bool(prime, [&](auto P) {
+        with_bool(odd, [&](auto O) {
+            if (T > 1 && !big)
+                hipLaunchKernelGGL((k_ifft_rows_sum_staged<P.value, O.value>), dim3(row_stage_blocks(Y, T), (T + 7) / 8),
+                                   dim3(64 * ROW_WAVES), row_stage_lds(a.wbuf, T), s, a);
+            else if (big)
+                hipLaunchKernelGGL((k_ifft_rows_sum<P.value, true, true>), dim3(row_blocks(Y, T, 2), (T + 7) / 8),
+                                   dim3(128), ifft_rows_sum_lds(a.maxfX), s, a);
+            else
+                hipLaunchKernelGGL((k_ifft_rows_sum<P.value, false, O.value>),
+                                   dim3(row_blocks(Y, T, ROWS_PER_WG), (T + 7) / 8), dim3(64 * ROWS_PER_WG),
+                                   ifft_rows_sum_lds(a.maxfX), s, a);
+        });
+    });
     return hipGetLastError();
 }
 // c2r of an even length runs as a half-length complex FFT in place.
 int c2r_wave_buffer(int fX) { return (fX & 1) ? fX : fX / 2; }
 size_t ifft_rows_plane_lds(int wbuf, bool big) { return ROWS_PER_WG * (size_t)wbuf * (big ? 2 : 1) * sizeof(float2); }
 hipError_t launch_ifft_rows_plane(const IfftRowPlaneArgs& a, int nplanes, hipStream_t s) {
-    size_t lds = ifft_rows_plane_lds(a.wbuf, a.big != 0);
-    const dim3 grid(row_blocks(a.Y, a.T, ROWS_PER_WG), (a.T + 7) / 8, nplanes), block(64 * ROWS_PER_WG);
-    if (a.prime) {
-        if (a.big) hipLaunchKernelGGL((k_ifft_rows_plane<true, true>), grid, block, lds, s, a);
-        else hipLaunchKernelGGL((k_ifft_rows_plane<true, false>), grid, block, lds, s, a);
-    } else {
-        if (a.big) hipLaunchKernelGGL((k_ifft_rows_plane<false, true>), grid, block, lds, s, a);
-        else hipLaunchKernelGGL((k_ifft_rows_plane<false, false>), grid, block, lds, s, a);
-    }
+    with_bool(a.prime != 0, [&](auto P) {
+        with_bool(a.odd != 0, [&](auto O) {
+            if (a.T > 1 && !a.big) {
+                hipLaunchKernelGGL((k_ifft_rows_plane_staged<P.value, O.value>),
+                                   dim3(row_stage_blocks(a.Y, a.T), (a.T + 7) / 8, nplanes), dim3(64 * ROW_WAVES),
+                                   row_stage_lds(a.wbuf, a.T), s, a);
+                return;
+            }
+            const dim3 grid(row_blocks(a.Y, a.T, ROWS_PER_WG), (a.T + 7) / 8, nplanes), block(64 * ROWS_PER_WG);
+            const size_t lds = ifft_rows_plane_lds(a.wbuf, a.big != 0);
+            if (a.big) hipLaunchKernelGGL((k_ifft_rows_plane<P.value, true, true>), grid, block, lds, s, a);
+            else hipLaunchKernelGGL((k_ifft_rows_plane<P.value, false, O.value>), grid, block, lds, s, a);
+        });
+    });
     return hipGetLastError();
 }
 hipError_t launch_fit(const float* img, const float* im, long long n_per_frame, int T, int im_frames, double* part,
@@ -1579,14 +1778,22 @@ hipError_t configure_kernels(size_t max_lds) {
                         (const void*)k_psf_rows<true>, (const void*)k_psf_cols<true>,
                         (const void*)k_ifft_cols<false, false>, (const void*)k_ifft_cols<true, false>,
                         (const void*)k_ifft_cols<false, true>, (const void*)k_ifft_cols<true, true>,
-                        (const void*)k_ifft_rows_sum<false, false>, (const void*)k_ifft_rows_sum<true, false>,
-                        (const void*)k_ifft_rows_sum<false, true>, (const void*)k_ifft_rows_sum<true, true>,
-                        (const void*)k_ifft_rows_plane<false, false>, (const void*)k_ifft_rows_plane<true, false>,
-                        (const void*)k_ifft_rows_plane<false, true>, (const void*)k_ifft_rows_plane<true, true>,
                         (const void*)k_spec_pack,
                         (const void*)k_small_fft_grouped, (const void*)k_ifft_cols_grouped<false>,
                         (const void*)k_ifft_cols_grouped<true>};
     std::vector<const void*> all(std::begin(ks), std::end(ks));
+    for (bool prime : {false, true})
+        for (bool odd : {false, true})
+            with_bool(prime, [&](auto P) {
+                with_bool(odd, [&](auto O) {
+                    all.push_back((const void*)k_ifft_rows_sum<P.value, false, O.value>);
+                    all.push_back((const void*)k_ifft_rows_sum_staged<P.value, O.value>);
+                    all.push_back((const void*)k_ifft_rows_plane<P.value, false, O.value>);
+                    all.push_back((const void*)k_ifft_rows_plane_staged<P.value, O.value>);
+                    all.push_back((const void*)k_ifft_rows_sum<P.value, true, true>);
+                    all.push_back((const void*)k_ifft_rows_plane<P.value, true, true>);
+                });
+            });
     for (int slots : {2, 4})
         for (int ns = 1; ns <= slots; ns *= 2)
             for (bool pp : {false, true})

@@ -142,7 +142,7 @@ __device__ __forceinline__ void wave_pass_prime(float2* buf, int es, int L, int 
 // pitches such as 7, 13, 19 are compiled separately, so that the prime pass's
 // registers do not lower the occupancy of the 5-smooth kernels).
 template <int LMAX, bool PRIME = false>
-__device__ void wave_fft(float2* buf, int es, const RadixPlan& rp, const float2* __restrict__ tw, bool inv,
+__device__ __forceinline__ void wave_fft(float2* buf, int es, const RadixPlan& rp, const float2* __restrict__ tw, bool inv,
                          int lane) {
     int Ns = 1;
     for (int p = 0; p < rp.n; ++p) {
