@@ -751,7 +751,7 @@ int flf_plan(flf_ctx* ctx, int nnum, int Y, int X, int T, int nz, const int* s2)
         // FFT workgroup shapes.
         g.RB = std::min(16, fft_batch_cap(g.rpX, ctx->max_lds));
         g.CBp = std::min(16, fft_batch_cap(g.rpY, ctx->max_lds));
-        g.CBi = 8;
+        g.CBi = 4;                               // (measured at COL_LANES)
         while (g.CBi > 1 && ifft_cols_lds(g.CBi, gt.fY) > ctx->max_lds) --g.CBi;
         if (g.RB < 1 || g.CBp < 1 || ifft_cols_lds(g.CBi, gt.fY) > ctx->max_lds)
             return fail(ctx, FLF_EINVAL, "Fourier grid too large for the LDS FFT");

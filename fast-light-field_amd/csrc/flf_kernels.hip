@@ -995,8 +995,8 @@ void k_mac_grouped(MacGrouped ga) {
 // that neighbouring lanes read neighbouring bins.  The output holds rows
 // [y][k1][frame of the block].
 // A workgroup takes CB columns: CB / nf columns k1 of nf frames, or CB of the
-// nf frames of one column.  grid (column blocks, planes x frame blocks), one
-// wave per column (blockDim = 64*CB); LDS CB*fY + fY (twiddles).
+// nf frames of one column.  grid (column blocks, planes x frame blocks),
+// COL_LANES lanes per column; LDS CB*fY + fY (twiddles).
 // ---------------------------------------------------------------------------
 struct ColBlocks {
     int fc, kc, nfg;                 // frames and columns per workgroup, frame groups
@@ -1004,6 +1004,16 @@ struct ColBlocks {
         : fc(nf < CB ? nf : CB), kc(nf < CB ? CB / nf : 1), nfg((nf + fc - 1) / fc) {}
     __host__ __device__ int count(int rfX) const { return (rfX + kc - 1) / kc * nfg; }
 };
+// Lanes per column: two waves (registers for half the butterflies each), one
+// where the transform runs out of place.  Bound: the LDS passes' latency.  The
+// columns of a workgroup fill LDS, so waves in flight come from the lanes per
+// column and overlap of one workgroup's loads with another's passes from two
+// workgroups per CU: 4 columns of 2 waves (the plan's default) against 8 of
+// one took 8 frames of 1455^2 x 41 planes from 4.62 to 2.85 ms (6.8 GB; 4
+// columns of one wave 3.40, 8 of two 4.04), one frame 603 -> 388 us.  XCD
+// neighbours share the 128-byte lines that 4 columns or frames split.
+template <bool BIG>
+constexpr int COL_LANES = BIG ? 64 : 128;
 template <bool PRIME, bool BIG>
 __device__ __forceinline__ void ifft_cols_body(const IfftColArgs& a, int colblk, int batch) {
     extern __shared__ float2 lds[];
@@ -1023,63 +1033,68 @@ __device__ __forceinline__ void ifft_cols_body(const IfftColArgs& a, int colblk,
     const float2* in = a.A + ((long long)plane * a.T + t0) * a.A_bstride + f0;
     const int* idx = a.colidx + (long long)k10 * fY;
     for (int i = threadIdx.x; i < fY; i += blockDim.x) tw[i] = a.twY[i];
-    constexpr int B = 8;                        // loads in flight per thread
-    const int total = fY * ncol;
-    const float rfn = 1.0f / (float)fn, rN = 1.0f / (float)a.N, rfY = 1.0f / (float)fY;
-    for (int i0 = threadIdx.x; i0 < total; i0 += blockDim.x * B) {
-        float2 v[B];
-        int src[B], dst[B];
+    // Thread -> frame fl and every nslot-th of the columns' entries (kk, y0, m),
+    // stepped without divisions.
+    const int tid = threadIdx.x, nslot = blockDim.x / fn;
+    const int slot = tid / fn, fl = tid - slot * fn;
+    if (slot < nslot) {
+        constexpr int B = 8;                    // loads in flight per thread
+        const int N = a.N, rY = a.rY, Q = fY * (ncol / fn);
+        const int sm = nslot % N, sy = nslot / N % rY, sk = nslot / N / rY;
+        int m = slot % N, y0 = slot / N % rY, kk = slot / N / rY;
+        for (int q0 = slot; q0 < Q; q0 += nslot * B) {
+            float2 v[B];
+            int src[B];
 #pragma unroll
-        for (int u = 0; u < B; ++u) {
-            // element -> frame (fastest), entry of the column, column
-            const int i = min(i0 + u * (int)blockDim.x, total - 1);
-            int fl, m, e;
-            const int q = div_small(i, fn, rfn, fl);
-            const int kk = div_small(q, fY, rfY, e);
-            const int y0 = div_small(e, a.N, rN, m);
-            src[u] = idx[q] * nf + fl;
-            dst[u] = (kk * fn + fl) * cs + y0 + m * a.rY;
+            for (int u = 0; u < B; ++u) src[u] = idx[min(q0 + u * nslot, Q - 1)] * nf + fl;
+#pragma unroll
+            for (int u = 0; u < B; ++u) v[u] = in[src[u]];
+            for (int q = 1; q < a.nsum; ++q) {     // partial accumulators, fixed order
+#pragma unroll
+                for (int u = 0; u < B; ++u) v[u] = cadd(v[u], in[src[u] + q * a.A_sstride]);
+            }
+#pragma unroll
+            for (int u = 0; u < B; ++u) {
+                if (q0 + u * nslot < Q) C[(kk * fn + fl) * cs + y0 + m * rY] = v[u];
+                m += sm;
+                y0 += sy;
+                kk += sk;
+                if (m >= N) { m -= N; ++y0; }
+                if (y0 >= rY) { y0 -= rY; ++kk; }
+            }
         }
-#pragma unroll
-        for (int u = 0; u < B; ++u) v[u] = in[src[u]];
-        for (int q = 1; q < a.nsum; ++q) {     // partial accumulators, fixed order
-#pragma unroll
-            for (int u = 0; u < B; ++u) v[u] = cadd(v[u], in[src[u] + q * a.A_sstride]);
-        }
-#pragma unroll
-        for (int u = 0; u < B; ++u)
-            if (i0 + u * (int)blockDim.x < total) C[dst[u]] = v[u];
     }
     __syncthreads();
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    constexpr int NT = COL_LANES<BIG>;
+    const int lane = tid & (NT - 1), col = tid / NT;
     if constexpr (BIG) {
-        if (wv < ncol) wave_fft_pp<PRIME>(C + wv * cs, C2 + wv * cs, a.rpY, tw, true, lane);
+        if (col < ncol) wave_fft_pp<PRIME>(C + col * cs, C2 + col * cs, a.rpY, tw, true, lane);
+        __syncthreads();
     } else {
-        if (wv < ncol) wave_fft<2048, PRIME>(C + wv * cs, 1, a.rpY, tw, true, lane);
+        wave_fft<2048, PRIME, NT>(C + col * cs, 1, a.rpY, tw, true, lane);   // (columns past ncol: not stored)
     }
-    __syncthreads();
     const float2* Res = (BIG && (a.rpY.n & 1)) ? C2 : C;   // after an odd pass count: the second buffer
     float2* out = a.out + ((long long)plane * a.T + t0) * a.out_bstride + (long long)k10 * nf + f0;
     const int rowst = a.rfX * nf;
-    for (int i = threadIdx.x; i < a.Yout * CB; i += blockDim.x) {
-        const int y = i / CB, cc = i - y * CB;
-        if (cc < ncol) {
-            int fl;
-            const int kk = div_small(cc, fn, rfn, fl);
-            out[(long long)y * rowst + kk * nf + fl] = Res[cc * cs + y];
-        }
+    const int cc = tid % CB;                    // blockDim = NT * CB: fixed column, every NT-th row
+    if (cc < ncol) {
+        const int kk = cc / fn;
+        const float2* R = Res + cc * cs;
+        out += kk * nf + cc - kk * fn;
+        for (int y = tid / CB; y < a.Yout; y += NT) out[(long long)y * rowst] = R[y];
     }
 }
 template <bool PRIME, bool BIG>
-__global__ __launch_bounds__(512) void k_ifft_cols(IfftColArgs a) {
-    ifft_cols_body<PRIME, BIG>(a, blockIdx.x, blockIdx.y);
+__global__ __launch_bounds__(8 * COL_LANES<BIG>) void k_ifft_cols(IfftColArgs a) {
+    ifft_cols_body<PRIME, BIG>(a, xcd_block(blockIdx.x, gridDim.x), blockIdx.y);
 }
 // All active grid groups: grid x flattened over (group, batch, column
 // block), nchunks[g] = column blocks of group g; one CB for every group.
 template <bool PRIME>
-__global__ __launch_bounds__(512) void k_ifft_cols_grouped(IfftColGrouped ga) {
+__global__ __launch_bounds__(8 * COL_LANES<false>) void k_ifft_cols_grouped(IfftColGrouped ga) {
     const GroupPick p = pick_group(ga.gg, blockIdx.x);
-    ifft_cols_body<PRIME, false>(ga.a[p.g], p.rem % p.nch, p.rem / p.nch);
+    const int b = xcd_block(p.rem, p.n);
+    ifft_cols_body<PRIME, false>(ga.a[p.g], b % p.nch, b / p.nch);
 }
 
 // c2r of one row by one wave.  row: rfX = L/2+1 half-spectrum values rs apart (global);
@@ -1239,13 +1254,13 @@ __device__ __forceinline__ void stage_rows(float2* buf, int bs, const float2* __
     constexpr int B = 8;                        // loads in flight per thread
     const int total = r.rows * rfX * r.n;
     const float rn = 1.0f / (float)r.n, rrf = 1.0f / (float)rfX;
-    for (int i0 = threadIdx.x; i0 < total; i0 += 64 * ROW_WAVES * B) {
+    for (int i0 = threadIdx.x; i0 < total; i0 += (int)blockDim.x * B) {
         float2 v[B];
 #pragma unroll
-        for (int u = 0; u < B; ++u) v[u] = src[min(i0 + u * 64 * ROW_WAVES, total - 1)];
+        for (int u = 0; u < B; ++u) v[u] = src[min(i0 + u * (int)blockDim.x, total - 1)];
 #pragma unroll
         for (int u = 0; u < B; ++u) {
-            const int i = i0 + u * 64 * ROW_WAVES;
+            const int i = i0 + u * (int)blockDim.x;
             int f, k;
             const int row = div_small(div_small(i, r.n, rn, f), rfX, rrf, k);
             if (i < total) buf[(row * r.n + f) * bs + k] = v[u];
@@ -1255,7 +1270,7 @@ __device__ __forceinline__ void stage_rows(float2* buf, int bs, const float2* __
 __device__ __forceinline__ void stage_table(float2* tab, int L, const float2* __restrict__ twh, const float2* __restrict__ twf) {
     const int n = (L & 1) ? L : L / 2;
     const float2* t = (L & 1) ? twf : twh;
-    for (int i = threadIdx.x; i < n; i += 64 * ROW_WAVES) tab[i] = t[i];
+    for (int i = threadIdx.x; i < n; i += blockDim.x) tab[i] = t[i];
 }
 
 template <int XPL>
@@ -1326,7 +1341,7 @@ __global__ __launch_bounds__(64 * (BIG ? 2 : ROWS_PER_WG)) void k_ifft_rows_sum(
 }
 
 // The same for several frames, rows staged through LDS (see stage_rows);
-// grid (ceil(Y / (ROW_WAVES / n)), ceil(T / 8)), block 64 * ROW_WAVES.
+// grid (ceil(Y / (ROW_WAVES / n)), ceil(T / 8)), a wave per row and frame.
 template <bool PRIME, bool ODD>
 __global__ __launch_bounds__(64 * ROW_WAVES) void k_ifft_rows_sum_staged(IfftRowSumArgs a) {
     extern __shared__ float2 lds[];
@@ -1444,9 +1459,10 @@ __global__ __launch_bounds__(64 * ROWS_PER_WG) void k_ifft_rows_plane(IfftRowPla
 }
 
 // The same for several frames, rows staged through LDS (see stage_rows);
-// grid (ceil(Y / (ROW_WAVES / n)), ceil(T / 8), nplanes), block 64 * ROW_WAVES.
+// grid (ceil(Y / (ROW_WAVES / n)), ceil(T / 8), nplanes), a wave per row and frame.
 template <bool PRIME, bool ODD>
-__global__ __launch_bounds__(64 * ROW_WAVES) void k_ifft_rows_plane_staged(IfftRowPlaneArgs a) {
+__global__ __launch_bounds__(64 * ROW_WAVES) __attribute__((amdgpu_waves_per_eu(4)))
+void k_ifft_rows_plane_staged(IfftRowPlaneArgs a) {
     extern __shared__ float2 lds[];
     reset_smax(a.smax, a.nsmax);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -1679,13 +1695,13 @@ int ifft_col_blocks(const IfftColArgs& a) {
 hipError_t launch_ifft_cols_grouped(const IfftColGrouped& ga, int CB, bool prime, size_t lds, hipStream_t s) {
     const GroupedGrid& gg = ga.gg;
     if (CB < 1 || CB > 8 || gg.ngroups < 1 || gg.ngroups > FLF_MAX_GROUPS) return hipErrorInvalidValue;
-    if (prime) hipLaunchKernelGGL(k_ifft_cols_grouped<true>, dim3(gg.start[gg.ngroups]), dim3(64 * CB), lds, s, ga);
-    else hipLaunchKernelGGL(k_ifft_cols_grouped<false>, dim3(gg.start[gg.ngroups]), dim3(64 * CB), lds, s, ga);
+    if (prime) hipLaunchKernelGGL(k_ifft_cols_grouped<true>, dim3(gg.start[gg.ngroups]), dim3(COL_LANES<false> * CB), lds, s, ga);
+    else hipLaunchKernelGGL(k_ifft_cols_grouped<false>, dim3(gg.start[gg.ngroups]), dim3(COL_LANES<false> * CB), lds, s, ga);
     return hipGetLastError();
 }
 hipError_t launch_ifft_cols(const IfftColArgs& a, int nbatch, hipStream_t s) {
     size_t lds = ifft_cols_lds(a.CB, a.rpY.L);
-    const dim3 grid(ifft_col_blocks(a), nbatch), block(64 * a.CB);
+    const dim3 grid(ifft_col_blocks(a), nbatch), block((wave_big(a.rpY.L) ? COL_LANES<true> : COL_LANES<false>) * a.CB);
     const bool big = wave_big(a.rpY.L);
     if (has_prime(a.rpY)) {
         if (big) hipLaunchKernelGGL((k_ifft_cols<true, true>), grid, block, lds, s, a);
@@ -1705,10 +1721,15 @@ size_t ifft_rows_sum_lds(int maxfX) {
 static int row_blocks(int Y, int T, int rows) { return (Y * std::min(8, T) + rows - 1) / rows; }
 // Staged rows: the transform's table and one buffer per wave (149 KB at most,
 // rows of 2047).
+static int row_stage_waves(int T) {
+    int w = 0;
+    for (int t0 = 0; t0 < T; t0 += 8) w = std::max(w, ROW_WAVES / std::min(8, T - t0) * std::min(8, T - t0));
+    return w;
+}
 static size_t row_stage_lds(int wbuf, int T) {
     int bs = 0;
     for (int n : {std::min(8, T), T > 8 && T % 8 ? T % 8 : std::min(8, T)}) bs = std::max(bs, row_stage_stride(wbuf, n));
-    return ((size_t)wbuf + (size_t)ROW_WAVES * bs) * sizeof(float2);
+    return ((size_t)wbuf + (size_t)row_stage_waves(T) * bs) * sizeof(float2);
 }
 // Workgroups over the rows: a block of n frames takes ROW_WAVES / n rows each.
 static int row_stage_blocks(int Y, int T) {
@@ -1734,7 +1755,7 @@ hipError_t launch_ifft_rows_sum(const IfftRowSumArgs& a, int Y, int T, hipStream
         with_bool(odd, [&](auto O) {
             if (T > 1 && !big)
                 hipLaunchKernelGGL((k_ifft_rows_sum_staged<P.value, O.value>), dim3(row_stage_blocks(Y, T), (T + 7) / 8),
-                                   dim3(64 * ROW_WAVES), row_stage_lds(a.wbuf, T), s, a);
+                                   dim3(64 * row_stage_waves(T)), row_stage_lds(a.wbuf, T), s, a);
             else if (big)
                 hipLaunchKernelGGL((k_ifft_rows_sum<P.value, true, true>), dim3(row_blocks(Y, T, 2), (T + 7) / 8),
                                    dim3(128), ifft_rows_sum_lds(a.maxfX), s, a);
@@ -1754,7 +1775,7 @@ hipError_t launch_ifft_rows_plane(const IfftRowPlaneArgs& a, int nplanes, hipStr
         with_bool(a.odd != 0, [&](auto O) {
             if (a.T > 1 && !a.big) {
                 hipLaunchKernelGGL((k_ifft_rows_plane_staged<P.value, O.value>),
-                                   dim3(row_stage_blocks(a.Y, a.T), (a.T + 7) / 8, nplanes), dim3(64 * ROW_WAVES),
+                                   dim3(row_stage_blocks(a.Y, a.T), (a.T + 7) / 8, nplanes), dim3(64 * row_stage_waves(a.T)),
                                    row_stage_lds(a.wbuf, a.T), s, a);
                 return;
             }

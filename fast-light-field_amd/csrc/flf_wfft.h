@@ -45,10 +45,18 @@ __device__ __forceinline__ void twiddle_powers(float2* a, const float2* __restri
     }
 }
 
-template <int R, int LMAX>
+// NT lanes on one sequence: 64 (one wave), or several waves, which then meet at
+// workgroup barriers (every sequence of the workgroup runs the same plan).
+template <int NT>
+__device__ __forceinline__ void seq_sync() {
+    if constexpr (NT == 64) wave_sync();
+    else __syncthreads();
+}
+
+template <int R, int LMAX, int NT>
 __device__ __forceinline__ void wave_pass(float2* buf, int es, int L, int Ns, const float2* __restrict__ tw,
                                           bool inv, int lane) {
-    constexpr int MAXQ = (LMAX / R + 63) / 64;
+    constexpr int MAXQ = (LMAX / R + NT - 1) / NT;
     const int M = L / R;
     const int tstep = L / (Ns * R);
     const float rNs = 1.0f / (float)Ns;
@@ -56,7 +64,7 @@ __device__ __forceinline__ void wave_pass(float2* buf, int es, int L, int Ns, co
     float2 v[MAXQ][R];
 #pragma unroll
     for (int q = 0; q < MAXQ; ++q) {
-        const int j = lane + 64 * q;
+        const int j = lane + NT * q;
         if (j < M) {
             int k;
             div_small(j, Ns, rNs, k);
@@ -69,10 +77,10 @@ __device__ __forceinline__ void wave_pass(float2* buf, int es, int L, int Ns, co
             for (int t = 0; t < R; ++t) v[q][t] = a[t];
         }
     }
-    wave_sync();
+    seq_sync<NT>();
 #pragma unroll
     for (int q = 0; q < MAXQ; ++q) {
-        const int j = lane + 64 * q;
+        const int j = lane + NT * q;
         if (j < M) {
             int k;
             const int o = div_small(j, Ns, rNs, k) * Ns * R + k;   // recomputed: fewer live registers
@@ -80,7 +88,7 @@ __device__ __forceinline__ void wave_pass(float2* buf, int es, int L, int Ns, co
             for (int t = 0; t < R; ++t) buf[(o + t * Ns) * es] = v[q][t];
         }
     }
-    wave_sync();
+    seq_sync<NT>();
 }
 
 // Last pass of an odd prime radix P (5 < P <= FLF_PRIME_MAX; Ns = L / P):
@@ -91,10 +99,11 @@ __device__ __forceinline__ void wave_pass(float2* buf, int es, int L, int Ns, co
 // twiddle sequences are running products of one table entry, re-read from
 // the table every 8 steps (at most 7 roundings), so that only a few table
 // reads are live at a time.
+template <int NT>
 __device__ __forceinline__ void wave_pass_prime(float2* buf, int es, int L, int P, const float2* __restrict__ tw,
                                                 bool inv, int lane) {
     const int M = L / P;
-    for (int j = lane; j < M; j += 64) {
+    for (int j = lane; j < M; j += NT) {
         float2 a[FLF_PRIME_MAX];
         a[0] = buf[j * es];
         {
@@ -134,28 +143,28 @@ __device__ __forceinline__ void wave_pass_prime(float2* buf, int es, int L, int 
             buf[(j + q * M) * es] = y;
         }
     }
-    wave_sync();
+    seq_sync<NT>();
 }
 
-// In-place transform of one sequence by one wave (inv: unnormalised inverse).
+// In-place transform of one sequence by NT lanes (inv: unnormalised inverse).
 // PRIME: the plan may end with an odd prime radix above 5 (kernels for lenslet
 // pitches such as 7, 13, 19 are compiled separately, so that the prime pass's
 // registers do not lower the occupancy of the 5-smooth kernels).
-template <int LMAX, bool PRIME = false>
-__device__ __forceinline__ void wave_fft(float2* buf, int es, const RadixPlan& rp, const float2* __restrict__ tw, bool inv,
-                         int lane) {
+template <int LMAX, bool PRIME = false, int NT = 64>
+__device__ __forceinline__ void wave_fft(float2* buf, int es, const RadixPlan& rp, const float2* __restrict__ tw,
+                                         bool inv, int lane) {
     int Ns = 1;
     for (int p = 0; p < rp.n; ++p) {
         const int R = rp.r[p];
         switch (R) {
-            case 8: wave_pass<8, LMAX>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 6: wave_pass<6, LMAX>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 4: wave_pass<4, LMAX>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 2: wave_pass<2, LMAX>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 3: wave_pass<3, LMAX>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 5: wave_pass<5, LMAX>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 8: wave_pass<8, LMAX, NT>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 6: wave_pass<6, LMAX, NT>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 4: wave_pass<4, LMAX, NT>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 2: wave_pass<2, LMAX, NT>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 3: wave_pass<3, LMAX, NT>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 5: wave_pass<5, LMAX, NT>(buf, es, rp.L, Ns, tw, inv, lane); break;
             default:
-                if constexpr (PRIME) wave_pass_prime(buf, es, rp.L, R, tw, inv, lane);   // last pass
+                if constexpr (PRIME) wave_pass_prime<NT>(buf, es, rp.L, R, tw, inv, lane);   // last pass
                 break;
         }
         Ns *= R;
