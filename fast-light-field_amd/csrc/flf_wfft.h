@@ -91,58 +91,73 @@ __device__ __forceinline__ void wave_pass(float2* buf, int es, int L, int Ns, co
     seq_sync<NT>();
 }
 
-// Last pass of an odd prime radix P (5 < P <= FLF_PRIME_MAX; Ns = L / P):
-// butterfly j < M = L/P reads x[j + t M], t < P, and writes y_q to
-// x[j + q M]: the same positions, so each lane takes its butterflies one at
-// a time.  y_q = sum_t x[j + t M] W^(j t) W^(M t q mod L), W = tw[1], the
-// table tw[m] = exp(-2 pi i m / L) (conjugated for the inverse).  Both
-// twiddle sequences are running products of one table entry, re-read from
-// the table every 8 steps (at most 7 roundings), so that only a few table
-// reads are live at a time.
+// Butterfly j of the last pass of an odd prime radix P (5 < P <= FLF_PRIME_MAX;
+// M = Ns = L / P): y_q = sum_t x[j + t M] W^(j t) W_P^(t q), W = tw[1], W_P =
+// W^M, the table tw[m] = exp(-2 pi i m / L) (conjugated for the inverse).  y_q
+// goes to dst[j + q M], the positions the inputs held in src.  The powers of
+// W^j are running products, re-read from the table every 8 steps (at most 7
+// roundings).  With a_t the twiddled inputs and (c, s) = W_P^(t q), outputs q and
+// P - q share their sums over the pairs (t, P - t),
+//   y = a_0 + sum c (a_t + a_(P-t)) +- i sum s (a_t - a_(P-t)),
+// 4 real operations and one table read (the same for every lane) per pair and
+// q, where the sum over all t took 10 and two running products per t and q.
+__device__ __forceinline__ void prime_butterfly(const float2* src, float2* dst, int es, int j, int M, int P,
+                                                const float2* __restrict__ tw, bool inv) {
+    constexpr int H = FLF_PRIME_MAX / 2;
+    const int h = P / 2;
+    const float2 a0 = src[j * es];
+    float2 sp[H], df[H], y0 = a0;
+    {
+        float2 w1 = tw[j], wP = tw[j * P];                     // W^j, W^(j P)
+        if (inv) { w1.y = -w1.y; wP.y = -wP.y; }
+        float2 w = w1;
+#pragma unroll
+        for (int t = 1; t <= H; ++t) {
+            if (t <= h) {
+                if ((t & 7) == 0) {                            // exact table value W^(j t), j t < L
+                    w = tw[j * t];
+                    if (inv) w.y = -w.y;
+                }
+                const float2 x = cmul(src[(j + t * M) * es], w);
+                const float2 y = cmul(src[(j + (P - t) * M) * es], cmul(wP, cconj(w)));
+                sp[t - 1] = cadd(x, y);
+                df[t - 1] = csub(x, y);
+                w = cmul(w, w1);
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 1; t <= H; ++t)
+        if (t <= h) y0 = cadd(y0, sp[t - 1]);
+    dst[j * es] = y0;
+    for (int q = 1; q <= h; ++q) {
+        float2 c = a0, d = make_float2(0.f, 0.f);
+        int m = 0;                                             // t q mod P
+#pragma unroll
+        for (int t = 1; t <= H; ++t) {
+            if (t <= h) {
+                m += q;
+                if (m >= P) m -= P;
+                const float2 w = tw[m * M];
+                c.x += sp[t - 1].x * w.x;
+                c.y += sp[t - 1].y * w.x;
+                d.x += df[t - 1].x * w.y;
+                d.y += df[t - 1].y * w.y;
+            }
+        }
+        if (inv) { d.x = -d.x; d.y = -d.y; }
+        dst[(j + q * M) * es] = make_float2(c.x - d.y, c.y + d.x);
+        dst[(j + (P - q) * M) * es] = make_float2(c.x + d.y, c.y - d.x);
+    }
+}
+
+// Last pass of a prime radix in place: each lane takes its butterflies one at
+// a time, whose outputs lie where its inputs did.
 template <int NT>
 __device__ __forceinline__ void wave_pass_prime(float2* buf, int es, int L, int P, const float2* __restrict__ tw,
                                                 bool inv, int lane) {
     const int M = L / P;
-    for (int j = lane; j < M; j += NT) {
-        float2 a[FLF_PRIME_MAX];
-        a[0] = buf[j * es];
-        {
-            float2 w1 = tw[j];                                 // W^j
-            if (inv) w1.y = -w1.y;
-            float2 w = w1;
-#pragma unroll
-            for (int t = 1; t < FLF_PRIME_MAX; ++t) {
-                if (t < P) {
-                    if ((t & 7) == 0) {                        // exact table value W^(j t), j t < L
-                        w = tw[j * t];
-                        if (inv) w.y = -w.y;
-                    }
-                    a[t] = cmul(buf[(j + t * M) * es], w);
-                    w = cmul(w, w1);
-                }
-            }
-        }
-        for (int q = 0; q < P; ++q) {
-            float2 wq = tw[q * M];                             // W_P^q
-            if (inv) wq.y = -wq.y;
-            float2 y = a[0], w = wq;
-            int m = q;                                         // t q mod P
-#pragma unroll
-            for (int t = 1; t < FLF_PRIME_MAX; ++t) {
-                if (t < P) {
-                    if ((t & 7) == 0) {
-                        w = tw[m * M];
-                        if (inv) w.y = -w.y;
-                    }
-                    y = cadd(y, cmul(a[t], w));
-                    w = cmul(w, wq);
-                    m += q;
-                    if (m >= P) m -= P;
-                }
-            }
-            buf[(j + q * M) * es] = y;
-        }
-    }
+    for (int j = lane; j < M; j += NT) prime_butterfly(buf, buf, es, j, M, P, tw, inv);
     seq_sync<NT>();
 }
 
@@ -197,51 +212,11 @@ __device__ __forceinline__ void wave_pass_oop(const float2* src, float2* dst, in
     wave_sync();
 }
 
-// The prime last pass (Ns = L / P) out of place: y_q of butterfly j goes to
-// dst[j + q M], the positions its inputs held in src.
+// The prime last pass out of place.
 __device__ __forceinline__ void wave_pass_prime_oop(const float2* src, float2* dst, int L, int P,
                                                     const float2* __restrict__ tw, bool inv, int lane) {
     const int M = L / P;
-    for (int j = lane; j < M; j += 64) {
-        float2 a[FLF_PRIME_MAX];
-        a[0] = src[j];
-        {
-            float2 w1 = tw[j];
-            if (inv) w1.y = -w1.y;
-            float2 w = w1;
-#pragma unroll
-            for (int t = 1; t < FLF_PRIME_MAX; ++t) {
-                if (t < P) {
-                    if ((t & 7) == 0) {
-                        w = tw[j * t];
-                        if (inv) w.y = -w.y;
-                    }
-                    a[t] = cmul(src[j + t * M], w);
-                    w = cmul(w, w1);
-                }
-            }
-        }
-        for (int q = 0; q < P; ++q) {
-            float2 wq = tw[q * M];
-            if (inv) wq.y = -wq.y;
-            float2 y = a[0], w = wq;
-            int m = q;
-#pragma unroll
-            for (int t = 1; t < FLF_PRIME_MAX; ++t) {
-                if (t < P) {
-                    if ((t & 7) == 0) {
-                        w = tw[m * M];
-                        if (inv) w.y = -w.y;
-                    }
-                    y = cadd(y, cmul(a[t], w));
-                    w = cmul(w, wq);
-                    m += q;
-                    if (m >= P) m -= P;
-                }
-            }
-            dst[j + q * M] = y;
-        }
-    }
+    for (int j = lane; j < M; j += 64) prime_butterfly(src, dst, 1, j, M, P, tw, inv);
     wave_sync();
 }
 
