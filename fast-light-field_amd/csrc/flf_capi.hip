@@ -27,6 +27,7 @@ struct Group {
     RadixPlan rpYw, rpXw, rpXhw;      // fY, fX, fX/2 for the wave-level inverse transforms (wide radices)
     int RB = 1, CBp = 1, CBi = 1;     // FFT batching (psf rows, psf cols, ifft cols)
     ChunkDesc* d_chunks = nullptr;
+    unsigned* d_sidx = nullptr;       // small-FFT output order (SmallFFTArgs::sidx)
     ItemDesc* d_items = nullptr;
     TileDesc* d_tiles = nullptr;
     int* d_bu = nullptr;
@@ -537,7 +538,7 @@ int run_backward_groups(flf_ctx* ctx, const float* img, const std::vector<char>&
         a.twY = g.twRY; a.twX = g.twRX;
         a.S = g.d_S_bwd;
         a.S_off = ctx->d_zeros;
-        a.chunks = g.d_chunks; a.nchunks = (int)gt.chunks.size(); a.NH = gt.slots;
+        a.sidx = g.d_sidx; a.nchunks = (int)gt.chunks.size(); a.NH = gt.slots;
         a.fY = gt.fY; a.fX = gt.fX;
         a.S_tstride = s_frame_stride(ctx, g);
         a.fdims = frame_dims(ctx);
@@ -726,8 +727,10 @@ int flf_plan(flf_ctx* ctx, int nnum, int Y, int X, int T, int nz, const int* s2)
             std::string e = build_grid_tables(nnum, fY, fX, g.gt);
             if (!e.empty()) return fail(ctx, FLF_EINVAL, e);
             const int ro = ctx->radix_order;
+            const bool wide = small_fft_big(g.gt.rY, g.gt.rX);   // (its wave-level passes take radices 2..5)
             if (!make_radix_plan(fY, g.rpY, false, ro) || !make_radix_plan(fX, g.rpX, false, ro) ||
-                !make_radix_plan(g.gt.rY, g.rpYr, false, ro) || !make_radix_plan(g.gt.rX, g.rpXr, false, ro) ||
+                !(wide ? make_radix_plan(g.gt.rY, g.rpYr, false, ro) : make_reduced_plan(g.gt.rY, g.rpYr, ro)) ||
+                !(wide ? make_radix_plan(g.gt.rX, g.rpXr, false, ro) : make_reduced_plan(g.gt.rX, g.rpXr, ro)) ||
                 !make_radix_plan(fY, g.rpYw, true, ro) || !make_radix_plan(fX, g.rpXw, true, ro) ||
                 (fX % 2 == 0 &&
                  (!make_radix_plan(fX / 2, g.rpXh, false, ro) || !make_radix_plan(fX / 2, g.rpXhw, true, ro))))
@@ -782,6 +785,14 @@ int flf_plan(flf_ctx* ctx, int nnum, int Y, int X, int T, int nz, const int* s2)
         int rc;
         if ((rc = upload(ctx, &g.d_chunks, gt.chunks))) return rc;
         if ((rc = upload(ctx, &g.d_items, gt.items))) return rc;
+        std::vector<unsigned> sidx;
+        for (auto& ch : gt.chunks)
+            for (int j = 0; j < gt.slots; ++j) {
+                const bool neg = 2 * ch.res1[j] > gt.rX;
+                const int k0 = neg ? (gt.rY - ch.res0[j]) % gt.rY : ch.res0[j], k1 = neg ? gt.rX - ch.res1[j] : ch.res1[j];
+                sidx.push_back((unsigned)k1 | (unsigned)k0 << 8 | (neg ? 1u << 31 : 0u));
+            }
+        if ((rc = upload(ctx, &g.d_sidx, sidx))) return rc;
         if ((rc = upload(ctx, &g.d_tiles, gt.tiles))) return rc;
         if ((rc = upload(ctx, &g.d_bu, gt.u_bu))) return rc;
         if ((rc = upload(ctx, &g.d_au, gt.u_au))) return rc;
@@ -1165,7 +1176,7 @@ int run_forward_groups(flf_ctx* ctx, const float* vol, const float* vol2, const 
         a.twY = g.twRY; a.twX = g.twRX;
         a.S = g.d_S_fwd;
         a.S_off = g.d_Soff_fwd;
-        a.chunks = g.d_chunks; a.nchunks = (int)gt.chunks.size(); a.NH = gt.slots;
+        a.sidx = g.d_sidx; a.nchunks = (int)gt.chunks.size(); a.NH = gt.slots;
         a.fY = gt.fY; a.fX = gt.fX;
         a.S_tstride = s_frame_stride(ctx, g);
         a.fdims = frame_dims(ctx);

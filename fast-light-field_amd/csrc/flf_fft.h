@@ -25,16 +25,23 @@ constexpr int FLF_PRIME_MAX = 31;
 template <int R>
 __device__ __forceinline__ void dft_small(float2* a, float sign);
 
-// cos and sin of 2 pi m / N for m = 0..3: the internal twiddles of the
-// two-level butterflies below (N = 6, 8).
+// cos and sin of 2 pi m / N, m = 0..6: the internal twiddles of the two-level
+// butterflies below (N = 6, 8, 9, 10, 12).
 template <int N>
 __device__ __forceinline__ float2 unit_root(int m, float sign) {
-    constexpr float c6[4] = {1.000000000e+00f, 5.000000000e-01f, -5.000000000e-01f, -1.000000000e+00f};
-    constexpr float s6[4] = {0.000000000e+00f, 8.660254038e-01f, 8.660254038e-01f, 0.000000000e+00f};
-    constexpr float c8[4] = {1.000000000e+00f, 7.071067812e-01f, 0.000000000e+00f, -7.071067812e-01f};
-    constexpr float s8[4] = {0.000000000e+00f, 7.071067812e-01f, 1.000000000e+00f, 7.071067812e-01f};
-    const float c = N == 6 ? c6[m] : c8[m];
-    const float sn = N == 6 ? s6[m] : s8[m];
+    constexpr float h = 8.660254038e-01f, r = 7.071067812e-01f;
+    constexpr float c6[7] = {1.f, 0.5f, -0.5f, -1.f, -0.5f, 0.5f, 1.f};
+    constexpr float s6[7] = {0.f, h, h, 0.f, -h, -h, 0.f};
+    constexpr float c8[7] = {1.f, r, 0.f, -r, -1.f, -r, 0.f};
+    constexpr float s8[7] = {0.f, r, 1.f, r, 0.f, -r, -1.f};
+    constexpr float c9[7] = {1.f, 7.660444431e-01f, 1.736481777e-01f, -0.5f, -9.396926208e-01f, -9.396926208e-01f, -0.5f};
+    constexpr float s9[7] = {0.f, 6.427876097e-01f, 9.848077530e-01f, h, 3.420201433e-01f, -3.420201433e-01f, -h};
+    constexpr float c10[7] = {1.f, 8.090169944e-01f, 3.090169944e-01f, -3.090169944e-01f, -8.090169944e-01f, -1.f, -8.090169944e-01f};
+    constexpr float s10[7] = {0.f, 5.877852523e-01f, 9.510565163e-01f, 9.510565163e-01f, 5.877852523e-01f, 0.f, -5.877852523e-01f};
+    constexpr float c12[7] = {1.f, h, 0.5f, 0.f, -0.5f, -h, -1.f};
+    constexpr float s12[7] = {0.f, 0.5f, h, 1.f, h, 0.5f, 0.f};
+    const float c = N == 6 ? c6[m] : N == 8 ? c8[m] : N == 9 ? c9[m] : N == 10 ? c10[m] : c12[m];
+    const float sn = N == 6 ? s6[m] : N == 8 ? s8[m] : N == 9 ? s9[m] : N == 10 ? s10[m] : s12[m];
     return make_float2(c, sign * sn);
 }
 
@@ -121,6 +128,12 @@ __device__ __forceinline__ void dft_small(float2* a, float sign) {
         dft_two_level<2, 3>(a, sign);
     } else if constexpr (R == 8) {
         dft_two_level<2, 4>(a, sign);
+    } else if constexpr (R == 9) {
+        dft_two_level<3, 3>(a, sign);
+    } else if constexpr (R == 10) {
+        dft_two_level<2, 5>(a, sign);
+    } else if constexpr (R == 12) {
+        dft_two_level<3, 4>(a, sign);
     }
 }
 

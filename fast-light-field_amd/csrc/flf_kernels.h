@@ -35,7 +35,7 @@ struct SmallFFTArgs {
     RadixPlan rpY, rpX;          // lengths rY, rX
     const float2* twY;           // exp(-2 pi i m / rY), m < rY
     const float2* twX;           // exp(-2 pi i m / rX)
-    const ChunkDesc* chunks;     // MAC chunks of the grid (output order)
+    const unsigned* sidx;        // [chunk][NH]: H column, H row << 8, conjugate << 31 (output order)
     int nchunks, NH;             // chunks; residues stored per chunk (4 quad / 2 pair)
     int fY, fX;
     float2* S;                   // [chunk][N*N][NH] per source plane and frame

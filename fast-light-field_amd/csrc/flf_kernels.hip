@@ -37,20 +37,22 @@ __device__ __forceinline__ int centred_res(int k, int r) {
 // ---------------------------------------------------------------------------
 // Small FFTs of the lenslet-subsampled source (py_light_field.cpp:1001-1027):
 // S_{b,a} = FFT_r(src[b::N, a::N] zero-padded to rY x rX), half spectrum.
-// grid (N*N, T, nsrc), block 64 * SFFT_WAVES.  Rows are real, so two rows are
-// transformed as one complex sequence, in place in those two rows' storage
-// (2 (rX/2+1) >= rX entries; one spare row at the end), and separated
-// afterwards; each wave transforms two such row pairs at once, then pairs of
-// columns of the half spectrum.  The r x (r/2+1) spectrum takes 60 KB of LDS
-// at r = 120, so two workgroups share a CU; at 80 VGPRs a SIMD holds 6
-// waves, i.e. 12 waves per workgroup (1455^2 forward projection: small FFT
-// part 1.5% faster than with 8; the kernel is bound by LDS latency).
-// Output S[z][t][off][k0][k1], k1 in [0, rX/2].
+// grid (N*N, T, nsrc), block 64 * sfft_waves.  Rows are real, so two rows are
+// transformed as one complex sequence, in those two rows' storage (2 (rX/2+1)
+// >= rX entries; one spare row at the end), and separated afterwards; then
+// the columns of the half spectrum.  Every pass is done by the whole
+// workgroup (wg_pass: two passes of radix 8 to 12 at most lengths from 64 to
+// 120, the first straight from memory): shared out by waves, two sequences
+// filled 40 to 50 of 64 lanes and took 3 passes of radix 2 to 5.  The r x
+// (r/2+1) spectrum takes 60 KB of LDS at r = 120, so two workgroups share a CU.
+// Bound: latency (the strided pixel loads, barriers), vector instructions for
+// half of the time: 42k per workgroup before at r = 110, 17k now.  1455^2 x 41
+// planes: 8 frames 5.05 -> 3.73 ms, one frame 700 -> 540 us.
 // ---------------------------------------------------------------------------
-#ifndef FLF_SFFT_WAVES
-#define FLF_SFFT_WAVES 12
-#endif
-constexpr int SFFT_WAVES = FLF_SFFT_WAVES;
+// Variants by the longer reduced length (see small_fft_variant).
+enum SmallFFT { SFFT_64, SFFT_128, SFFT_256 };
+constexpr int sfft_len(SmallFFT v) { return v == SFFT_64 ? 64 : v == SFFT_128 ? 128 : 256; }
+constexpr int sfft_waves(SmallFFT v) { return v == SFFT_64 ? 4 : 12; }
 
 // Workgroup id -> work index such that the workgroups of one XCD take a
 // contiguous range: the dispatcher deals consecutive workgroup ids of a grid
@@ -115,10 +117,10 @@ __device__ __forceinline__ void reset_smax(float* smax, int n) {
 
 // One (lenslet offset, frame, source plane) of a grid group; src0/src2/
 // tsplit: the source buffers of the call.
-template <bool BIG>
+template <SmallFFT V>
 __device__ __forceinline__ void small_fft_body(const SmallFFTArgs& a, const float* src0, const float* src2,
                                                int tsplit, int off, int t, int z) {
-    constexpr int RMAX = BIG ? 256 : 128;          // reduced grid length (BIG: 129..256)
+    constexpr int RMAX = sfft_len(V), SFFT_WAVES = sfft_waves(V);
     extern __shared__ float2 lds[];
     const int N = a.N;
     const int b = off / N, aa = off % N;
@@ -139,73 +141,8 @@ __device__ __forceinline__ void small_fft_body(const SmallFFTArgs& a, const floa
     const int Yv = a.fdims ? a.fdims[t].x : a.Y, Xv = a.fdims ? a.fdims[t].y : a.X;
     const int Ys = max(0, (Yv - b + N - 1) / N);
     const int Xs = max(0, (Xv - aa + N - 1) / N);
-    for (int i = Ys * rXh + threadIdx.x; i < rY * rXh; i += blockDim.x) H[i] = make_float2(0.f, 0.f);
-    __syncthreads();
-    for (int q = wv; 4 * q < Ys; q += SFFT_WAVES) {
-        const int y0 = 4 * q;
-        const int np = (y0 + 2 < Ys) ? 2 : 1;      // row pairs in this group of four rows
-        float2* P = H + (long long)y0 * rXh;      // pair s at P + 2 s rXh
-        // All loads of the group's four rows are issued before any is used.
-        constexpr int XC = RMAX / 64;              // 64-lane column chunks per row
-        float v[2][XC][2];
-#pragma unroll
-        for (int sq = 0; sq < 2; ++sq) {
-            const int ya = y0 + 2 * sq, yb = ya + 1;
-            const float* r0 = src + (long long)(b + N * ya) * a.src_pitch + aa;
-            const float* r1 = src + (long long)(b + N * yb) * a.src_pitch + aa;
-#pragma unroll
-            for (int c = 0; c < XC; ++c) {
-                const int x = lane + 64 * c;
-                const bool in = sq < np && x < Xs;
-                v[sq][c][0] = in ? r0[N * x] : 0.f;
-                v[sq][c][1] = (in && yb < Ys) ? r1[N * x] : 0.f;
-            }
-        }
-#pragma unroll
-        for (int sq = 0; sq < 2; ++sq)
-#pragma unroll
-            for (int c = 0; c < XC; ++c) {
-                const int x = lane + 64 * c;
-                if (sq < np && x < rX) P[2 * sq * rXh + x] = make_float2(v[sq][c][0], v[sq][c][1]);
-            }
-        wave_sync();
-        wave_fft_ns<RMAX, 2>(P, 1, 2 * rXh, np, a.rpX, twX, false, lane);
-        // Separate: row ya = (Z + Zc)/2, row yb = (Z - Zc)/(2i), Zc = conj Z(-k);
-        // all reads before the in-place writes.
-        float2 ev[2][2], od[2][2];
-#pragma unroll
-        for (int sq = 0; sq < 2; ++sq)
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                const int k = lane + 64 * m;
-                if (sq < np && k < rXh) {
-                    const float2* Z = P + 2 * sq * rXh;
-                    const float2 zk = Z[k];
-                    const float2 zc = cconj(Z[(rX - k) % rX]);
-                    ev[sq][m] = make_float2(0.5f * (zk.x + zc.x), 0.5f * (zk.y + zc.y));
-                    od[sq][m] = make_float2(0.5f * (zk.y - zc.y), -0.5f * (zk.x - zc.x));
-                }
-            }
-        wave_sync();
-#pragma unroll
-        for (int sq = 0; sq < 2; ++sq)
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                const int k = lane + 64 * m;
-                if (sq < np && k < rXh) {
-                    const int ya = y0 + 2 * sq;
-                    H[ya * rXh + k] = ev[sq][m];
-                    H[(ya + 1) * rXh + k] = (ya + 1 < Ys) ? od[sq][m] : make_float2(0.f, 0.f);
-                }
-            }
-        wave_sync();
-    }
-    __syncthreads();
-    for (int c = 2 * wv; c < rXh; c += 2 * SFFT_WAVES)
-        wave_fft_ns<RMAX, 2>(H + c, rXh, 1, min(2, rXh - c), a.rpY, twY, false, lane);
     // Sub-sampling phases of this offset: exp(-2 pi i b kt0 / fY) and
     // exp(-2 pi i a kt1 / fX), kt the centred residue (0 for r/2).
-    __syncthreads();
     for (int i = threadIdx.x; i < rY + rX; i += blockDim.x) {
         const bool isY = i < rY;
         const int k = isY ? i : i - rY;
@@ -217,36 +154,161 @@ __device__ __forceinline__ void small_fft_body(const SmallFFTArgs& a, const floa
         sincospif(-2.0f * (float)m / (float)f, &sn, &cs);
         (isY ? phY : phX)[k] = make_float2(cs, sn);
     }
-    __syncthreads();
+    if constexpr (V == SFFT_256) {
+        for (int i = Ys * rXh + threadIdx.x; i < rY * rXh; i += blockDim.x) H[i] = make_float2(0.f, 0.f);
+        __syncthreads();
+        for (int q = wv; 4 * q < Ys; q += SFFT_WAVES) {
+            const int y0 = 4 * q;
+            const int np = (y0 + 2 < Ys) ? 2 : 1;      // row pairs in this group of four rows
+            float2* P = H + (long long)y0 * rXh;      // pair s at P + 2 s rXh
+            // All loads of the group's four rows are issued before any is used.
+            constexpr int XC = RMAX / 64;              // 64-lane column chunks per row
+            float v[2][XC][2];
+#pragma unroll
+            for (int sq = 0; sq < 2; ++sq) {
+                const int ya = y0 + 2 * sq, yb = ya + 1;
+                const float* r0 = src + (long long)(b + N * ya) * a.src_pitch + aa;
+                const float* r1 = src + (long long)(b + N * yb) * a.src_pitch + aa;
+#pragma unroll
+                for (int c = 0; c < XC; ++c) {
+                    const int x = lane + 64 * c;
+                    const bool in = sq < np && x < Xs;
+                    v[sq][c][0] = in ? r0[N * x] : 0.f;
+                    v[sq][c][1] = (in && yb < Ys) ? r1[N * x] : 0.f;
+                }
+            }
+#pragma unroll
+            for (int sq = 0; sq < 2; ++sq)
+#pragma unroll
+                for (int c = 0; c < XC; ++c) {
+                    const int x = lane + 64 * c;
+                    if (sq < np && x < rX) P[2 * sq * rXh + x] = make_float2(v[sq][c][0], v[sq][c][1]);
+                }
+            wave_sync();
+            wave_fft_ns<RMAX, 2>(P, 1, 2 * rXh, np, a.rpX, twX, false, lane);
+            // Separate: row ya = (Z + Zc)/2, row yb = (Z - Zc)/(2i), Zc = conj Z(-k);
+            // all reads before the in-place writes.
+            float2 ev[2][2], od[2][2];
+#pragma unroll
+            for (int sq = 0; sq < 2; ++sq)
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    const int k = lane + 64 * m;
+                    if (sq < np && k < rXh) {
+                        const float2* Z = P + 2 * sq * rXh;
+                        const float2 zk = Z[k];
+                        const float2 zc = cconj(Z[(rX - k) % rX]);
+                        ev[sq][m] = make_float2(0.5f * (zk.x + zc.x), 0.5f * (zk.y + zc.y));
+                        od[sq][m] = make_float2(0.5f * (zk.y - zc.y), -0.5f * (zk.x - zc.x));
+                    }
+                }
+            wave_sync();
+#pragma unroll
+            for (int sq = 0; sq < 2; ++sq)
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    const int k = lane + 64 * m;
+                    if (sq < np && k < rXh) {
+                        const int ya = y0 + 2 * sq;
+                        H[ya * rXh + k] = ev[sq][m];
+                        H[(ya + 1) * rXh + k] = (ya + 1 < Ys) ? od[sq][m] : make_float2(0.f, 0.f);
+                    }
+                }
+            wave_sync();
+        }
+        __syncthreads();
+        for (int c = 2 * wv; c < rXh; c += 2 * SFFT_WAVES)
+            wave_fft_ns<RMAX, 2>(H + c, rXh, 1, min(2, rXh - c), a.rpY, twY, false, lane);
+        __syncthreads();
+    } else {
+        // Every pass by the whole workgroup.  Rows: sequence q is the row pair
+        // (2 q, 2 q + 1) as one complex sequence, stored in the pair's rows of H;
+        // the first pass loads it from memory.
+        constexpr int NTH = 64 * SFFT_WAVES, MAXB = (RMAX / 2 + 1) * RMAX;
+        const int np = (Ys + 1) / 2;
+        for (int i = 2 * np * rXh + threadIdx.x; i < rY * rXh; i += NTH) H[i] = make_float2(0.f, 0.f);
+        const float* r0 = src + (long long)b * a.src_pitch + aa;
+        const int rp = N * a.src_pitch;           // (row offsets within a plane: 32 bits)
+        auto load = [&](auto& v, int q, int j, int M) {
+            constexpr int R = sizeof(v) / sizeof(v[0]);
+            const float* ra = r0 + 2 * q * rp + N * j;
+            const bool two = 2 * q + 1 < Ys;
+#pragma unroll
+            for (int t = 0; t < R; ++t) {
+                const bool in = j + t * M < Xs;
+                const int x = in ? N * t * M : 0;
+                v[t].x = in ? ra[x] : 0.f;
+                v[t].y = in && two ? ra[x + rp] : 0.f;
+            }
+        };
+        if (np > 0) {
+            wg_pass_any<MAXB, NTH, true>(a.rpX.n ? a.rpX.r[0] : 1, H, 1, 2 * rXh, np, false, rX, 1, twX, load);
+            int Ns = a.rpX.n ? a.rpX.r[0] : 1;
+            for (int p = 1; p < a.rpX.n; ++p) {
+                wg_pass_any<MAXB, NTH, false>(a.rpX.r[p], H, 1, 2 * rXh, np, false, rX, Ns, twX, NoLoad());
+                Ns *= a.rpX.r[p];
+            }
+        }
+        // Separate: row ya = (Z + Zc)/2, row yb = (Z - Zc)/(2i), Zc = conj Z(-k);
+        // all reads before the in-place writes.
+        {
+            constexpr int MQ = (RMAX / 2 * (RMAX / 2 + 1) + NTH - 1) / NTH;
+            const float rrx = 1.0f / (float)rXh;
+            float2 ev[MQ], od[MQ];
+#pragma unroll
+            for (int m = 0; m < MQ; ++m) {
+                const int i = threadIdx.x + m * NTH;
+                if (i < np * rXh) {
+                    int k;
+                    const int q = div_small(i, rXh, rrx, k);
+                    const float2* Z = H + 2 * q * rXh;
+                    const float2 zk = Z[k], zc = cconj(Z[k == 0 ? 0 : rX - k]);
+                    ev[m] = make_float2(0.5f * (zk.x + zc.x), 0.5f * (zk.y + zc.y));
+                    od[m] = make_float2(0.5f * (zk.y - zc.y), -0.5f * (zk.x - zc.x));
+                    if (2 * q + 1 >= Ys) od[m] = make_float2(0.f, 0.f);
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < MQ; ++m) {
+                const int i = threadIdx.x + m * NTH;
+                if (i < np * rXh) {
+                    int k;
+                    const int q = div_small(i, rXh, rrx, k);
+                    H[2 * q * rXh + k] = ev[m];
+                    H[(2 * q + 1) * rXh + k] = od[m];
+                }
+            }
+            __syncthreads();
+        }
+        int Ns = 1;
+        for (int p = 0; p < a.rpY.n; ++p) {
+            wg_pass_any<MAXB, NTH, false>(a.rpY.r[p], H, rXh, 1, rXh, true, rY, Ns, twY, NoLoad());
+            Ns *= a.rpY.r[p];
+        }
+    }
     // Orbit-ordered, phase-folded output S[chunk][off][j] for the first NH
     // residues of each chunk's residue list (the MAC reads one contiguous
-    // block per chunk).
-    float2* S = a.S + a.S_off[z] + (long long)t * a.S_tstride;
-    // OU entries per thread at a time: their residue loads (chunk
-    // descriptors, from the caches) are all in flight before the first is
-    // used.
-    const int NH = a.NH, NN = N * N;
+    // block per chunk), by the table sidx: H row and column, conjugated where
+    // only the negated residue is in the half plane (its phases are conjugates
+    // too).  All of a thread's table loads are in flight before the first is used.
+    float2* S = a.S + a.S_off[z] + (long long)t * a.S_tstride + off * a.NH;
+    const int NH = a.NH, lg = NH == 4 ? 2 : 1, step = N * N * NH;
     const int total = a.nchunks * NH;
     float mx = 0.f;                               // largest component written
-    constexpr int OU = 4;
+    constexpr int OU = 8;
     for (int i0 = threadIdx.x; i0 < total; i0 += OU * blockDim.x) {
-        int k0[OU], k1[OU];
+        unsigned sx[OU];
 #pragma unroll
-        for (int u = 0; u < OU; ++u) {
-            const int i = min(i0 + u * (int)blockDim.x, total - 1);
-            const int w = i / NH, j = i - w * NH;
-            k0[u] = a.chunks[w].res0[j];
-            k1[u] = a.chunks[w].res1[j];
-        }
+        for (int u = 0; u < OU; ++u) sx[u] = a.sidx[min(i0 + u * (int)blockDim.x, total - 1)];
 #pragma unroll
         for (int u = 0; u < OU; ++u) {
             const int i = i0 + u * (int)blockDim.x;
             if (i < total) {
-                const int w = i / NH, j = i - w * NH;
-                float2 v = (2 * k1[u] <= rX) ? H[k0[u] * rXh + k1[u]]
-                                             : cconj(H[((rY - k0[u]) % rY) * rXh + (rX - k1[u])]);
-                v = cmul(v, cmul(phY[k0[u]], phX[k1[u]]));
-                S[((long long)w * NN + off) * NH + j] = v;
+                const int k1 = sx[u] & 0xff, k0 = (sx[u] >> 8) & 0xff;
+                float2 v = cmul(H[k0 * rXh + k1], cmul(phY[k0], phX[k1]));
+                if (sx[u] >> 31) v.y = -v.y;
+                S[(long long)(i >> lg) * step + (i & (NH - 1))] = v;
                 mx = fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y)));   // (NaN does not count: it scales to NaN)
             }
         }
@@ -262,16 +324,17 @@ __device__ __forceinline__ void small_fft_body(const SmallFFTArgs& a, const floa
                   *wgmax);
 }
 
-template <bool BIG>
-__global__ __launch_bounds__(64 * SFFT_WAVES) void k_small_fft(SmallFFTArgs a) {
-    small_fft_body<BIG>(a, a.src, a.src2, a.tsplit, xcd_block(blockIdx.x, a.N * a.N), blockIdx.y, blockIdx.z);
+template <SmallFFT V>
+__global__ __launch_bounds__(64 * sfft_waves(V)) void k_small_fft(SmallFFTArgs a) {
+    small_fft_body<V>(a, a.src, a.src2, a.tsplit, xcd_block(blockIdx.x, a.N * a.N), blockIdx.y, blockIdx.z);
 }
 // grid (N*N, T, sum over groups of their source planes): z flattened over
 // (group, plane).
-__global__ __launch_bounds__(64 * SFFT_WAVES) void k_small_fft_grouped(SmallFFTGrouped ga) {
+template <SmallFFT V>
+__global__ __launch_bounds__(64 * sfft_waves(V)) void k_small_fft_grouped(SmallFFTGrouped ga) {
     const GroupPick p = pick_group(ga.gg, blockIdx.z);
     const SmallFFTArgs& a = ga.a[p.g];
-    small_fft_body<false>(a, a.src, a.src2, a.tsplit, xcd_block(blockIdx.x, a.N * a.N), blockIdx.y, p.rem);
+    small_fft_body<V>(a, a.src, a.src2, a.tsplit, xcd_block(blockIdx.x, a.N * a.N), blockIdx.y, p.rem);
 }
 
 // ---------------------------------------------------------------------------
@@ -1595,21 +1658,34 @@ static bool has_prime(const RadixPlan& rp) { return plan_has_prime(rp); }
 size_t small_fft_lds(int rY, int rX) {
     return ((size_t)(rY + 1) * (rX / 2 + 1) + 2 * (size_t)(rY + rX) + 1) * sizeof(float2);
 }
-// Reduced grids above 128 points take the 256-point wave transforms.
+// Reduced grids above 128 points take the 256-point wave transforms, those up
+// to 64 workgroups of 4 waves (a pass of a 64 x 64 grid has 256 butterflies; 8
+// workgroups share a CU), the others 12 (a pass of 120 x 120 has 720, LDS holds
+// 2 workgroups).
 bool small_fft_big(int rY, int rX) { return rY > 128 || rX > 128; }
+static SmallFFT small_fft_variant(int rY, int rX) {
+    return small_fft_big(rY, rX) ? SFFT_256 : std::max(rY, rX) > 64 ? SFFT_128 : SFFT_64;
+}
 hipError_t launch_small_fft(const SmallFFTArgs& a, int nsrc, int T, hipStream_t s) {
     size_t lds = small_fft_lds(a.rpY.L, a.rpX.L);
     if (a.rpY.L > 256 || a.rpX.L > 256) return hipErrorInvalidValue;
-    if (small_fft_big(a.rpY.L, a.rpX.L))
-        hipLaunchKernelGGL(k_small_fft<true>, dim3(a.N * a.N, T, nsrc), dim3(64 * SFFT_WAVES), lds, s, a);
-    else
-        hipLaunchKernelGGL(k_small_fft<false>, dim3(a.N * a.N, T, nsrc), dim3(64 * SFFT_WAVES), lds, s, a);
+    const dim3 grid(a.N * a.N, T, nsrc);
+    switch (small_fft_variant(a.rpY.L, a.rpX.L)) {
+        case SFFT_256: hipLaunchKernelGGL(k_small_fft<SFFT_256>, grid, dim3(64 * sfft_waves(SFFT_256)), lds, s, a); break;
+        case SFFT_128: hipLaunchKernelGGL(k_small_fft<SFFT_128>, grid, dim3(64 * sfft_waves(SFFT_128)), lds, s, a); break;
+        default: hipLaunchKernelGGL(k_small_fft<SFFT_64>, grid, dim3(64 * sfft_waves(SFFT_64)), lds, s, a);
+    }
     return hipGetLastError();
 }
 hipError_t launch_small_fft_grouped(const SmallFFTGrouped& ga, int N, int T, size_t lds, hipStream_t s) {
-    if (ga.gg.ngroups < 1 || ga.gg.ngroups > FLF_MAX_GROUPS) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_small_fft_grouped, dim3(N * N, T, ga.gg.start[ga.gg.ngroups]), dim3(64 * SFFT_WAVES), lds, s,
-                       ga);
+    const GroupedGrid& gg = ga.gg;
+    if (gg.ngroups < 1 || gg.ngroups > FLF_MAX_GROUPS) return hipErrorInvalidValue;
+    SmallFFT v = SFFT_64;
+    for (int g = 0; g < gg.ngroups; ++g) v = std::max(v, small_fft_variant(ga.a[g].rpY.L, ga.a[g].rpX.L));
+    const dim3 grid(N * N, T, gg.start[gg.ngroups]);
+    if (v == SFFT_256) return hipErrorInvalidValue;               // (not grouped)
+    if (v == SFFT_128) hipLaunchKernelGGL(k_small_fft_grouped<SFFT_128>, grid, dim3(64 * sfft_waves(v)), lds, s, ga);
+    else hipLaunchKernelGGL(k_small_fft_grouped<SFFT_64>, grid, dim3(64 * sfft_waves(v)), lds, s, ga);
     return hipGetLastError();
 }
 hipError_t launch_psf_rows(const PsfRowArgs& a, int nu, hipStream_t s) {
@@ -1794,13 +1870,13 @@ hipError_t launch_fit(const float* img, const float* im, long long n_per_frame, 
     return hipGetLastError();
 }
 hipError_t configure_kernels(size_t max_lds) {
-    const void* ks[] = {(const void*)k_small_fft<false>, (const void*)k_small_fft<true>,
+    const void* ks[] = {(const void*)k_small_fft<SFFT_64>, (const void*)k_small_fft<SFFT_128>, (const void*)k_small_fft<SFFT_256>,
                         (const void*)k_psf_rows<false>, (const void*)k_psf_cols<false>,
                         (const void*)k_psf_rows<true>, (const void*)k_psf_cols<true>,
                         (const void*)k_ifft_cols<false, false>, (const void*)k_ifft_cols<true, false>,
                         (const void*)k_ifft_cols<false, true>, (const void*)k_ifft_cols<true, true>,
                         (const void*)k_spec_pack,
-                        (const void*)k_small_fft_grouped, (const void*)k_ifft_cols_grouped<false>,
+                        (const void*)k_small_fft_grouped<SFFT_64>, (const void*)k_small_fft_grouped<SFFT_128>, (const void*)k_ifft_cols_grouped<false>,
                         (const void*)k_ifft_cols_grouped<true>};
     std::vector<const void*> all(std::begin(ks), std::end(ks));
     for (bool prime : {false, true})

@@ -89,6 +89,28 @@ bool make_radix_plan(int L, RadixPlan& rp, bool wide, int order) {
     return m == 1;
 }
 
+bool make_reduced_plan(int L, RadixPlan& rp, int order) {
+    if (L > 128 || order < 0 || order >= FLF_RADIX_ORDERS) return false;
+    // best[m]: the last radix of the shortest plan of m (then of the least sum
+    // of radices, that is of work)
+    const int radices[9] = {2, 3, 4, 5, 6, 8, 9, 10, 12};
+    std::vector<std::array<int, 3>> best(L + 1, {1 << 20, 0, 0});      // passes, sum, radix
+    best[1] = {0, 0, 0};
+    for (int m = 2; m <= L; ++m)
+        for (int R : radices)
+            if (m % R == 0) {
+                const std::array<int, 3> b{best[m / R][0] + 1, best[m / R][1] + R, R};
+                if (b < best[m]) best[m] = b;
+            }
+    if (best[L][0] > FLF_MAX_RADIX_PASSES) return false;
+    rp.L = L;
+    rp.n = 0;
+    for (int m = L; m > 1; m /= best[m][2]) rp.r[rp.n++] = best[m][2];
+    std::sort(rp.r, rp.r + rp.n);
+    if (order != 1) std::reverse(rp.r, rp.r + rp.n);
+    return true;
+}
+
 // Half-unit alias of coordinate x on an axis of length N*r.
 static int alias2(int x, int r, int N) {
     int k = x % r, m = x / r;

@@ -49,6 +49,9 @@ struct GridTables {
 };
 
 // Builds the tables; returns an empty string or an error message.
+// Plan of a reduced-grid transform (L <= 128, 5-smooth): radices up to 12, as
+// few passes as possible, largest first (order 1: reversed).
+bool make_reduced_plan(int L, RadixPlan& rp, int order = 0);
 std::string build_grid_tables(int N, int fY, int fX, GridTables& gt);
 
 }  // namespace flf

@@ -20,6 +20,14 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Values of a pass that the compiler is not to reason about: the indices of
+// every radix would otherwise be computed ahead of the loop over the passes
+// and held in registers (60 to 100 more in the workgroup-level passes).
+__device__ __forceinline__ void opaque_lane_length(int& lane, int& L) {
+    L = __builtin_amdgcn_readfirstlane(L);
+    asm volatile("" : "+v"(lane), "+s"(L));
+}
+
 // q = n / d and r = n % d for 0 <= n < 2^22 and d >= 1, from the float
 // reciprocal rd = 1/d of the pass (one correction step makes it exact:
 // n * rd is within 0.5 of n / d).
@@ -53,9 +61,12 @@ __device__ __forceinline__ void seq_sync() {
     else __syncthreads();
 }
 
-template <int R, int LMAX, int NT>
+template <int R, int LMAX, int NT, bool OPAQUE>
 __device__ __forceinline__ void wave_pass(float2* buf, int es, int L, int Ns, const float2* __restrict__ tw,
                                           bool inv, int lane) {
+    // (one wave of 5-smooth plans: the registers do not limit its kernels, held
+    // indices are 10 % faster)
+    if constexpr (OPAQUE) opaque_lane_length(lane, L);
     constexpr int MAXQ = (LMAX / R + NT - 1) / NT;
     const int M = L / R;
     const int tstep = L / (Ns * R);
@@ -156,6 +167,7 @@ __device__ __forceinline__ void prime_butterfly(const float2* src, float2* dst, 
 template <int NT>
 __device__ __forceinline__ void wave_pass_prime(float2* buf, int es, int L, int P, const float2* __restrict__ tw,
                                                 bool inv, int lane) {
+    opaque_lane_length(lane, L);
     const int M = L / P;
     for (int j = lane; j < M; j += NT) prime_butterfly(buf, buf, es, j, M, P, tw, inv);
     seq_sync<NT>();
@@ -172,12 +184,12 @@ __device__ __forceinline__ void wave_fft(float2* buf, int es, const RadixPlan& r
     for (int p = 0; p < rp.n; ++p) {
         const int R = rp.r[p];
         switch (R) {
-            case 8: wave_pass<8, LMAX, NT>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 6: wave_pass<6, LMAX, NT>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 4: wave_pass<4, LMAX, NT>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 2: wave_pass<2, LMAX, NT>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 3: wave_pass<3, LMAX, NT>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 5: wave_pass<5, LMAX, NT>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 8: wave_pass<8, LMAX, NT, PRIME || (NT > 64)>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 6: wave_pass<6, LMAX, NT, PRIME || (NT > 64)>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 4: wave_pass<4, LMAX, NT, PRIME || (NT > 64)>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 2: wave_pass<2, LMAX, NT, PRIME || (NT > 64)>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 3: wave_pass<3, LMAX, NT, PRIME || (NT > 64)>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 5: wave_pass<5, LMAX, NT, PRIME || (NT > 64)>(buf, es, rp.L, Ns, tw, inv, lane); break;
             default:
                 if constexpr (PRIME) wave_pass_prime<NT>(buf, es, rp.L, R, tw, inv, lane);   // last pass
                 break;
@@ -193,6 +205,7 @@ __device__ __forceinline__ void wave_fft(float2* buf, int es, const RadixPlan& r
 template <int R>
 __device__ __forceinline__ void wave_pass_oop(const float2* src, float2* dst, int L, int Ns,
                                               const float2* __restrict__ tw, bool inv, int lane) {
+    opaque_lane_length(lane, L);
     const int M = L / R;
     const int tstep = L / (Ns * R);
     const float rNs = 1.0f / (float)Ns;
@@ -309,6 +322,82 @@ __device__ void wave_fft_ns(float2* buf, int es, int ss, int nseq, const RadixPl
             default: wave_pass_ns<5, LMAX, NS>(buf, es, ss, nseq, rp.L, Ns, tw, inv, lane); break;
         }
         Ns *= R;
+    }
+}
+
+// One pass of nseq sequences of length L by the whole workgroup (NTH threads):
+// element e of sequence q is buf[q * ss + e * es], butterflies dealt to the
+// threads with the sequence (by_seq) or the butterfly of a sequence fastest.
+// FIRST: inputs from ld(sequence, element) instead (Ns = 1, buf only written).
+// Twiddles: powers of one table entry, restarted from the table at every fourth
+// (at most 2 roundings).
+template <int R, int MAXB, int NTH, bool FIRST, class Ld>
+__device__ __forceinline__ void wg_pass(float2* buf, int es, int ss, int nseq, bool by_seq, int L, int Ns,
+                                        const float2* __restrict__ tw, Ld ld) {
+    int tid = threadIdx.x;
+    opaque_lane_length(tid, L);
+    constexpr int MAXQ = (MAXB / R + NTH - 1) / NTH;   // MAXB: most nseq * L
+    const int M = L / R, total = nseq * M, d = by_seq ? nseq : M;
+    const float rd = 1.0f / (float)d, rNs = 1.0f / (float)Ns;
+    const int tstep = L / (Ns * R);
+    float2 v[MAXQ][R];
+    int o[MAXQ];
+#pragma unroll
+    for (int q = 0; q < MAXQ; ++q) {
+        const int idx = tid + q * NTH;
+        if (idx < total) {
+            int lo, k = 0;
+            const int hi = div_small(idx, d, rd, lo);
+            const int seq = by_seq ? lo : hi, j = by_seq ? hi : lo;
+            if constexpr (FIRST) {
+                o[q] = seq * ss + j * R * es;
+                ld(v[q], seq, j, M);
+            } else {
+                const int g = div_small(j, Ns, rNs, k);
+                o[q] = seq * ss + (g * Ns * R + k) * es;
+                const float2* b = buf + seq * ss + j * es;
+#pragma unroll
+                for (int t = 0; t < R; ++t) v[q][t] = b[t * M * es];
+                if (Ns > 1) {
+                    const float2 w1 = tw[k * tstep];
+                    float2 w = w1;
+#pragma unroll
+                    for (int t = 1; t < R; ++t) {
+                        if (t > 1) w = (t & 3) == 0 ? tw[t * k * tstep] : cmul(w, w1);
+                        v[q][t] = cmul(v[q][t], w);
+                    }
+                }
+            }
+            dft_small<R>(v[q], -1.f);
+        }
+    }
+    if constexpr (!FIRST) __syncthreads();
+#pragma unroll
+    for (int q = 0; q < MAXQ; ++q)
+        if (tid + q * NTH < total) {
+#pragma unroll
+            for (int t = 0; t < R; ++t) buf[o[q] + t * Ns * es] = v[q][t];
+        }
+    __syncthreads();
+}
+struct NoLoad {
+    template <int R>
+    __device__ void operator()(float2 (&)[R], int, int, int) const {}
+};
+template <int MAXB, int NTH, bool FIRST, class Ld>
+__device__ __forceinline__ void wg_pass_any(int R, float2* buf, int es, int ss, int nseq, bool by_seq, int L, int Ns,
+                                            const float2* __restrict__ tw, Ld ld) {
+    switch (R) {
+        case 12: wg_pass<12, MAXB, NTH, FIRST>(buf, es, ss, nseq, by_seq, L, Ns, tw, ld); break;
+        case 10: wg_pass<10, MAXB, NTH, FIRST>(buf, es, ss, nseq, by_seq, L, Ns, tw, ld); break;
+        case 9: wg_pass<9, MAXB, NTH, FIRST>(buf, es, ss, nseq, by_seq, L, Ns, tw, ld); break;
+        case 8: wg_pass<8, MAXB, NTH, FIRST>(buf, es, ss, nseq, by_seq, L, Ns, tw, ld); break;
+        case 6: wg_pass<6, MAXB, NTH, FIRST>(buf, es, ss, nseq, by_seq, L, Ns, tw, ld); break;
+        case 5: wg_pass<5, MAXB, NTH, FIRST>(buf, es, ss, nseq, by_seq, L, Ns, tw, ld); break;
+        case 4: wg_pass<4, MAXB, NTH, FIRST>(buf, es, ss, nseq, by_seq, L, Ns, tw, ld); break;
+        case 3: wg_pass<3, MAXB, NTH, FIRST>(buf, es, ss, nseq, by_seq, L, Ns, tw, ld); break;
+        case 2: wg_pass<2, MAXB, NTH, FIRST>(buf, es, ss, nseq, by_seq, L, Ns, tw, ld); break;
+        default: wg_pass<1, MAXB, NTH, FIRST>(buf, es, ss, nseq, by_seq, L, Ns, tw, ld); break;   // L = 1
     }
 }
 
