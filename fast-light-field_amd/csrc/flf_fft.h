@@ -15,7 +15,7 @@ namespace flf {
 
 // Largest radix of a pass (wave-level transforms; the block-level passes
 // below use 2..5).
-constexpr int FLF_RADIX_MAX = 8;
+constexpr int FLF_RADIX_MAX = 12;
 // Largest odd prime radix (a prime factor of Nnum above 5, Nnum <= 31).  Such
 // a radix is always the last pass of a plan: then Ns * P = L, every
 // butterfly writes its outputs onto its own inputs, and a thread can take its

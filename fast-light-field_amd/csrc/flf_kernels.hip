@@ -1524,7 +1524,7 @@ __global__ __launch_bounds__(64 * ROWS_PER_WG) void k_ifft_rows_plane(IfftRowPla
 // The same for several frames, rows staged through LDS (see stage_rows);
 // grid (ceil(Y / (ROW_WAVES / n)), ceil(T / 8), nplanes), a wave per row and frame.
 template <bool PRIME, bool ODD>
-__global__ __launch_bounds__(64 * ROW_WAVES) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(64 * ROW_WAVES) __attribute__((amdgpu_waves_per_eu(PRIME || ODD ? 4 : 6)))
 void k_ifft_rows_plane_staged(IfftRowPlaneArgs a) {
     extern __shared__ float2 lds[];
     reset_smax(a.smax, a.nsmax);
@@ -1647,11 +1647,11 @@ namespace flf {
 
 // Whether a plan ends with an odd prime radix above 5 (7, 11, ..., 31; the
 // kernels built with that pass are launched only then).  The other radices
-// are 2..6 and 8.
+// are 2..6, 8, 9, 10 and 12.
 bool plan_has_prime(const RadixPlan& rp) {
     if (rp.n == 0) return false;
     const int r = rp.r[rp.n - 1];
-    return r == 7 || r > 8;
+    return r == 7 || r == 11 || r > 12;
 }
 static bool has_prime(const RadixPlan& rp) { return plan_has_prime(rp); }
 

@@ -51,29 +51,58 @@ int fourier_len(int s1, int s2, int N) {
     return N * smooth5_at_least(red);
 }
 
+// Plan of a 5-smooth length with radices up to 12: as few passes as possible,
+// then the least sum of radices (work), largest first.
+static bool shortest_plan(int L, RadixPlan& rp) {
+    const int radices[9] = {2, 3, 4, 5, 6, 8, 9, 10, 12};
+    std::vector<std::array<int, 3>> best(L + 1, {1 << 20, 0, 0});      // passes, sum, last radix
+    best[1] = {0, 0, 0};
+    for (int m = 2; m <= L; ++m) {
+        if (L % m) continue;
+        for (int R : radices)
+            if (m % R == 0) {
+                const std::array<int, 3> b{best[m / R][0] + 1, best[m / R][1] + R, R};
+                if (b < best[m]) best[m] = b;
+            }
+    }
+    if (best[L][0] > FLF_MAX_RADIX_PASSES - 1) return false;
+    rp.L = L;
+    rp.n = 0;
+    for (int m = L; m > 1; m /= best[m][2]) rp.r[rp.n++] = best[m][2];
+    std::sort(rp.r, rp.r + rp.n);
+    std::reverse(rp.r, rp.r + rp.n);
+    return true;
+}
+
 bool make_radix_plan(int L, RadixPlan& rp, bool wide, int order) {
     rp.L = L;
     rp.n = 0;
-    int m = L;
-    // Block-level transforms use radices 2..5; wave-level ones also take the
-    // composite radices 8 and 6 first, one pass (an LDS round trip) fewer at
-    // most lengths used here.  Radices 9 and 10 were tried: their butterflies
-    // raised the register count of every wave-FFT kernel past the occupancy
-    // its LDS allows, with spills.  Orders 2 and 3 change the radices of
-    // wave-level plans only: the block-level kernels size their butterfly
-    // registers from the plan's radices (fft_batch_cap).
-    const int narrow[4] = {4, 2, 3, 5};
-    const int wider[4][6] = {{8, 6, 4, 5, 3, 2}, {8, 6, 4, 5, 3, 2}, {6, 4, 5, 3, 2, 0}, {5, 3, 8, 6, 4, 2}};
     if (order < 0 || order >= FLF_RADIX_ORDERS) return false;
-    const int* list = wide ? wider[order] : narrow;
-    const int nlist = wide ? 6 : 4;
-    for (int k = 0; k < nlist; ++k) {
-        const int R = list[k];
-        if (R == 0) break;
-        while (m % R == 0) {
-            if (rp.n >= FLF_MAX_RADIX_PASSES) return false;
-            rp.r[rp.n++] = R;
-            m /= R;
+    // Block-level transforms use radices 2..5, wave-level ones the composite
+    // radices up to 12 too, for fewer passes (LDS round trips): 3 or 4 instead
+    // of 4 or 5 at most lengths of 700 to 1800.  Orders 2 and 3 change the
+    // radices of wave-level plans only: the block-level kernels size their
+    // butterfly registers from the plan's radices (fft_batch_cap).
+    const int narrow[4] = {4, 2, 3, 5};
+    const int wider[2][6] = {{6, 4, 5, 3, 2, 0}, {5, 3, 8, 6, 4, 2}};
+    int m = L;
+    if (wide && order < 2) {
+        int smooth = 1;
+        for (int R : {2, 3, 5})
+            while (m % R == 0) { m /= R; smooth *= R; }
+        if (!shortest_plan(smooth, rp)) return false;
+        rp.L = L;
+    } else {
+        const int* list = wide ? wider[order - 2] : narrow;
+        const int nlist = wide ? 6 : 4;
+        for (int k = 0; k < nlist; ++k) {
+            const int R = list[k];
+            if (R == 0) break;
+            while (m % R == 0) {
+                if (rp.n >= FLF_MAX_RADIX_PASSES) return false;
+                rp.r[rp.n++] = R;
+                m /= R;
+            }
         }
     }
     if (order == 1)
@@ -90,24 +119,8 @@ bool make_radix_plan(int L, RadixPlan& rp, bool wide, int order) {
 }
 
 bool make_reduced_plan(int L, RadixPlan& rp, int order) {
-    if (L > 128 || order < 0 || order >= FLF_RADIX_ORDERS) return false;
-    // best[m]: the last radix of the shortest plan of m (then of the least sum
-    // of radices, that is of work)
-    const int radices[9] = {2, 3, 4, 5, 6, 8, 9, 10, 12};
-    std::vector<std::array<int, 3>> best(L + 1, {1 << 20, 0, 0});      // passes, sum, radix
-    best[1] = {0, 0, 0};
-    for (int m = 2; m <= L; ++m)
-        for (int R : radices)
-            if (m % R == 0) {
-                const std::array<int, 3> b{best[m / R][0] + 1, best[m / R][1] + R, R};
-                if (b < best[m]) best[m] = b;
-            }
-    if (best[L][0] > FLF_MAX_RADIX_PASSES) return false;
-    rp.L = L;
-    rp.n = 0;
-    for (int m = L; m > 1; m /= best[m][2]) rp.r[rp.n++] = best[m][2];
-    std::sort(rp.r, rp.r + rp.n);
-    if (order != 1) std::reverse(rp.r, rp.r + rp.n);
+    if (L > 128 || order < 0 || order >= FLF_RADIX_ORDERS || !shortest_plan(L, rp)) return false;
+    if (order == 1) std::reverse(rp.r, rp.r + rp.n);
     return true;
 }
 

@@ -38,9 +38,9 @@ __device__ __forceinline__ int div_small(int n, int d, float rd, int& r) {
     return q;
 }
 
-// a[t] *= w^t for t = 1..R-1, w = tw[k * tstep] (conjugated for the inverse):
-// one table read, the higher powers as running products (at most R - 2
-// roundings, a few ulp), two values live.
+// a[t] *= w^t for t = 1..R-1, w = tw[idx] (conjugated for the inverse): running
+// products, restarted from the table at every fourth power (at most 2
+// roundings).
 template <int R>
 __device__ __forceinline__ void twiddle_powers(float2* a, const float2* __restrict__ tw, int idx, bool inv) {
     float2 w1 = tw[idx];
@@ -48,8 +48,13 @@ __device__ __forceinline__ void twiddle_powers(float2* a, const float2* __restri
     float2 w = w1;
 #pragma unroll
     for (int t = 1; t < R; ++t) {
+        if (t > 1 && (t & 3) == 0) {
+            w = tw[t * idx];
+            if (inv) w.y = -w.y;
+        } else if (t > 1) {
+            w = cmul(w, w1);
+        }
         a[t] = cmul(a[t], w);
-        if (t + 1 < R) w = cmul(w, w1);
     }
 }
 
@@ -64,8 +69,8 @@ __device__ __forceinline__ void seq_sync() {
 template <int R, int LMAX, int NT, bool OPAQUE>
 __device__ __forceinline__ void wave_pass(float2* buf, int es, int L, int Ns, const float2* __restrict__ tw,
                                           bool inv, int lane) {
-    // (one wave of 5-smooth plans: the registers do not limit its kernels, held
-    // indices are 10 % faster)
+    // (one wave, 5-smooth plans up to 1024: the registers do not limit its
+    // kernels, held indices are 6 % faster)
     if constexpr (OPAQUE) opaque_lane_length(lane, L);
     constexpr int MAXQ = (LMAX / R + NT - 1) / NT;
     const int M = L / R;
@@ -180,16 +185,20 @@ __device__ __forceinline__ void wave_pass_prime(float2* buf, int es, int L, int 
 template <int LMAX, bool PRIME = false, int NT = 64>
 __device__ __forceinline__ void wave_fft(float2* buf, int es, const RadixPlan& rp, const float2* __restrict__ tw,
                                          bool inv, int lane) {
+    constexpr bool OPQ = PRIME || NT > 64 || LMAX > 1024;
     int Ns = 1;
     for (int p = 0; p < rp.n; ++p) {
         const int R = rp.r[p];
         switch (R) {
-            case 8: wave_pass<8, LMAX, NT, PRIME || (NT > 64)>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 6: wave_pass<6, LMAX, NT, PRIME || (NT > 64)>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 4: wave_pass<4, LMAX, NT, PRIME || (NT > 64)>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 2: wave_pass<2, LMAX, NT, PRIME || (NT > 64)>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 3: wave_pass<3, LMAX, NT, PRIME || (NT > 64)>(buf, es, rp.L, Ns, tw, inv, lane); break;
-            case 5: wave_pass<5, LMAX, NT, PRIME || (NT > 64)>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 12: wave_pass<12, LMAX, NT, OPQ>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 10: wave_pass<10, LMAX, NT, OPQ>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 9: wave_pass<9, LMAX, NT, OPQ>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 8: wave_pass<8, LMAX, NT, OPQ>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 6: wave_pass<6, LMAX, NT, OPQ>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 4: wave_pass<4, LMAX, NT, OPQ>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 2: wave_pass<2, LMAX, NT, OPQ>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 3: wave_pass<3, LMAX, NT, OPQ>(buf, es, rp.L, Ns, tw, inv, lane); break;
+            case 5: wave_pass<5, LMAX, NT, OPQ>(buf, es, rp.L, Ns, tw, inv, lane); break;
             default:
                 if constexpr (PRIME) wave_pass_prime<NT>(buf, es, rp.L, R, tw, inv, lane);   // last pass
                 break;
@@ -244,6 +253,9 @@ __device__ float2* wave_fft_pp(float2* a, float2* b, const RadixPlan& rp, const 
     for (int p = 0; p < rp.n; ++p) {
         const int R = rp.r[p];
         switch (R) {
+            case 12: wave_pass_oop<12>(src, dst, rp.L, Ns, tw, inv, lane); break;
+            case 10: wave_pass_oop<10>(src, dst, rp.L, Ns, tw, inv, lane); break;
+            case 9: wave_pass_oop<9>(src, dst, rp.L, Ns, tw, inv, lane); break;
             case 8: wave_pass_oop<8>(src, dst, rp.L, Ns, tw, inv, lane); break;
             case 6: wave_pass_oop<6>(src, dst, rp.L, Ns, tw, inv, lane); break;
             case 4: wave_pass_oop<4>(src, dst, rp.L, Ns, tw, inv, lane); break;
