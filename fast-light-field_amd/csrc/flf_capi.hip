@@ -856,9 +856,10 @@ int flf_plan(flf_ctx* ctx, int nnum, int Y, int X, int T, int nz, const int* s2)
             rd.twh = g.twXh;
         }
         Tbwd_total += (long long)nP * Y * gt.rfX;
-        // (rows of a grid up to 2048 points hold X < 2048 samples; longer
-        // ones take the out-of-place kernels, which hold up to 4096)
-        if (ifft_rows_sum_lds(gt.fX) > ctx->max_lds || X > 4096)
+        // The longest rows plans accept (3723 points in 160 KB): tables and four
+        // buffers of a full row, what two long rows per workgroup needed.
+        const size_t row_limit = ((size_t)gt.fX + gt.fX / 2 + 1 + 4 * (size_t)gt.fX) * sizeof(float2);
+        if (row_limit > ctx->max_lds || X > 4096)
             return fail(ctx, FLF_EINVAL, "image row too long for the row transform");
     }
     int rc;

@@ -210,7 +210,6 @@ __host__ __device__ inline int ifft_col_stride(int fY, int CB) {
     const int r = (m / CB) % m;
     return fY + ((r - fY) % m + m) % m;
 }
-size_t ifft_rows_sum_lds(int maxfX);
 size_t ifft_rows_plane_lds(int wbuf, bool big);
 bool wave_big(int L);
 bool small_fft_big(int rY, int rX);

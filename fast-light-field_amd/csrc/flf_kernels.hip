@@ -1160,7 +1160,7 @@ __global__ __launch_bounds__(8 * COL_LANES<false>) void k_ifft_cols_grouped(Ifft
     ifft_cols_body<PRIME, false>(ga.a[p.g], b % p.nch, b / p.nch);
 }
 
-// c2r of one row by one wave.  row: rfX = L/2+1 half-spectrum values rs apart (global);
+// c2r of one row by NT lanes (one wave, or a workgroup).  row: rfX = L/2+1 half-spectrum values rs apart (global);
 // buf: LDS work area (L/2 entries for even L, L for odd L; BIG, for L above
 // 2048: buf2 is a second such area for the out-of-place passes).  For even L the
 // length-L/2 complex transform of Z[k] = E[k] + i O[k],
@@ -1169,20 +1169,20 @@ __global__ __launch_bounds__(8 * COL_LANES<false>) void k_ifft_cols_grouped(Ifft
 // extension and a full-length transform.  The imaginary parts of X[0] and
 // X[L/2] are dropped, as a c2r transform does.  Returns with the result in
 // buf (interleaved real samples for even L, real parts for odd L).
-template <bool PRIME, bool BIG, bool ODD>
+template <bool PRIME, bool BIG, bool ODD, int NT = 64>
 __device__ __forceinline__ float2* wave_c2r(float2* buf, float2* buf2, const float2* __restrict__ row, int L,
                                             const RadixPlan& rph, const float2* twh,
                                             const RadixPlan& rpf, const float2* twf, int lane, int rs) {
     // Loads are issued C2R_BATCH per lane at a time, so that their latencies
     // overlap instead of adding up.
-    constexpr int B = 8;
+    constexpr int B = NT == 64 ? 8 : 4, LE = NT == 64 ? 1024 : 2048;   // (LE: longest half-length transform)
     if (!ODD || (L & 1) == 0) {
         const int L2 = L / 2;
-        for (int k0 = lane; k0 < L2; k0 += 64 * B) {
+        for (int k0 = lane; k0 < L2; k0 += NT * B) {
             float2 xs[B], xrs[B];
 #pragma unroll
             for (int u = 0; u < B; ++u) {
-                const int k = k0 + 64 * u;
+                const int k = k0 + NT * u;
                 if (k < L2) {
                     xs[u] = row[k * rs];
                     xrs[u] = row[(L2 - k) * rs];
@@ -1190,7 +1190,7 @@ __device__ __forceinline__ float2* wave_c2r(float2* buf, float2* buf2, const flo
             }
 #pragma unroll
             for (int u = 0; u < B; ++u) {
-                const int k = k0 + 64 * u;
+                const int k = k0 + NT * u;
                 if (k < L2) {
                     float2 x = xs[u];
                     float2 xr = cconj(xrs[u]);
@@ -1203,22 +1203,22 @@ __device__ __forceinline__ float2* wave_c2r(float2* buf, float2* buf2, const flo
                 }
             }
         }
-        wave_sync();
+        seq_sync<NT>();
         if constexpr (BIG) return wave_fft_pp<PRIME>(buf, buf2, rph, twh, true, lane);
-        wave_fft<1024, PRIME>(buf, 1, rph, twh, true, lane);
+        wave_fft<LE, PRIME, NT>(buf, 1, rph, twh, true, lane);
         return buf;
     } else {
         const int rfX = L / 2 + 1;
-        for (int k0 = lane; k0 < L; k0 += 64 * B) {
+        for (int k0 = lane; k0 < L; k0 += NT * B) {
             float2 vs[B];
 #pragma unroll
             for (int u = 0; u < B; ++u) {
-                const int k = k0 + 64 * u;
+                const int k = k0 + NT * u;
                 if (k < L) vs[u] = k < rfX ? row[k * rs] : cconj(row[(L - k) * rs]);
             }
 #pragma unroll
             for (int u = 0; u < B; ++u) {
-                const int k = k0 + 64 * u;
+                const int k = k0 + NT * u;
                 if (k < L) {
                     float2 v = vs[u];
                     if (k == 0) v.y = 0.f;
@@ -1226,9 +1226,9 @@ __device__ __forceinline__ float2* wave_c2r(float2* buf, float2* buf2, const flo
                 }
             }
         }
-        wave_sync();
+        seq_sync<NT>();
         if constexpr (BIG) return wave_fft_pp<PRIME>(buf, buf2, rpf, twf, true, lane);
-        wave_fft<2048, PRIME>(buf, 1, rpf, twf, true, lane);
+        wave_fft<2 * LE, PRIME, NT>(buf, 1, rpf, twf, true, lane);
         return buf;
     }
 }
@@ -1336,14 +1336,14 @@ __device__ __forceinline__ void stage_table(float2* tab, int L, const float2* __
     for (int i = threadIdx.x; i < n; i += blockDim.x) tab[i] = t[i];
 }
 
-template <int XPL>
+template <int XPL, int NT>
 __device__ __forceinline__ void store_row_sum(const IfftRowSumArgs& a, const float* acc, int y, int t, int lane) {
     const int Yv = a.fdims ? a.fdims[t].x : a.Y, Xv = a.fdims ? a.fdims[t].y : a.X;
     const long long ro = (long long)t * a.img_tstride + (long long)y * a.X;
     if (a.img) {
 #pragma unroll
         for (int q = 0; q < XPL; ++q) {
-            const int x = lane + 64 * q;
+            const int x = lane + NT * q;
             if (x < a.X) a.img[ro + x] = (y < Yv && x < Xv) ? acc[q] : 0.f;
         }
     }
@@ -1352,29 +1352,35 @@ __device__ __forceinline__ void store_row_sum(const IfftRowSumArgs& a, const flo
         // division: 0/0 gives NaN and x/0 inf, as in numpy
 #pragma unroll
         for (int q = 0; q < XPL; ++q) {
-            const int x = lane + 64 * q;
+            const int x = lane + NT * q;
             if (x < a.X) a.ratio[ro + x] = (y < Yv && x < Xv) ? a.im[ro + x] / acc[q] : 0.f;
         }
     }
 }
 
 // Forward projection, stage 2: per output row, c2r each grid group's row and
-// sum the groups in a fixed order.  One wave per (row, frame), the frames of
-// a block of 8 fastest (they are interleaved in memory);
-// grid (ceil(Y * min(8, T) / RPB), ceil(T / 8)), block 64 * RPB.
-template <bool PRIME, bool BIG, bool ODD>
-__global__ __launch_bounds__(64 * (BIG ? 2 : ROWS_PER_WG)) void k_ifft_rows_sum(IfftRowSumArgs a) {
+// sum the groups in a fixed order.  One workgroup of ROW_SUM_LANES per (row,
+// frame), the frames of a block of 8 fastest (they are interleaved in memory);
+// grid (Y * min(8, T), ceil(T / 8)).  Bound: latency (the groups follow each
+// other, each a load, 3 or 4 passes and the samples), so a row gets 4 waves:
+// one wave per row, 4 rows per workgroup, held 200 registers and left 300 rows
+// on 75 CUs (300^2 x 11 planes 41 -> 30 us, 150^2 x 2 16.4 -> 10.9, 2048^2, rows
+// longer than 2048 then out of place, 211 -> 72; 1455^2 67 either way; with a
+// prime pass, whose few butterflies fill a third of the lanes, 103 -> 130 us at
+// 1273 x 1463, Nnum 19, 0.2 % of a projection).
+constexpr int ROW_SUM_LANES = 256;
+template <bool PRIME, bool ODD>
+__global__ __launch_bounds__(ROW_SUM_LANES) void k_ifft_rows_sum(IfftRowSumArgs a) {
     extern __shared__ float2 lds[];
     reset_smax(a.smax, a.nsmax);
-    constexpr int RPB = BIG ? 2 : ROWS_PER_WG;  // rows (waves) per workgroup
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const RowFrame rf = row_frame(blockIdx.x * RPB + wv, blockIdx.y, a.T);
+    const int lane = threadIdx.x;
+    const RowFrame rf = row_frame(blockIdx.x, blockIdx.y, a.T);
     const int y = rf.y, t = rf.t;
+    if (y >= a.Y) return;                       // (a block of fewer frames has fewer workgroups)
     float2* twf = lds;                          // [maxfX]
-    float2* twh = twf + a.maxfX;                // [maxfX/2]
-    float2* buf = twh + a.maxfX / 2 + 1 + wv * (BIG ? 2 : 1) * a.maxfX;
-    float2* buf2 = buf + a.maxfX;               // BIG only
-    constexpr int XPL = (BIG ? 4096 : 2048) / 64;   // output samples per lane (X <= 2048, BIG: 4096)
+    float2* twh = twf + a.maxfX;                // [maxfX/2 + 1]
+    float2* buf = twh + a.maxfX / 2 + 1;        // [wbuf]
+    constexpr int XPL = 4096 / ROW_SUM_LANES;   // output samples per lane (X <= 4096)
     float acc[XPL];
 #pragma unroll
     for (int q = 0; q < XPL; ++q) acc[q] = 0.f;
@@ -1383,24 +1389,21 @@ __global__ __launch_bounds__(64 * (BIG ? 2 : ROWS_PER_WG)) void k_ifft_rows_sum(
         if (!G.active) continue;
         const int L = G.rp.L;
         __syncthreads();
-        for (int i = threadIdx.x; i < L; i += blockDim.x) twf[i] = G.twf[i];
+        for (int i = lane; i < L; i += ROW_SUM_LANES) twf[i] = G.twf[i];
         if ((L & 1) == 0)
-            for (int i = threadIdx.x; i < L / 2; i += blockDim.x) twh[i] = G.twh[i];
+            for (int i = lane; i < L / 2; i += ROW_SUM_LANES) twh[i] = G.twh[i];
+        const int b0 = t / G.FB * G.FB, nf = min(G.FB, a.T - b0);
+        const float2* row = G.T + (long long)b0 * G.tstride + (long long)y * G.rfX * nf + (t - b0);
         __syncthreads();
-        if (y < a.Y) {
-            const int b0 = t / G.FB * G.FB, nf = min(G.FB, a.T - b0);
-            const float2* row = G.T + (long long)b0 * G.tstride + (long long)y * G.rfX * nf + (t - b0);
-            const float2* res = wave_c2r<PRIME, BIG, ODD>(buf, buf2, row, L, G.rph, twh, G.rp, twf, lane, nf);
-            const float sc = G.scale;
+        wave_c2r<PRIME, false, ODD, ROW_SUM_LANES>(buf, nullptr, row, L, G.rph, twh, G.rp, twf, lane, nf);
+        const float sc = G.scale;
 #pragma unroll
-            for (int q = 0; q < XPL; ++q) {
-                const int x = lane + 64 * q;
-                if (x < a.X) acc[q] += c2r_sample(res, L, x) * sc;
-            }
-            wave_sync();
+        for (int q = 0; q < XPL; ++q) {
+            const int x = lane + ROW_SUM_LANES * q;
+            if (x < a.X) acc[q] += c2r_sample(buf, L, x) * sc;
         }
     }
-    if (y < a.Y) store_row_sum<XPL>(a, acc, y, t, lane);
+    store_row_sum<XPL, ROW_SUM_LANES>(a, acc, y, t, lane);
 }
 
 // The same for several frames, rows staged through LDS (see stage_rows);
@@ -1440,7 +1443,7 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void k_ifft_rows_sum_staged(IfftRow
             }
         }
     }
-    if (busy) store_row_sum<XPL>(a, acc, y, t, lane);
+    if (busy) store_row_sum<XPL, 64>(a, acc, y, t, lane);
 }
 
 // One row's samples to the volume: stored, or the Richardson-Lucy update.  Two
@@ -1788,12 +1791,8 @@ hipError_t launch_ifft_cols(const IfftColArgs& a, int nbatch, hipStream_t s) {
     }
     return hipGetLastError();
 }
-// Twiddles (full and half length), then per wave one buffer (two for rows
-// longer than 2048, which take two waves per workgroup instead of four).
-size_t ifft_rows_sum_lds(int maxfX) {
-    const bool big = wave_big(maxfX);
-    return ((size_t)maxfX + maxfX / 2 + 1 + (big ? 2 * 2 : ROWS_PER_WG) * (size_t)maxfX) * sizeof(float2);
-}
+// Twiddles (full and half length) and one row.
+static size_t row_sum_lds(int maxfX, int wbuf) { return ((size_t)maxfX + maxfX / 2 + 1 + wbuf) * sizeof(float2); }
 static int row_blocks(int Y, int T, int rows) { return (Y * std::min(8, T) + rows - 1) / rows; }
 // Staged rows: the transform's table and one buffer per wave (149 KB at most,
 // rows of 2047).
@@ -1826,19 +1825,14 @@ hipError_t launch_ifft_rows_sum(const IfftRowSumArgs& a, int Y, int T, hipStream
         prime = prime || has_prime(a.grp[g].rp) || has_prime(a.grp[g].rph);
         odd = odd || (a.grp[g].rp.L & 1);
     }
-    const bool big = wave_big(a.maxfX);
     with_bool(prime, [&](auto P) {
         with_bool(odd, [&](auto O) {
-            if (T > 1 && !big)
+            if (T > 1 && !wave_big(a.maxfX))
                 hipLaunchKernelGGL((k_ifft_rows_sum_staged<P.value, O.value>), dim3(row_stage_blocks(Y, T), (T + 7) / 8),
                                    dim3(64 * row_stage_waves(T)), row_stage_lds(a.wbuf, T), s, a);
-            else if (big)
-                hipLaunchKernelGGL((k_ifft_rows_sum<P.value, true, true>), dim3(row_blocks(Y, T, 2), (T + 7) / 8),
-                                   dim3(128), ifft_rows_sum_lds(a.maxfX), s, a);
             else
-                hipLaunchKernelGGL((k_ifft_rows_sum<P.value, false, O.value>),
-                                   dim3(row_blocks(Y, T, ROWS_PER_WG), (T + 7) / 8), dim3(64 * ROWS_PER_WG),
-                                   ifft_rows_sum_lds(a.maxfX), s, a);
+                hipLaunchKernelGGL((k_ifft_rows_sum<P.value, O.value>), dim3(Y * std::min(8, T), (T + 7) / 8),
+                                   dim3(ROW_SUM_LANES), row_sum_lds(a.maxfX, a.wbuf), s, a);
         });
     });
     return hipGetLastError();
@@ -1883,11 +1877,10 @@ hipError_t configure_kernels(size_t max_lds) {
         for (bool odd : {false, true})
             with_bool(prime, [&](auto P) {
                 with_bool(odd, [&](auto O) {
-                    all.push_back((const void*)k_ifft_rows_sum<P.value, false, O.value>);
+                    all.push_back((const void*)k_ifft_rows_sum<P.value, O.value>);
                     all.push_back((const void*)k_ifft_rows_sum_staged<P.value, O.value>);
                     all.push_back((const void*)k_ifft_rows_plane<P.value, false, O.value>);
                     all.push_back((const void*)k_ifft_rows_plane_staged<P.value, O.value>);
-                    all.push_back((const void*)k_ifft_rows_sum<P.value, true, true>);
                     all.push_back((const void*)k_ifft_rows_plane<P.value, true, true>);
                 });
             });
