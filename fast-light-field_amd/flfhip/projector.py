@@ -281,7 +281,9 @@ class Projector_hip(object):
         planes, arr = self._plane_array(planes, hMatrix.numZ)
         self._ensure_psf(hMatrix, planes, 1)
         if out is None:
-            out = torch.zeros((hMatrix.numZ, T, Y, X), dtype=torch.float32, device=self.device)
+            # (every sample of a listed plane is written)
+            new = torch.empty if set(planes) == set(range(hMatrix.numZ)) else torch.zeros
+            out = new((hMatrix.numZ, T, Y, X), dtype=torch.float32, device=self.device)
         self._check(self.lib.flf_backward(self._ctx, _ptr(img), _ptr(out), arr, len(planes), _stream_handle()),
                     "flf_backward")
         return out
