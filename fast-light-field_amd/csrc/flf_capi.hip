@@ -731,9 +731,9 @@ int flf_plan(flf_ctx* ctx, int nnum, int Y, int X, int T, int nz, const int* s2)
             if (!make_radix_plan(fY, g.rpY, false, ro) || !make_radix_plan(fX, g.rpX, false, ro) ||
                 !(wide ? make_radix_plan(g.gt.rY, g.rpYr, false, ro) : make_reduced_plan(g.gt.rY, g.rpYr, ro)) ||
                 !(wide ? make_radix_plan(g.gt.rX, g.rpXr, false, ro) : make_reduced_plan(g.gt.rX, g.rpXr, ro)) ||
-                !make_radix_plan(fY, g.rpYw, true, ro) || !make_radix_plan(fX, g.rpXw, true, ro) ||
+                !make_wave_plan(fY, g.rpYw, ro) || !make_wave_plan(fX, g.rpXw, ro) ||
                 (fX % 2 == 0 &&
-                 (!make_radix_plan(fX / 2, g.rpXh, false, ro) || !make_radix_plan(fX / 2, g.rpXhw, true, ro))))
+                 (!make_radix_plan(fX / 2, g.rpXh, false, ro) || !make_wave_plan(fX / 2, g.rpXhw, ro))))
                 return fail(ctx, FLF_EINVAL, "Fourier grid length has a prime factor other than 2, 3, 5 and one odd "
                                              "prime up to 31");
             gi = (int)ctx->groups.size() - 1;

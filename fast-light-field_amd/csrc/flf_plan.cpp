@@ -77,36 +77,26 @@ static bool shortest_plan(int L, RadixPlan& rp) {
 bool make_radix_plan(int L, RadixPlan& rp, bool wide, int order) {
     rp.L = L;
     rp.n = 0;
-    if (order < 0 || order >= FLF_RADIX_ORDERS) return false;
-    // Block-level transforms use radices 2..5, wave-level ones the composite
-    // radices up to 12 too, for fewer passes (LDS round trips): 3 or 4 instead
-    // of 4 or 5 at most lengths of 700 to 1800.  Orders 2 and 3 change the
-    // radices of wave-level plans only: the block-level kernels size their
-    // butterfly registers from the plan's radices (fft_batch_cap).
-    const int narrow[4] = {4, 2, 3, 5};
-    const int wider[2][6] = {{6, 4, 5, 3, 2, 0}, {5, 3, 8, 6, 4, 2}};
     int m = L;
-    if (wide && order < 2) {
-        int smooth = 1;
-        for (int R : {2, 3, 5})
-            while (m % R == 0) { m /= R; smooth *= R; }
-        if (!shortest_plan(smooth, rp)) return false;
-        rp.L = L;
-    } else {
-        const int* list = wide ? wider[order - 2] : narrow;
-        const int nlist = wide ? 6 : 4;
-        for (int k = 0; k < nlist; ++k) {
-            const int R = list[k];
-            if (R == 0) break;
-            while (m % R == 0) {
-                if (rp.n >= FLF_MAX_RADIX_PASSES) return false;
-                rp.r[rp.n++] = R;
-                m /= R;
-            }
+    // Block-level transforms use radices 2..5, wave-level ones 8 and 6 too.
+    // Orders 2 and 3 change the radices of wave-level plans only: the
+    // block-level kernels size their butterfly registers from the plan's
+    // radices (fft_batch_cap).
+    const int narrow[4] = {4, 2, 3, 5};
+    const int wider[4][6] = {{8, 6, 4, 5, 3, 2}, {8, 6, 4, 5, 3, 2}, {6, 4, 5, 3, 2, 0}, {5, 3, 8, 6, 4, 2}};
+    if (order < 0 || order >= FLF_RADIX_ORDERS) return false;
+    const int* list = wide ? wider[order] : narrow;
+    const int nlist = wide ? 6 : 4;
+    for (int k = 0; k < nlist; ++k) {
+        const int R = list[k];
+        if (R == 0) break;
+        while (m % R == 0) {
+            if (rp.n >= FLF_MAX_RADIX_PASSES) return false;
+            rp.r[rp.n++] = R;
+            m /= R;
         }
     }
-    if (order == 1)
-        for (int i = 0, j = rp.n - 1; i < j; ++i, --j) std::swap(rp.r[i], rp.r[j]);
+    if (order == 1) std::reverse(rp.r, rp.r + rp.n);
     // One odd prime factor above 5 (a lenslet pitch such as 7, 13 or 19) is
     // taken as the last pass, the only position where a radix-P butterfly
     // writes onto its own inputs (see stockham_pass_prime, wave_pass_prime).
@@ -116,6 +106,22 @@ bool make_radix_plan(int L, RadixPlan& rp, bool wide, int order) {
         m = 1;
     }
     return m == 1;
+}
+
+bool make_wave_plan(int L, RadixPlan& rp, int order) {
+    // 3 or 4 passes (LDS round trips) instead of 4 or 5 at most lengths of 700
+    // to 1800 (8 frames of 1455^2 x 41 planes: columns 2.85 -> 2.50 ms).
+    if (order < 0 || order > 1) return make_radix_plan(L, rp, true, order);
+    int m = L, smooth = 1;
+    for (int R : {2, 3, 5})
+        while (m % R == 0) { m /= R; smooth *= R; }
+    if (!shortest_plan(smooth, rp)) return false;
+    rp.L = L;
+    if (order == 1) std::reverse(rp.r, rp.r + rp.n);
+    if (m == 1) return true;
+    if (m <= 5 || m > FLF_PRIME_RADIX_MAX || max_prime_factor(m) != m) return false;
+    rp.r[rp.n++] = m;
+    return true;
 }
 
 bool make_reduced_plan(int L, RadixPlan& rp, int order) {

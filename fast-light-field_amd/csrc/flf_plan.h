@@ -49,6 +49,10 @@ struct GridTables {
 };
 
 // Builds the tables; returns an empty string or an error message.
+// Plan of a row or column transform: order 0 as few passes as possible with
+// radices up to 12, largest first (a prime pass last), 1 reversed, 2 and 3 as
+// make_radix_plan's wide plans.
+bool make_wave_plan(int L, RadixPlan& rp, int order = 0);
 // Plan of a reduced-grid transform (L <= 128, 5-smooth): radices up to 12, as
 // few passes as possible, largest first (order 1: reversed).
 bool make_reduced_plan(int L, RadixPlan& rp, int order = 0);

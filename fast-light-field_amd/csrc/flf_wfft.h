@@ -1,4 +1,5 @@
-// Wave-level mixed-radix (2/3/4/5) FFTs in LDS.
+// Mixed-radix FFTs in LDS (radices 2..6, 8..10, 12 and a last prime), by one
+// wave, several waves or a workgroup per sequence.
 //
 // One 64-lane wave transforms one sequence held in LDS (element stride es).
 // Stockham passes as in flf_fft.h, but each pass is executed by the wave

@@ -121,7 +121,7 @@ int flf_set_frame_dims(flf_ctx* ctx, const int* dims, int T, void* stream);
  * Plan options, applied by the next flf_plan (the FFTW_MEASURE-style
  * choices of py_light_field.cpp:25-31):
  *   "radix_order"    0..3 pass order of every FFT: 0 largest radices first,
- *                    1 reversed, 2 no radix 8 (wave-level transforms), 3 odd
+ *                    1 reversed, 2 up to 6 (wave-level transforms), 3 odd
  *                    radices first (wave-level); a prime pass stays last
  *   "mac_ipt"        1, 2 or 4: as mac_frames
  * Results do not depend on them beyond FP32 rounding (group_streams: not at
@@ -241,7 +241,9 @@ int flf_profile_read(flf_ctx* ctx, double* mac_ms, long long* mac_launches, doub
  * items, max residues per orbit, stored spectra per plane, slots per item,
  * max items per workgroup}.  Returns FLF_EINVAL if the tables are invalid.
  * flf_radix_plan: the passes of a length-L transform for plan option
- * radix_order = order (wide = 1: a wave-level transform) into radices[16];
+ * radix_order = order (wide = 1: a wave-level transform of radices 2 to 8; the
+ * row and column transforms merge these into radices 9, 10 and 12 where that
+ * saves passes in orders 0 and 1) into radices[16];
  * *npass receives their count.  FLF_EINVAL if L has no such plan. */
 int flf_fourier_len(int s1, int s2, int nnum);
 int flf_grid_check(int nnum, int fY, int fX, long long* stats);
