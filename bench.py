@@ -24,7 +24,7 @@ Also reported:
   rl_iteration  the same ratio for a whole RL iteration of one frame:
                 S_H + S_Ht + (4*nz+2)*Y*X*4 bytes / iteration time
                 (rl_iteration_batch: the same for all B frames of a step,
-                where the MAC is FP32-bound instead).
+                which share each read of the spectra).
   cpu_baseline  the FP64 numpy oracle (single thread) timed on one plane's
                 projection at full size and scaled to a volume.
 
@@ -47,7 +47,9 @@ import numpy as np  # noqa: E402
 from flfhip.workloads import BATCHES, RAGGED, WORKLOADS, setup  # noqa: E402
 
 PEAK_HBM = 8.0e12  # MI355X HBM3E, bytes/s
-PEAK_FP32 = 157.3e12  # MI355X FP32, flop/s
+# MI355X dense fp16 on the matrix cores, flop/s, over the four fp16 products
+# that the MAC takes per fp32 product
+PEAK_SPLIT = 2.5e15 / 4
 
 
 def log(*a):
@@ -245,8 +247,8 @@ def ragged_main(args):
         "roofline": {"bound": "hbm", "achieved": achieved / 1e9, "peak": PEAK_HBM / 1e9, "unit": "GB/s",
                      "frac": achieved / PEAK_HBM, "traffic": None, "kernel": "k_mac",
                      "launch_avg_ms": mac_avg_ms, "launches": mac_n, "bytes_per_launch": mac_bytes / max(mac_n, 1)},
-        "valu_fp32": {"kernel": "k_mac", "achieved_TFLOPs": flop_rate / 1e12, "peak_TFLOPs": PEAK_FP32 / 1e12,
-                      "frac": flop_rate / PEAK_FP32, "mac_share_of_step": mac_ms / prof_steps / ms_step},
+        "matrix": {"kernel": "k_mac", "achieved_TFLOPs": flop_rate / 1e12, "peak_TFLOPs": PEAK_SPLIT / 1e12,
+                      "frac": flop_rate / PEAK_SPLIT, "mac_share_of_step": mac_ms / prof_steps / ms_step},
         "spectra_precompute_s": t_prep,
         "device_bytes": dev_bytes,
     }
@@ -506,13 +508,12 @@ def batch_main(args):
                           "plain_volumes_per_s": 1e3 / plain1_ms, "learned_volumes_per_s": 1e3 / learned1_ms,
                           "speedup": plain1_ms / learned1_ms},
         },
-        "roofline": {"bound": "fp32", "achieved": flop_rate / 1e12, "peak": PEAK_FP32 / 1e12, "unit": "TFLOP/s",
-                     "frac": flop_rate / PEAK_FP32, "traffic": measured_traffic(args.workload), "kernel": "k_mac",
+        "roofline": {"bound": "matrix", "achieved": flop_rate / 1e12, "peak": PEAK_SPLIT / 1e12, "unit": "TFLOP/s",
+                     "frac": flop_rate / PEAK_SPLIT, "traffic": measured_traffic(args.workload), "kernel": "k_mac",
                      "launch_avg_ms": mac_avg_ms, "launches": mac_n,
                      "flops_per_launch": mac_flops / max(mac_n, 1),
-                     "note": "several frames per workgroup: the MAC is bound on the CU, not by HBM: VALU 57% "
-                             "busy, one 16-byte LDS table read per 8 FMAs, two to three waves per SIMD "
-                             "(profiles/k_mac_rl1455x32_sq_counters.txt)",
+                     "note": "8 frames per workgroup: the MAC is bound by matrix and vector issue (P/M table, "
+                             "operand splits) beside its memory stream; peak: fp16 matrix rate / 4 products",
                      "hbm": {"achieved": hbm_rate / 1e9, "peak": PEAK_HBM / 1e9, "unit": "GB/s",
                              "frac": hbm_rate / PEAK_HBM, "bytes_per_launch": mac_bytes / max(mac_n, 1)}},
         "rl_iteration": {"ms": it1_s * 1e3, "frames": 1, "algorithmic_bytes": it1_bytes,
@@ -520,7 +521,7 @@ def batch_main(args):
                          "note": "one frame: every cached spectrum read once per projection, HBM-bound"},
         "rl_iteration_batch": {"ms": it_s * 1e3, "frames": T, "algorithmic_bytes": it_bytes,
                                "achieved_GBps": it_bytes / it_s / 1e9, "frac": it_bytes / it_s / PEAK_HBM,
-                               "note": "all frames of a step: FP32-bound (see roofline), not HBM-bound"},
+                               "note": "all frames of a step: the spectra are read once per 8 frames (see roofline)"},
         "spectra_precompute_s": t_prep,
     }
     del X1s
